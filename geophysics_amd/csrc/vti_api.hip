@@ -401,6 +401,8 @@ int vti_destroy(vti_ctx *c)
     hipFree(c->tab);
     hipFree(c->dgw);
     hipFree(c->dtap);
+    hipFree(c->damp);
+    run2d_free(c);
     hipFree(c->rec);
     hipFree(c->rec_t);
     for (hipEvent_t e : c->ev_acc)
@@ -611,6 +613,11 @@ int vti_set_shot(vti_ctx *c, const vti_shot *s)
         c->tapR = k.sv_R;
     }
     HIP_TRY(hipMemcpy(c->dtap, tap.data(), tap.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (!is3d(c)) {   // the resident 2D steps read the gains on the device
+        if (!c->damp && hipMalloc(&c->damp, (size_t)k.nt * sizeof(float)) != hipSuccess)
+            return fail(VTI_ERR_ALLOC, "vti_set_shot: source gains");
+        HIP_TRY(hipMemcpy(c->damp, c->amp.data(), (size_t)k.nt * sizeof(float), hipMemcpyHostToDevice));
+    }
     c->have_shot = true;
     return VTI_OK;
 }
@@ -693,6 +700,10 @@ int vti_step(vti_ctx *c, int it0, int nsteps)
         }
         c->alt_valid = true;   // both sets hold the same cells outside the updated region
         return VTI_OK;
+    }
+    if (c->cfg.ndim == 2 && !c->prof) {
+        st = run2d_steps(c, it0, nsteps);
+        if (st) return st < 0 ? st : VTI_OK;
     }
     for (int it = it0; it < it0 + nsteps; ++it) {
         hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
@@ -809,14 +820,14 @@ int vti_run(vti_ctx *c)
     st = vti_step(c, 0, c->cfg.nt);
     if (st) return st;
     HIP_TRY(hipStreamSynchronize(c->stream));
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_sync(vti_ctx *c)
 {
     if (!c) return fail(VTI_ERR_ARG, "vti_sync: null ctx");
     HIP_TRY(hipStreamSynchronize(c->stream));
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_nrec(const vti_ctx *c) { return c ? c->nrec : 0; }
@@ -869,7 +880,7 @@ int vti_get_record(vti_ctx *c, float *dst)
     HIP_TRY(launch_transpose(c->rec, c->rec_t, nt, nrec, c->stream));
     HIP_TRY(hipMemcpyAsync(dst, c->rec_t, (size_t)nt * nrec * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 static float *field_ptr(vti_ctx *c, int which)
@@ -890,7 +901,7 @@ int vti_get_field(vti_ctx *c, int which, float *dst)
     HIP_TRY(hipMemcpy2DAsync(dst, g.nnz * sizeof(float), p, g.ldz * sizeof(float),
                              g.nnz * sizeof(float), (size_t)g.nnx * g.nny, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_set_field(vti_ctx *c, int which, const float *src)

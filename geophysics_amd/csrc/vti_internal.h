@@ -126,6 +126,8 @@ struct VtiState {
     float *f[11] = {};
 };
 
+namespace vti { struct Run2dPlan; }
+
 // Context: model, tables, the main wavefield state and per-shot buffers.
 struct vti_ctx {
     vti_cfg cfg{};
@@ -144,6 +146,7 @@ struct vti_ctx {
     float d0 = 0.0f;
 
     std::vector<float> amp;     // per-step source gain
+    float *damp = nullptr;      // the same on the device
     double *dtap = nullptr;     // SV taper factors
     int tapR = 0;
     double *dgw = nullptr;      // 7x7 Gaussian weights
@@ -185,6 +188,7 @@ struct vti_ctx {
     // 2D TTI (vti_set_theta): cos and sin of the padded tilt, two pitched
     // volumes; nullptr: VTI
     float *tti = nullptr;
+    vti::Run2dPlan *run2d = nullptr;   // resident 2D steps (vti_run2d.hip), made at their first use
 };
 
 namespace vti {
@@ -216,4 +220,10 @@ StressArgs with_snap(vti_ctx *c, StressArgs a, float *snap);
 // one angle-gather accumulation (vti_adcig.hip) from a source and a receiver
 // state of the context's grid, when the context has gathers configured
 hipError_t launch_adcig(vti_ctx *c, const VtiState &src, const VtiState &rcv);
+// vti_run2d.hip: n steps of the main state in one resident launch (1:
+// launched, 0: not applicable, < 0: error); its workspace; its error check
+// after a wait for the stream
+int run2d_steps(vti_ctx *c, int it0, int n);
+void run2d_free(vti_ctx *c);
+int run2d_check(vti_ctx *c);
 }  // namespace vti

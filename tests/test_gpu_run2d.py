@@ -1,0 +1,86 @@
+"""The resident 2D steps (vti_step / vti_run of a 2D context) against the
+per-step kernels behind vti_update_vel / vti_update_stress: the same
+arithmetic, so every field and record must be equal bit for bit."""
+import numpy as np
+import pytest
+
+from geophysics_amd import vti
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("u", "w", "px", "pz", "qx", "qz", "P", "Q")
+
+
+def build(form, nx, nz, npml, nt, unsplit, seed):
+    rng = np.random.default_rng(seed)
+    mode = vti.MODE_CPU_REF if form == "cpu" else vti.MODE_GPU_REF
+    cfg = vti.cfg_ref2d(mode, nx, nz, 10, 10, npml, 1, 20, nt, 1000)
+    vp = (2200.0 + 600.0 * rng.random((nx, nz))).astype(np.float32)
+    ep = (0.2 * rng.random((nx, nz))).astype(np.float32)
+    dl = (0.5 * ep * rng.random((nx, nz))).astype(np.float32)
+    p = vti.Propagator(cfg, vp, ep, dl)
+    if form == "tti":
+        p.set_theta((50.0 * rng.random((nx, nz)) - 25.0).astype(np.float32), degrees=True)
+    p.set_unsplit(unsplit)
+    p.set_shot(vti.shot_ref2d(cfg, 1, nx // 2, 0, nz // 2, rec_depth=max(1, nz // 3)))
+    p.reset()
+    # every cell of every field seeded, the four border cells too; the split fields add up to P and Q
+    f = {k: (1e-2 * rng.standard_normal(p.shape)).astype(np.float32) for k in FIELDS}
+    f["P"], f["Q"] = f["px"] + f["pz"], f["qx"] + f["qz"]
+    for k in FIELDS:
+        p.set_field(k, f[k])
+    return p
+
+
+# One tile; tiles of the smallest allowed height and width; widths that
+# leave 1, 2 and 3 cells in the last unit; a grid of all tiles (two, three
+# and four units a thread); one too large for the chip (per-step kernels).
+@pytest.mark.parametrize("nx,nz,npml", [(16, 17, 0), (11, 13, 5), (15, 12, 4), (60, 50, 20), (101, 78, 10),
+                                        (333, 71, 20), (64, 403, 9), (700, 301, 20), (1401, 503, 20),
+                                        (2001, 602, 30), (2401, 803, 20), (2500, 1000, 20)])
+@pytest.mark.parametrize("form,unsplit", [("gpu", False), ("gpu", True), ("cpu", False), ("tti", False)])
+def test_resident_steps_equal_per_step_kernels(form, unsplit, nx, nz, npml):
+    if form == "cpu" and (nx < 20 or nz < 20 or npml == 0):
+        pytest.skip("the 7x7 footprint needs room inside the updated region")
+    nt = 24
+    out = []
+    for resident in (True, False):
+        with build(form, nx, nz, npml, nt, unsplit, 7) as p:
+            if resident:
+                p.step(0, 8)
+                p.step(8, 3)      # below the resident form's least step count
+                p.step(11, 13)
+            else:
+                for it in range(nt):
+                    p.update_vel(it)
+                    p.update_stress(it)
+            out.append(({k: p.field(k) for k in FIELDS}, p.record()))
+    (f0, r0), (f1, r1) = out
+    assert np.isfinite(r1).all()
+    assert np.array_equal(r0, r1)
+    for k in FIELDS:
+        assert np.array_equal(f0[k], f1[k]), k
+
+
+def test_resident_steps_of_several_contexts_and_threads():
+    """Contexts on streams of their own, stepped from four threads at once."""
+    import threading
+    sizes = [(120, 90), (333, 71), (700, 301), (60, 50)]
+    ref, got = {}, {}
+
+    def work(k, n, into):
+        with build("gpu", n[0], n[1], 20, 64, False, k) as p:
+            for _ in range(4):
+                p.step(0, 64)
+            p.sync()
+            into[k] = p.field("P")
+
+    for k, n in enumerate(sizes):
+        work(k, n, ref)
+    th = [threading.Thread(target=work, args=(k, n, got)) for k, n in enumerate(sizes)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for k in ref:
+        assert np.array_equal(ref[k], got[k]), k
