@@ -100,12 +100,22 @@ hipError_t state_zero(vti_ctx *c, const VtiState &s)
 
 hipError_t state_copy(vti_ctx *c, const VtiState &dst, const VtiState &src)
 {
-    for (int k = 0; k < 11; ++k)
-        if (src.f[k]) {
-            hipError_t e = hipMemcpyAsync(dst.f[k], src.f[k], c->nvol * sizeof(float),
-                                          hipMemcpyDeviceToDevice, c->stream);
-            if (e != hipSuccess) return e;
+    // fields that follow each other in both states go as one copy (all of
+    // them, unless fused steps have swapped some): eight copies of a 2D field
+    // take 17 us, one of the state 4
+    for (int k = 0; k < 11;) {
+        if (!src.f[k]) { ++k; continue; }
+        const float *s0 = src.f[k];
+        float *d0 = dst.f[k];
+        size_t n = c->nvol;
+        for (++k; k < 11; ++k) {
+            if (!src.f[k]) continue;
+            if (src.f[k] != s0 + n || dst.f[k] != d0 + n) break;
+            n += c->nvol;
         }
+        hipError_t e = hipMemcpyAsync(d0, s0, n * sizeof(float), hipMemcpyDeviceToDevice, c->stream);
+        if (e != hipSuccess) return e;
+    }
     return hipSuccess;
 }
 

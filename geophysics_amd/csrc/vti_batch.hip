@@ -292,8 +292,10 @@ __device__ __forceinline__ int find_row(const BShot *S, int ns, int r)
 // [xlo, xhi) x [zlo, zhi), the cells that never read or write them.  One
 // workgroup per grid row of every shot, 16-byte pieces (rows are ldz floats,
 // a multiple of 32).
+// fields: bit k for field k of the state (a checkpoint that is only imaged
+// keeps P alone).
 __global__ void bckpt(const BShot *__restrict__ S, int ns, int nrows, const float *__restrict__ base,
-                      float *__restrict__ slot, int store)
+                      float *__restrict__ slot, int store, int fields)
 {
     for (int r = blockIdx.x; r < nrows; r += gridDim.x) {
         const BShot &b = S[find_row(S, ns, r)];
@@ -301,6 +303,7 @@ __global__ void bckpt(const BShot *__restrict__ S, int ns, int nrows, const floa
         const bool mid = ix >= b.xlo && ix < b.xhi;
         const int n4 = b.ldz / 4;
         for (int k = 0; k < 8; ++k) {
+            if (!(fields >> k & 1)) continue;
             const size_t o = (size_t)(b.f[k] - base) + (size_t)ix * b.ldz;
             const float4 *src = reinterpret_cast<const float4 *>(store ? base + o : slot + o);
             float4 *dst = reinterpret_cast<float4 *>(store ? slot + o : const_cast<float *>(base) + o);
@@ -803,10 +806,16 @@ int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, 
                             : hipMemcpyAsync(B->state_base, B->slots[i], sb, hipMemcpyDeviceToDevice, B->stream),
                       "checkpoint");
         hipLaunchKernelGGL(bckpt, dim3((unsigned)std::min(B->nrows, 8192)), dim3(256), 0, B->stream, B->db, B->nshot,
-                           B->nrows, B->state_base, B->slots[i], store);
+                           B->nrows, B->state_base, B->slots[i], store, 0xff);
         return ok(hipGetLastError(), "checkpoint");
     };
     op.store = [&](int i) { slot_it[i] = cur_it; return ckpt(i, 1); };
+    op.store_light = [&](int i) {
+        slot_it[i] = cur_it;
+        hipLaunchKernelGGL(bckpt, dim3((unsigned)std::min(B->nrows, 8192)), dim3(256), 0, B->stream, B->db, B->nshot,
+                           B->nrows, B->state_base, B->slots[i], 1, 1 << 6);
+        return ok(hipGetLastError(), "checkpoint");
+    };
     op.restore = [&](int i) {
         cur_it = slot_it[i];
         hipLaunchKernelGGL(bset_it, dim3(1), dim3(64), 0, B->stream, B->itp, cur_it);

@@ -691,7 +691,19 @@ struct Grad : vti_grad {
             return hipMemcpy(res, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice) == hipSuccess
                        ? VTI_OK : fail(VTI_ERR_HIP, "residual upload");
         };
+        // the adjoint reads u, v and w of the forward state, from a slot too;
+        // a checkpoint that no step starts from keeps those alone
         op.consume = [&](int k) { adj_step(k - 1, f); return hip_ok(); };
+        op.consume_slot = [&](int k, int i) {
+            Fields<T> s{};
+            set_fields(s, slots[i], nvol, g.three);
+            adj_step(k - 1, s);
+            return hip_ok();
+        };
+        op.store_light = [&](int i) {   // u, v, w (2D: u, w) lead the state
+            return hipMemcpyAsync(slots[i], state_base(f), (g.three ? 3 : 2) * nvol * sizeof(T), hipMemcpyDeviceToDevice,
+                                  stream) == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "store");
+        };
         int st = reverse_sweep(nt, nslot, op, steps);
         if (st || (st = sync())) return st;
         if (misfit) *misfit = J;

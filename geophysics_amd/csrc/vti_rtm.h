@@ -21,6 +21,10 @@ struct SweepOps {
     // optional: X_k read from checkpoint slot i without restoring it (a
     // checkpointed state is consumed once, then its slot is freed)
     std::function<int(int, int)> consume_slot;
+    // optional, with consume_slot: checkpoint slot i <- what consume_slot
+    // reads of the working state; for a checkpoint that no later step starts
+    // from (most of them: the innermost runs store every state they pass)
+    std::function<int(int)> store_light;
 };
 
 // Runs the first sweep, then calls consume(k) for k = nt, nt-1, ..., 1 in

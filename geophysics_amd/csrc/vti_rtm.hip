@@ -385,6 +385,12 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
     op.zero = [&]() { return hip(state_zero(c, W), "zero"); };
     op.store = [&](int i) { return hip(ck_copy(c, rc.ck, i, W, true), "store"); };
     op.restore = [&](int i) { return hip(ck_copy(c, rc.ck, i, W, false), "restore"); };
+    // the image reads P alone (the angle gathers Q and the velocities too)
+    if (!c->adcig)
+        op.store_light = [&](int i) {
+            return hip(hipMemcpyAsync(rc.ck.view[i].f[VTI_F_P], W.f[VTI_F_P], c->nvol * sizeof(float),
+                                      hipMemcpyDeviceToDevice, c->stream), "store");
+        };
     op.step = [&](int it) {
         if (launch_vel(nd, vel_args_for(c, W, it, true), c->stream) != hipSuccess) return fail(VTI_ERR_HIP, "vel");
         return hip(launch_stress(nd, src_stress_args(c, W, it, svf, nullptr), c->stream), "stress");

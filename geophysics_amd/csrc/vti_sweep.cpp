@@ -52,12 +52,13 @@ int reverse_sweep(int nt, int nslot, const SweepOps &op, long long *fwd_steps)
     int work = -1, frontier = 0;
     bool first_done = false;
     std::vector<int> free_slots, pos_slot(nt + 1, -1);
+    std::vector<char> light(nt + 1, 0);
     for (int i = nslot - 1; i >= 0; --i) free_slots.push_back(i);
     auto restore = [&](int pos) -> int {
         if (pos == work) return VTI_OK;
         int e;
         if (pos == 0) e = op.zero();
-        else if (pos_slot[pos] < 0) return fail(VTI_ERR_STATE, "reverse_sweep: missing checkpoint");
+        else if (pos_slot[pos] < 0 || light[pos]) return fail(VTI_ERR_STATE, "reverse_sweep: missing checkpoint");
         else e = op.restore(pos_slot[pos]);
         if (!e) work = pos;
         return e;
@@ -121,7 +122,10 @@ int reverse_sweep(int nt, int nslot, const SweepOps &op, long long *fwd_steps)
         if (free_slots.empty()) return fail(VTI_ERR_STATE, "reverse_sweep: slot overflow");
         const int i = free_slots.back();
         free_slots.pop_back();
-        if ((e = op.store(i))) return e;
+        // X_m is started from again unless (m, r] goes one state at a time
+        const int n2 = t.r - m, s2 = t.s - 1;
+        light[m] = op.store_light && op.consume_slot && (n2 <= 1 || (s2 >= 1 && split_len(n2, s2) == 1));
+        if ((e = light[m] ? op.store_light(i) : op.store(i))) return e;
         pos_slot[m] = i;
         todo.push_back({1, t.l, m, t.s});
         todo.push_back({0, m, t.r, t.s - 1});
@@ -137,17 +141,19 @@ extern "C" {
 // Runs the schedule on integer positions: the working "state" is the number
 // of steps taken from X_0, a slot holds a position.  Fails unless consume(k)
 // sees X_k for k = nt .. 1 in that order with at most nslot slots in use,
-// both with checkpointed states restored before they are consumed and
-// consumed from their slots (the same forward steps either way).
+// with checkpointed states restored before they are consumed, consumed from
+// their slots, and with light checkpoints besides (the same forward steps
+// each way).
 int vti_sweep_check(int nt, int nslot, long long *fwd_steps, int *max_slots)
 {
     if (nt < 1 || nslot < 0) return vti::fail(VTI_ERR_ARG, "vti_sweep_check: nt >= 1 and nslot >= 0");
-    long long steps[2] = {0, 0};
+    long long steps[3] = {0, 0, 0};
     int peak = 0;
-    for (int from_slot = 0; from_slot < 2; ++from_slot) {
+    for (int from_slot = 0; from_slot < 3; ++from_slot) {
         int work = -1, next = nt, used = 0;
         peak = 0;
         std::vector<int> slot(nslot, -1);
+        std::vector<char> whole(nslot, 1);   // the slot can be started from
         bool first_done = false, bad = false;
         vti::SweepOps op;
         op.zero = [&]() { work = 0; return VTI_OK; };
@@ -155,10 +161,17 @@ int vti_sweep_check(int nt, int nslot, long long *fwd_steps, int *max_slots)
             if (i < 0 || i >= nslot) { bad = true; return VTI_ERR_STATE; }
             if (slot[i] < 0) peak = std::max(peak, ++used);
             slot[i] = work;
+            whole[i] = 1;
             return VTI_OK;
         };
+        if (from_slot == 2)
+            op.store_light = [&](int i) {
+                const int e = op.store(i);
+                if (!e) whole[i] = 0;
+                return e;
+            };
         op.restore = [&](int i) {
-            if (i < 0 || i >= nslot || slot[i] < 0) { bad = true; return VTI_ERR_STATE; }
+            if (i < 0 || i >= nslot || slot[i] < 0 || !whole[i]) { bad = true; return VTI_ERR_STATE; }
             work = slot[i];
             return VTI_OK;
         };
@@ -192,7 +205,7 @@ int vti_sweep_check(int nt, int nslot, long long *fwd_steps, int *max_slots)
         const int st = vti::reverse_sweep(nt, nslot, op, &steps[from_slot]);
         if (st || bad || next != 0) return vti::fail(VTI_ERR_STATE, "vti_sweep_check: schedule out of order");
     }
-    if (steps[0] != steps[1]) return vti::fail(VTI_ERR_STATE, "vti_sweep_check: slot consumes change the steps");
+    if (steps[0] != steps[1] || steps[0] != steps[2]) return vti::fail(VTI_ERR_STATE, "vti_sweep_check: slot consumes change the steps");
     if (fwd_steps) *fwd_steps = steps[0];
     if (max_slots) *max_slots = peak;
     return VTI_OK;
