@@ -385,11 +385,12 @@ int vti_create(const vti_cfg *cfg, vti_ctx **out)
     x->vp = p; p += x->nvol;
     x->ep = p; p += x->nvol;
     x->de = p; p += x->nvol;
-    if (hipMalloc(&x->tab, 12 * (size_t)x->nnmax * sizeof(float)) != hipSuccess ||
+    if (hipMalloc(&x->tab, (12 * (size_t)x->nnmax + c.nt) * sizeof(float)) != hipSuccess ||
         hipMalloc(&x->dgw, 49 * sizeof(double)) != hipSuccess) {
         vti_destroy(x.release());
         return fail(VTI_ERR_ALLOC, "vti_create: table allocation");
     }
+    x->damp = x->tab + 12 * (size_t)x->nnmax;
     x->htab.assign(12 * (size_t)x->nnmax, 1.0f);
     double gw[49];
     gaussian_weights(gw);
@@ -411,7 +412,6 @@ int vti_destroy(vti_ctx *c)
     hipFree(c->tab);
     hipFree(c->dgw);
     hipFree(c->dtap);
-    hipFree(c->damp);
     run2d_free(c);
     hipFree(c->rec);
     hipFree(c->rec_t);
@@ -623,11 +623,8 @@ int vti_set_shot(vti_ctx *c, const vti_shot *s)
         c->tapR = k.sv_R;
     }
     HIP_TRY(hipMemcpy(c->dtap, tap.data(), tap.size() * sizeof(double), hipMemcpyHostToDevice));
-    if (!is3d(c)) {   // the resident 2D steps read the gains on the device
-        if (!c->damp && hipMalloc(&c->damp, (size_t)k.nt * sizeof(float)) != hipSuccess)
-            return fail(VTI_ERR_ALLOC, "vti_set_shot: source gains");
+    if (!is3d(c))   // the resident 2D steps read the gains on the device
         HIP_TRY(hipMemcpy(c->damp, c->amp.data(), (size_t)k.nt * sizeof(float), hipMemcpyHostToDevice));
-    }
     c->have_shot = true;
     return VTI_OK;
 }

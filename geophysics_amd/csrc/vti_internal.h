@@ -146,7 +146,7 @@ struct vti_ctx {
     float d0 = 0.0f;
 
     std::vector<float> amp;     // per-step source gain
-    float *damp = nullptr;      // the same on the device
+    float *damp = nullptr;      // the same on the device (after the damping tables)
     double *dtap = nullptr;     // SV taper factors
     int tapR = 0;
     double *dgw = nullptr;      // 7x7 Gaussian weights

@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <functional>
 #include <string>
@@ -23,6 +24,7 @@
 
 #include "vti_internal.h"
 #include "vti_rtm.h"
+#include "vti_run2d.h"
 
 namespace vti {
 namespace {
@@ -440,8 +442,78 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
     op.consume = [&](int k) { return consume_from(W, k); };
     op.consume_slot = [&](int k, int i) { return consume_from(rc.ck.view[i], k); };
     c->rtm_illum_mode = o->illum_mode;
+
+    // 2D: runs of steps of either side as resident launches.  The kernel
+    // images and injects inside the updated region only, so the interior and
+    // every receiver must lie in it; the TTI update and the gathers go step
+    // by step.
+    Run2dGroup grp;
+    struct GroupGuard {
+        Run2dGroup &g;
+        ~GroupGuard() { run2d_group_free(g); }
+    } group_guard{grp};
+    RtmQueue q;
+    if (nd == 2 && nt >= 8 && c->cfg.mode == VTI_MODE_GPU_REF && !c->tti && !c->adcig && c->cfg.npml >= 4 &&
+        c->shot.rec_x0 >= 4 && c->shot.rec_x0 + (c->shot.rec_nx - 1) * c->shot.rec_dx < c->g.nnx - 4 &&
+        c->shot.rec_z >= 4 && c->shot.rec_z < c->g.nnz - 4) {
+        Run2dShot a = run2d_shot(c, W), b = run2d_shot(c, rc.g);
+        a.sv = svf;
+        b.sv = svb;
+        a.img = b.img = c->img;
+        a.illum = b.illum = c->illum;
+        a.clamp = clamp;
+        b.rillum = o->illum_mode == 1;
+        b.split_z = b.rzi = inj_z;
+        b.srcP = W.f[VTI_F_P];
+        if ((st = run2d_group_make(grp, {a}, {b}, c->unsplit, c->device, c->stream)) < 0) return st;
+    }
+    if (grp.ok == 1) {
+        const float *P = W.f[VTI_F_P];
+        auto slot_off = [&](int i) {
+            return ((long long)reinterpret_cast<intptr_t>(rc.ck.view[i].f[VTI_F_P]) -
+                    (long long)reinterpret_cast<intptr_t>(P)) / (long long)sizeof(float);
+        };
+        auto at = [&](long long off) {
+            VtiState s;
+            s.f[VTI_F_P] = const_cast<float *>(P) + off;
+            return s;
+        };
+        q.run_forward = [&](bool first, int it0, int n, const long long *off) {
+            return run2d_group_run(grp, 1, it0, n, first, first, 1, off, c->stream);
+        };
+        q.run_receive = [&](int it0, int n, const long long *off) {
+            return run2d_group_run(grp, 2, it0, n, false, false, o->image_every, off, c->stream);
+        };
+        const auto step1 = op.step, first1 = op.first_step;
+        q.step = [&, step1, first1](bool first, int it) { return first ? first1(it) : step1(it); };
+        q.keep = [&](long long off) {
+            return hip(hipMemcpyAsync(at(off).f[VTI_F_P], P, c->nvol * sizeof(float), hipMemcpyDeviceToDevice, c->stream),
+                       "store");
+        };
+        q.receive = [&](int it, long long off) { return consume_from(at(off), it + 1); };
+        // every other operation finds the states as if each step had been
+        // taken when it was asked for
+        auto flushed = [&q](std::function<int()> f) {
+            return [&q, f]() { const int e = q.flush(); return e ? e : f(); };
+        };
+        auto flushed1 = [&q](std::function<int(int)> f) {
+            return [&q, f](int i) { const int e = q.flush(); return e ? e : f(i); };
+        };
+        op.zero = flushed(op.zero);
+        op.after_first = flushed(op.after_first);
+        op.store = flushed1(op.store);
+        op.restore = flushed1(op.restore);
+        op.store_light = [&, slot_off](int i) { return q.keep_last(slot_off(i)); };
+        op.step = [&](int it) { return q.forward(false, it); };
+        op.first_step = [&](int it) { return q.forward(true, it); };
+        op.consume = [&](int k) { return q.receiver(k - 1, 0); };
+        op.consume_slot = [&, slot_off](int k, int i) { return q.receiver(k - 1, slot_off(i)); };
+        if (c->unsplit) c->us_dirty = true;
+    }
     if ((st = reverse_sweep(nt, nslot, op, fwd_steps))) return st;
-    return hip(hipStreamSynchronize(c->stream), "sync");
+    if (grp.ok && (st = q.flush())) return st;
+    if ((st = hip(hipStreamSynchronize(c->stream), "sync"))) return st;
+    return run2d_group_check(grp);
 }
 
 // One imaging step of a caller-driven RTM (cal_migration

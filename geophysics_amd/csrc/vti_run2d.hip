@@ -36,9 +36,11 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <new>
 #include <string>
 
 #include "vti_internal.h"
+#include "vti_run2d.h"
 
 namespace vti {
 namespace {
@@ -52,23 +54,17 @@ __device__ __forceinline__ float cst(int m)
 constexpr unsigned long long kWaitTicks = 2000000000ull;
 
 struct Run2dArgs {
-    int nnx, nnz, ldz, M;
-    float *u, *w, *px, *pz, *qx, *qz, *P, *Q;
-    const float *vp, *ep, *de, *cth, *sth, *tab;
-    float dtx, dtz;
-    int sv, svR, cx, cz;
-    const double *tap;
-    int point, sx, sz;          // point source (load-time) or the 7x7 footprint in the stress update
-    const double *gw;
-    const float *amp;           // nt source gains
-    float *rec;                 // [it][nrec], nullptr: no record
-    int nrec, rec_kind, rz, rx0, rdx, rnx;
-    int it0, n;
-    int gx, gz;                 // tiles in x and z
-    unsigned long long *xP, *xQ;   // exchange planes, two each, of (tag, float) words
-    long long xstride;
+    Run2dShot one;              // role 0: the shot
+    const Run2dShot *many;      // roles 1, 2: ns shots in device memory, tile0 ascending
+    int ns;
+    int it0, n;                 // first time index, steps (role 2: descending indices)
     unsigned base;              // tag of the call's first step
     int *dead;                  // host-visible error word
+    int rec, illum;             // role 1: keep the record, accumulate the source illumination
+    int image_every;            // role 2
+    // role 1: where step k's P also goes, as floats from the shot's own P
+    // (0: nowhere); role 2: where step k's source P lies, from srcP
+    long long off[kRun2dMax];
 };
 
 // an opaque copy: what is derived from it inside the step loop is not hoisted
@@ -156,6 +152,18 @@ __device__ __forceinline__ float await(const unsigned long long *p, unsigned lon
     return __uint_as_float((unsigned)w);
 }
 
+// the shot of a tile (tile0 ascending)
+__device__ __forceinline__ int find_shot2d(const Run2dShot *s, int ns, int tile)
+{
+    int lo = 0, hi = ns - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s[mid].tile0 <= tile) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 // k / n and k % n of 0 <= k < 2^20 by a reciprocal (exact: the rounding is
 // far below the half added to k)
 __device__ __forceinline__ void divmod(int k, int n, float inv, int &q, int &r)
@@ -189,17 +197,25 @@ __device__ __forceinline__ float diff_z(const float *p)
 // fields of a damped one).  One cell a lane and 16 wavefronts a CU: four cells
 // a lane (16-byte LDS accesses, 8 wavefronts) took 3.8 against 3.6 us a step
 // at 400 x 400 and 14.9 against 14.1 at 2401 x 803.
-template <bool TTI, bool US, int NT, int NU>
+// ROLE 0: vti_step (source and record of one shot); 1: the source side of an
+// RTM, of many shots at once: record and illumination (first sweep), P into
+// checkpoints; 2: its receiver side, backward in time: the records written
+// into P and Q on the injection row before each step (only the velocity
+// update reads them: the split form of that row rebuilds P and Q), the image
+// img += P_source * P and, where asked for, the receiver illumination.
+template <bool TTI, bool US, int ROLE, int NT, int NU>
 __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
 {
     extern __shared__ float4 smem4[];
     float *sm = reinterpret_cast<float *>(smem4);
     __shared__ int s_dead;
     const int tid = threadIdx.x;
-    const Tile t = tile_of(a.nnx, a.nnz, a.gx, a.gz, blockIdx.x / a.gz, blockIdx.x % a.gz);
+    const Run2dShot &b = ROLE ? a.many[find_shot2d(a.many, a.ns, blockIdx.x)] : a.one;
+    const int tile = blockIdx.x - (ROLE ? b.tile0 : 0);
+    const Tile t = tile_of(b.nnx, b.nnz, b.gx, b.gz, tile / b.gz, tile % b.gz);
     const int nx = t.nx, nz = t.nz, x0 = t.x0, z0 = t.z0;
     const Lds<TTI> L(nx, nz);
-    const int ldz = a.ldz, zend = a.nnz - 4, xend = a.nnx - 4, M = a.M;
+    const int ldz = b.ldz, zend = b.nnz - 4, xend = b.nnx - 4, M = b.M;
     float *sP = sm + L.p0, *sQ = sm + L.oq + L.q0, *sU = sm + L.ou + L.u0, *sW = sm + L.ow + L.w0;
     float *sC = sm + L.oc + L.u0, *sS = sm + L.os + L.u0;   // TTI only
     float *kz1 = sm + L.ot + 4, *kz2 = kz1 + nz + 8;        // cells -4 .. nz + 3
@@ -213,24 +229,24 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         const bool q = k >= L.oq;
         const int i = q ? k - L.oq : k, pitch = q ? L.qp : L.pp;
         const int r = i / pitch - (q ? (TTI ? 7 : 0) : 7), c = i % pitch - ((q || TTI) ? 8 : 0);
-        *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? a.Q : a.P, a.nnx, ldz, x0 + r, z0 + c);
+        *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? b.f[7] : b.f[6], b.nnx, ldz, x0 + r, z0 + c);
     }
     for (int k = L.ou + 4 * tid; k < L.oc; k += 4 * NT) {   // u and w
         const bool q = k >= L.ow;
         const int i = q ? k - L.ow : k - L.ou, pitch = q ? L.wp : L.up;
         const int r = i / pitch - (q ? (TTI ? 4 : 0) : 4), c = i % pitch - ((q || TTI) ? 4 : 0);
-        *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? a.w : a.u, a.nnx, ldz, x0 + r, z0 + c);
+        *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? b.f[1] : b.f[0], b.nnx, ldz, x0 + r, z0 + c);
     }
     if (TTI)
         for (int k = L.oc + 4 * tid; k < L.ot; k += 4 * NT) {
             const bool q = k >= L.os;
             const int i = q ? k - L.os : k - L.oc;
-            *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? a.sth : a.cth, a.nnx, ldz, x0 + i / L.up - 4, z0 + i % L.up - 4);
+            *reinterpret_cast<float4 *>(sm + k) = ldg4(q ? b.sth : b.cth, b.nnx, ldz, x0 + i / L.up - 4, z0 + i % L.up - 4);
         }
-    auto tabv = [&](int row, int i) { return i >= 0 && i < M ? a.tab[(long long)row * M + i] : 0.0f; };
+    auto tabv = [&](int row, int i) { return i >= 0 && i < M ? b.tab[(long long)row * M + i] : 0.0f; };
     // velocity tables: VTI: coff1 * dt/dx (the reference's first product), coff2; TTI: the factors themselves
     for (int k = tid; k < nx + 7; k += NT) {
-        kx1[k - 4] = TTI ? tabv(0, x0 + k - 4) : tabv(0, x0 + k - 4) * a.dtx;
+        kx1[k - 4] = TTI ? tabv(0, x0 + k - 4) : tabv(0, x0 + k - 4) * b.dtx;
         kx2[k - 4] = tabv(1, x0 + k - 4);
     }
     for (int k = tid; k < nx; k += NT) {
@@ -238,7 +254,7 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         ax2[k] = tabv(7, x0 + k);
     }
     for (int k = tid; k < nz + 8; k += NT) {
-        kz1[k - 4] = TTI ? tabv(4, z0 + k - 4) : tabv(4, z0 + k - 4) * a.dtz;
+        kz1[k - 4] = TTI ? tabv(4, z0 + k - 4) : tabv(4, z0 + k - 4) * b.dtz;
         kz2[k - 4] = tabv(5, z0 + k - 4);
     }
     for (int k = tid; k < nz; k += NT) {
@@ -264,17 +280,17 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         if (!live || i >= rows) continue;
         const int x = x0 + r0 + i, z = z0 + c;
         const long long g = (long long)x * ldz + z;
-        const float v = a.vp[g];
-        float ee = a.ep[g], dd = a.de[g];
-        s0[i] = a.px[g];
-        s1[i] = a.qx[g];
-        s2[i] = a.pz[g];
-        s3[i] = a.qz[g];
+        const float v = b.vp[g];
+        float ee = b.ep[g], dd = b.de[g];
+        s0[i] = b.f[2][g];
+        s1[i] = b.f[4][g];
+        s2[i] = b.f[3][g];
+        s3[i] = b.f[5][g];
         const float tx1 = ax1[r0 + i], tx2 = ax2[r0 + i], tz1 = az1[c], tz2 = az2[c];
-        if (a.sv) {   // SV taper (GPU_vti2dfd_kernels.cu:260-278)
-            const int rx = x - a.cx, rz = z - a.cz, r2 = rx * rx + rz * rz;
-            if (r2 <= a.svR * a.svR) {
-                const double f = a.tap[r2];
+        if (b.sv) {   // SV taper (GPU_vti2dfd_kernels.cu:260-278)
+            const int rx = x - b.cx, rz = z - b.cz, r2 = rx * rx + rz * rz;
+            if (r2 <= b.svR * b.svR) {
+                const double f = b.tap[r2];
                 ee = (float)(f * (double)ee);
                 dd = (float)(f * (double)dd);
             }
@@ -288,28 +304,62 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
             c2[i] = g1 * v * v;
             c3[i] = tx2 * tz2;
         } else {
-            c0[i] = tx1 * v * v * e2 * a.dtx;
-            c1[i] = tx1 * v * v * sd * a.dtx;
-            c2[i] = tz1 * v * v * sd * a.dtz;
-            c3[i] = tz1 * v * v * a.dtz;
+            c0[i] = tx1 * v * v * e2 * b.dtx;
+            c1[i] = tx1 * v * v * sd * b.dtx;
+            c2[i] = tz1 * v * v * sd * b.dtz;
+            c3[i] = tz1 * v * v * b.dtz;
         }
-        if (US && tx1 == 1.0f && tx2 == 1.0f && tz1 == 1.0f && tz2 == 1.0f) {
+        if (US && z != b.split_z && tx1 == 1.0f && tx2 == 1.0f && tz1 == 1.0f && tz2 == 1.0f) {
             und |= 1 << i;
             s0[i] = sP[(r0 + i) * L.pp + c];
             s1[i] = sQ[(r0 + i) * L.qp + c];
         }
-        if (a.rec && z == a.rz) {
-            const int k = x - a.rx0;
-            if (k >= 0 && k % a.rdx == 0 && k / a.rdx < a.rnx) {
-                if (!recs) krec = k / a.rdx;
+        if (ROLE != 2 && b.rec && (!ROLE || a.rec) && z == b.rz) {
+            const int k = x - b.rx0;
+            if (k >= 0 && k % b.rdx == 0 && k / b.rdx < b.rnx) {
+                if (!recs) krec = k / b.rdx;
                 recs |= 1 << i;
             }
         }
     }
 
-    const int srow = a.sx - x0, scol = a.sz - z0;
-    const bool src_p = a.point && srow >= -7 && srow < nx + 7 && scol >= (TTI ? -8 : 0) && scol < nz + (TTI ? 8 : 0);
-    const bool src_q = a.point && srow >= (TTI ? -7 : 0) && srow < nx + (TTI ? 7 : 0) && scol >= -8 && scol < nz + 8;
+    // images: interior cell (r0 + i, c) at img[io + i * inz]
+    const bool inz_ok = ROLE && live && z0 + c >= b.inp && z0 + c < b.inp + b.inz;
+    const long long io = (long long)(x0 + row0 - b.inp) * b.inz + (z0 + col0 - b.inp);
+    const bool lit = ROLE == 1 ? a.illum != 0 : (ROLE == 2 && b.rillum);
+    int inn = 0;                               // rows of the strip in the interior
+    float il[ROLE ? NU : 1], im[ROLE == 2 ? NU : 1];
+    if (ROLE) {
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+            const int jx = x0 + row0 + i - b.inp;
+            il[i] = 0.0f;
+            if (ROLE == 2) im[i] = 0.0f;
+            if (!inz_ok || i >= rows || jx < 0 || jx >= b.inx) continue;
+            inn |= 1 << i;
+            if (lit) il[i] = b.illum[io + (long long)i * b.inz];
+            if (ROLE == 2) im[i] = b.img[io + (long long)i * b.inz];
+        }
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+            asm volatile("" : "+v"(il[i]));
+            if (ROLE == 2) asm volatile("" : "+v"(im[i]));
+        }
+    }
+    const bool clamp = ROLE == 1 && b.clamp;
+    // receiver samples of this lane's row of the injection row (tile and halo)
+    const int zi = ROLE == 2 ? b.rzi - z0 : 0;
+    const bool inj_p = ROLE == 2 && zi >= 0 && zi < nz, inj_q = ROLE == 2 && zi >= -8 && zi < nz + 8;
+    int kinj = -1;
+    if (inj_q && tid < nx + 14) {
+        const int k = x0 + tid - 7 - b.rx0;
+        if (k >= 0 && k % b.rdx == 0 && k / b.rdx < b.rnx) kinj = k / b.rdx;
+    }
+    const float *srcP = b.srcP;
+    float *ownP = b.f[6];
+    const int srow = b.sx - x0, scol = b.sz - z0;
+    const bool src_p = ROLE != 2 && b.point && srow >= -7 && srow < nx + 7 && scol >= (TTI ? -8 : 0) && scol < nz + (TTI ? 8 : 0);
+    const bool src_q = ROLE != 2 && b.point && srow >= (TTI ? -7 : 0) && srow < nx + (TTI ? 7 : 0) && scol >= -8 && scol < nz + 8;
 
     // the strip is in registers before the step loop, whose waits would
     // otherwise count these loads as possibly still on their way
@@ -319,19 +369,28 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
     if (US) __syncthreads();   // P and Q are in s0 and s1 before the source is added to them in LDS
     float amps = 0.0f;   // lane k: the gain of step k of the current 64
     for (int s = 0; s < a.n; ++s) {
-        const int it = a.it0 + s;
-        if ((s & 63) == 0) {
-            amps = a.amp[a.it0 + min(s + (tid & 63), a.n - 1)];
+        const int it = ROLE == 2 ? a.it0 - s : a.it0 + s;
+        if (ROLE != 2 && (s & 63) == 0) {
+            amps = b.amp[a.it0 + min(s + (tid & 63), a.n - 1)];
             // taken here: waited for at the top of each step, the load would
             // hold the step until the stores before it are acknowledged too
             asm volatile("" : "+v"(amps));
         }
-        const float amp = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(amps), s & 63));
+        const float amp = ROLE == 2 ? 0.0f : __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(amps), s & 63));
         const int vt = opaque(tid), r0 = opaque(row0), c = opaque(col0);
+        // what this step reads from memory: its latency passes behind the exchange
+        float inj = 0.0f, sp[ROLE == 2 ? NU : 1];
+        const bool imaged = ROLE == 2 && it % a.image_every == 0;
+        if (ROLE == 2) {
+            if (kinj >= 0) inj = b.rec[(long long)it * b.nrec + kinj];
+            const float *src = srcP + a.off[s] + (long long)(x0 + r0) * ldz + z0 + c;
+#pragma unroll
+            for (int i = 0; i < NU; ++i) sp[i] = imaged && (inn >> i & 1) ? src[(long long)i * ldz] : 0.0f;
+        }
         if (s > 0) {
             // ---- the neighbours' outer rows and columns of the last step ----
             const unsigned tag = a.base + s;
-            const unsigned long long *gP = a.xP + (s & 1) * a.xstride, *gQ = a.xQ + (s & 1) * a.xstride;
+            const unsigned long long *gP = b.xP + (s & 1) * b.xstride, *gQ = b.xQ + (s & 1) * b.xstride;
             const int nrow = 14 * nz;
             const int wide = 14 * (nz + 14), nget = (TTI ? wide : nrow) + 14 * nx;
             const int total = TTI ? 2 * nget : nget;
@@ -371,7 +430,15 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 return;
             }
         }
-        if (amp != 0.0f && (src_p || src_q)) {   // P[src] += amp, Q[src] += amp before the update (add_source2d :204-205)
+        if (ROLE == 2 && inj_q) {   // shot_record(load) Toa_gpu2DvtiFdRtmAdcigsLaplace.cu:525-528
+            if (kinj >= 0) {
+                const int r = tid - 7;
+                if (inj_p) sP[r * L.pp + zi] = inj;
+                if (r >= 0 && r < nx) sQ[r * L.qp + zi] = inj;
+            }
+            __syncthreads();
+        }
+        if (ROLE != 2 && amp != 0.0f && (src_p || src_q)) {   // P[src] += amp, Q[src] += amp before the update (add_source2d :204-205)
             if (tid == 0) {
                 if (src_p) sP[srow * L.pp + scol] += amp;
                 if (src_q) sQ[srow * L.qp + scol] += amp;
@@ -416,8 +483,8 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                             const float cs = sC[(r + i) * L.up + cc], sn = sS[(r + i) * L.up + cc];
                             const float Pz = diff_z<1>(p + i * L.pp), Qx = diff8(h + i), Qz = diff_z<1>(q + i * L.qp);
                             const float g2 = k2 * z2, g1 = k1 * z1;
-                            const float u = g2 * *pu - g1 * (cs * a.dtx * d - sn * a.dtz * Pz);
-                            const float w = g2 * *pw - g1 * (sn * a.dtx * Qx + cs * a.dtz * Qz);
+                            const float u = g2 * *pu - g1 * (cs * b.dtx * d - sn * b.dtz * Pz);
+                            const float w = g2 * *pw - g1 * (sn * b.dtx * Qx + cs * b.dtz * Qz);
                             if (on) {
                                 *pu = u;
                                 *pw = w;
@@ -445,9 +512,10 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
 
         // ---- stress update of the tile ----
         if (live) {
-            const int nr = opaque(rows), ub = opaque(und), rb = opaque(recs);
-            const bool foot = !a.point && amp != 0.0f, more = s + 1 < a.n;
-            unsigned long long *gP = a.xP + ((s + 1) & 1) * a.xstride, *gQ = a.xQ + ((s + 1) & 1) * a.xstride;
+            const int nr = opaque(rows), ub = opaque(und), rb = opaque(recs), in_ = ROLE ? opaque(inn) : 0;
+            float *keep = ROLE == 1 && a.off[s] ? ownP + a.off[s] : nullptr;
+            const bool foot = ROLE == 0 && !b.point && amp != 0.0f, more = s + 1 < a.n;
+            unsigned long long *gP = b.xP + ((s + 1) & 1) * b.xstride, *gQ = b.xQ + ((s + 1) & 1) * b.xstride;
             const unsigned tag = a.base + s + 1;
             const bool ez = c < 7 || c >= nz - 7;
             const float *pu = sU + r0 * L.up + c, *pw = sW + r0 * L.wp + c;
@@ -466,8 +534,8 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 if (TTI) {   // the rotated x derivative of u and z derivative of w
                     const float uz = diff_z<0>(pu + i * L.up), wx = diff8(h + i);
                     const float cs = sC[r * L.up + c], sn = sS[r * L.up + c];
-                    xx = cs * a.dtx * xx - sn * a.dtz * uz;
-                    zz = sn * a.dtx * wx + cs * a.dtz * zz;
+                    xx = cs * b.dtx * xx - sn * b.dtz * uz;
+                    zz = sn * b.dtx * wx + cs * b.dtz * zz;
                 }
                 float Pn, Qn;
                 if (US && (ub >> i & 1)) {
@@ -482,9 +550,9 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                     Pn = s0[i] + s2[i];
                     Qn = s1[i] + s3[i];
                     if (foot) {   // P = px+pz+s (CPU_vti2dfd_kernels.c:173-174), 7x7 footprint
-                        const int fdx = x0 + r - a.sx, fdz = z0 + c - a.sz;
+                        const int fdx = x0 + r - b.sx, fdz = z0 + c - b.sz;
                         if (fdx >= -3 && fdx <= 3 && fdz >= -3 && fdz <= 3) {
-                            const float sc = (float)((double)amp * a.gw[(fdx + 3) * 7 + (fdz + 3)]);
+                            const float sc = (float)((double)amp * b.gw[(fdx + 3) * 7 + (fdz + 3)]);
                             Pn = Pn + sc;
                             Qn = Qn + sc;
                         }
@@ -499,9 +567,17 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                     if (ex || (TTI && ez)) put(gP + g, Pn, tag);
                     if (ez || (TTI && ex)) put(gQ + g, Qn, tag);
                 }
-                if (rb >> i & 1) {
+                if (ROLE && (in_ >> i & 1)) {
+                    if (lit) {   // cal_illumination :654-677
+                        il[i] += Pn * Pn + Qn * Qn;
+                        if (clamp && il[i] <= 0.0f) il[i] = 1.0f;
+                    }
+                    if (ROLE == 2 && imaged) im[i] += sp[i] * Pn;   // cal_migration :679-698
+                }
+                if (ROLE == 1 && keep) keep[(long long)(x0 + r) * ldz + z0 + c] = Pn;
+                if (ROLE != 2 && (rb >> i & 1)) {
                     const int k = krec + __popc(rb & ((1 << i) - 1));
-                    a.rec[(long long)it * a.nrec + k] = a.rec_kind == 0 ? Pn : (a.rec_kind == 1 ? Pn + Pn : Pn + Qn);
+                    b.rec[(long long)it * b.nrec + k] = b.rec_kind == 0 ? Pn : (b.rec_kind == 1 ? Pn + Pn : Pn + Qn);
                 }
             }
         }
@@ -509,27 +585,35 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
     }
 
     // ---- write the tile back (n >= 2: every neighbour has loaded its halo) ----
-    // the field pointers come from the argument segment again: held through
-    // the loop they would cost the registers that it needs
+    // the field pointers come from memory again: held through the loop they
+    // would cost the registers that it needs
     using KArgs = const __attribute__((address_space(4))) Run2dArgs;
-    KArgs *b = (KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(b));
-    float *gu = b->u, *gw = b->w, *gP = b->P, *gQ = b->Q, *gpx = b->px, *gqx = b->qx, *gpz = b->pz, *gqz = b->qz;
+    KArgs *ka = (KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    const Run2dShot *bm = ROLE ? &b : nullptr;
+    asm volatile("" : "+s"(bm));
+    float *gf[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) gf[k] = ROLE ? bm->f[k] : ka->one.f[k];
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
         if (i >= rows) continue;
         const int r = r0 + i;
         const long long g = (long long)(x0 + r) * ldz + z0 + c;
-        gu[g] = sU[r * L.up + c];
-        gw[g] = sW[r * L.wp + c];
-        gP[g] = sP[r * L.pp + c];
-        gQ[g] = sQ[r * L.qp + c];
+        gf[0][g] = sU[r * L.up + c];
+        gf[1][g] = sW[r * L.wp + c];
+        gf[6][g] = sP[r * L.pp + c];
+        gf[7][g] = sQ[r * L.qp + c];
+        if (ROLE && (inn >> i & 1)) {
+            if (lit) b.illum[io + (long long)i * b.inz] = il[i];
+            if (ROLE == 2) b.img[io + (long long)i * b.inz] = im[i];
+        }
         if (US && (und >> i & 1)) continue;   // no split fields there
-        gpx[g] = s0[i];
-        gqx[g] = s1[i];
-        gpz[g] = s2[i];
-        gqz[g] = s3[i];
+        gf[2][g] = s0[i];
+        gf[4][g] = s1[i];
+        gf[3][g] = s2[i];
+        gf[5][g] = s3[i];
     }
 }
 
@@ -541,31 +625,178 @@ struct Shape2d {
 };
 constexpr Shape2d kShapes[] = {{512, 1}, {1024, 1}, {1024, 2}, {1024, 3}, {1024, 4}, {1024, 6}, {1024, 8}};
 constexpr int kNumShapes = (int)(sizeof(kShapes) / sizeof(kShapes[0]));
+constexpr int kRtmShapes = kNumShapes - 1;   // the RTM roles' images leave no registers for strips of 8
 
-template <bool TTI, bool US>
+template <bool TTI, bool US, int ROLE>
 KernelFn kernel_of(int shape)
 {
     switch (shape) {
-    case 0: return run2d_kernel<TTI, US, 512, 1>;
-    case 1: return run2d_kernel<TTI, US, 1024, 1>;
-    case 2: return run2d_kernel<TTI, US, 1024, 2>;
-    case 3: return run2d_kernel<TTI, US, 1024, 3>;
-    case 4: return run2d_kernel<TTI, US, 1024, 4>;
-    case 5: return run2d_kernel<TTI, US, 1024, 6>;
-    default: return run2d_kernel<TTI, US, 1024, 8>;
+    case 0: return run2d_kernel<TTI, US, ROLE, 512, 1>;
+    case 1: return run2d_kernel<TTI, US, ROLE, 1024, 1>;
+    case 2: return run2d_kernel<TTI, US, ROLE, 1024, 2>;
+    case 3: return run2d_kernel<TTI, US, ROLE, 1024, 3>;
+    case 4: return run2d_kernel<TTI, US, ROLE, 1024, 4>;
+    case 5: return run2d_kernel<TTI, US, ROLE, 1024, 6>;
+    default: return run2d_kernel<TTI, US, ROLE, 1024, ROLE ? 6 : 8>;
     }
+}
+
+// Tiles of one grid: at least 7 rows and 8 columns (a halo never reaches past
+// the next tile), small enough for LDS and for one strip per thread.  cost:
+// the estimated cycles of the largest tile's step: instructions at one
+// wavefront instruction a cycle and CU (about 20 a velocity cell, 26 with its
+// z-stencil, 50 a stress cell; the TTI update twice that), or, where few
+// wavefronts leave the CU waiting, the rounds of strips by their latency;
+// and the exchanged words.
+struct Cut {
+    int gx, gz, tiles;
+    size_t lds;
+    double cost;
+};
+void cuts_of(int nnx, int nnz, bool tti, int shape, int cus, int lds_max, std::vector<Cut> &out)
+{
+    out.clear();
+    const int ux = nnx - 8, uq = (nnz - 8 + 3) / 4;
+    if (uq < 2) return;
+    const int nt = kShapes[shape].nt, nu = kShapes[shape].nu;
+    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); ++gx)
+        for (int gz = 1; gz <= std::min(cus / gx, std::max(1, uq / 2)); ++gz) {
+            const int nx = (ux + gx - 1) / gx, nz = 4 * ((uq + gz - 1) / gz);
+            const int strips = (nx + nu - 1) / nu * nz;
+            if (strips > nt || nx + 14 > nt) continue;
+            const size_t b = 4 * (size_t)(tti ? Lds<true>(nx, nz).total : Lds<false>(nx, nz).total);
+            if (b + 64 > (size_t)lds_max) continue;
+            const int us = (nx + 7 + nu - 1) / nu * (tti ? nz + 8 : nz), ws = tti ? 0 : (nx + nu - 1) / nu * (nz + 8);
+            const double f = tti ? 2.0 : 1.0;
+            const double issue = f * nu * (20.0 * us + 26.0 * ws + 50.0 * strips) / 64.0;
+            const double wait = f * ((us + ws + nt - 1) / nt * (350.0 + 60.0 * nu) + 300.0 + 90.0 * nu);
+            const double words = (tti ? 2.0 : 1.0) * 14.0 * (nx + nz + (tti ? 14 : 0));
+            out.push_back(Cut{gx, gz, gx * gz, b, std::max(issue, wait) + 0.25 * words});
+        }
+}
+
+struct Device2d {
+    int cus = 0, lds = 0;
+};
+bool device_2d(int device, Device2d &d)
+{
+    int coop = 0;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !coop ||
+        hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipDeviceGetAttribute(&d.lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// One tile per CU for all shots together, the same launch shape: the shape
+// and the cuts with the least cost of the slowest tile.
+bool plan_group(std::vector<Run2dShot> &shots, bool tti, int nshape, const Device2d &d, int &shape, size_t &lds, int &ntile)
+{
+    const int ns = (int)shots.size();
+    double best = 1e300;
+    std::vector<Cut> pick(ns), chosen;
+    for (int k = 0; k < nshape; ++k) {
+        std::vector<std::vector<Cut>> cuts(ns);
+        std::vector<double> costs;
+        bool all = true;
+        for (int s = 0; s < ns && all; ++s) {
+            cuts_of(shots[s].nnx, shots[s].nnz, tti, k, d.cus, d.lds, cuts[s]);
+            all = !cuts[s].empty();
+            for (const Cut &c : cuts[s]) costs.push_back(c.cost);
+        }
+        if (!all) continue;
+        std::sort(costs.begin(), costs.end());
+        auto fits = [&](double c) {   // fewest tiles of every shot within cost c
+            int n = 0;
+            for (int s = 0; s < ns; ++s) {
+                const Cut *b = nullptr;
+                for (const Cut &x : cuts[s])
+                    if (x.cost <= c && (!b || x.tiles < b->tiles || (x.tiles == b->tiles && x.cost < b->cost))) b = &x;
+                if (!b || (n += b->tiles) > d.cus) return false;
+                pick[s] = *b;
+            }
+            return true;
+        };
+        size_t lo = 0, hi = costs.size();
+        while (lo < hi) {   // the least cost that fits
+            const size_t mid = (lo + hi) / 2;
+            if (fits(costs[mid])) hi = mid;
+            else lo = mid + 1;
+        }
+        if (lo == costs.size() || costs[lo] >= best || !fits(costs[lo])) continue;
+        best = costs[lo];
+        shape = k;
+        chosen = pick;
+    }
+    if (best == 1e300) return false;
+    lds = 0;
+    ntile = 0;
+    for (int s = 0; s < ns; ++s) {
+        shots[s].gx = chosen[s].gx;
+        shots[s].gz = chosen[s].gz;
+        shots[s].tile0 = ntile;
+        ntile += chosen[s].tiles;
+        lds = std::max(lds, chosen[s].lds);
+    }
+    return true;
+}
+
+size_t plane_of(const Run2dShot &s) { return (size_t)s.ldz * s.nnx; }
+
+// the exchange planes of every shot, zeroed, and the error word
+bool alloc_group(std::vector<Run2dShot> &shots, unsigned long long *&xbuf, int *&dead, hipStream_t s)
+{
+    size_t n = 0;
+    for (const Run2dShot &b : shots) n += 4 * plane_of(b);
+    if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess ||
+        launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    *dead = 0;
+    unsigned long long *p = xbuf;
+    for (Run2dShot &b : shots) {
+        b.xstride = (long long)plane_of(b);
+        b.xP = p;
+        b.xQ = p + 2 * plane_of(b);
+        p += 4 * plane_of(b);
+    }
+    return true;
+}
+
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
+{
+    void *args[] = {&a};
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+            hipSuccess ||
+        hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
 }
 
 }  // namespace
 
 struct Run2dPlan {
     int ok = 0;                 // 1: usable, -1: this grid or device takes the per-step kernels
-    int gx = 0, gz = 0, shape = 0;
+    std::vector<Run2dShot> shot;   // one: the plan's share of it
+    int shape = 0, ntile = 0;
     size_t lds = 0;
     bool tti = false;
-    unsigned long long *xbuf = nullptr;   // xP[2], xQ[2]
-    unsigned base = 1;          // the planes start with tag 0
-    int *dead = nullptr;        // pinned, mapped
+    unsigned long long *xbuf = nullptr;
+    unsigned base = 1;
+    int *dead = nullptr;
 };
 
 void run2d_free(vti_ctx *c)
@@ -577,101 +808,16 @@ void run2d_free(vti_ctx *c)
     c->run2d = nullptr;
 }
 
-namespace {
-
-// Tiles: at most one per CU, at least 7 rows and 8 columns (a halo never
-// reaches past the next tile), small enough for LDS and for one strip per
-// thread.  Among those the least estimated cycles of the largest tile's step:
-// instructions at one wavefront instruction a cycle and CU (about 20 a
-// velocity cell, 26 with its z-stencil, 50 a stress cell; the TTI update
-// twice that), or, where few wavefronts leave the CU waiting, the rounds of
-// strips by their latency; and the exchanged words.
-bool plan_tiles(int nnx, int nnz, bool tti, int cus, int lds_max, Run2dPlan &p)
+// The forward side of a context's shot on state s.
+Run2dShot run2d_shot(vti_ctx *c, const VtiState &s)
 {
-    const int ux = nnx - 8, uq = (nnz - 8 + 3) / 4;
-    double best = 1e300;
-    if (uq < 2) return false;
-    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); ++gx)
-        for (int gz = 1; gz <= std::min(cus / gx, std::max(1, uq / 2)); ++gz) {
-            const int nx = (ux + gx - 1) / gx, nz = 4 * ((uq + gz - 1) / gz);
-            const size_t b = 4 * (size_t)(tti ? Lds<true>(nx, nz).total : Lds<false>(nx, nz).total);
-            if (b + 64 > (size_t)lds_max) continue;
-            for (int k = 0; k < kNumShapes; ++k) {
-                const int nt = kShapes[k].nt, nu = kShapes[k].nu;
-                const int strips = (nx + nu - 1) / nu * nz;
-                if (strips > nt) continue;
-                const int us = (nx + 7 + nu - 1) / nu * (tti ? nz + 8 : nz), ws = tti ? 0 : (nx + nu - 1) / nu * (nz + 8);
-                const double f = tti ? 2.0 : 1.0;
-                const double issue = f * nu * (20.0 * us + 26.0 * ws + 50.0 * strips) / 64.0;
-                const double wait = f * ((us + ws + nt - 1) / nt * (350.0 + 60.0 * nu) + 300.0 + 90.0 * nu);
-                const double words = (tti ? 2.0 : 1.0) * 14.0 * (nx + nz + (tti ? 14 : 0));
-                const double cost = std::max(issue, wait) + 0.25 * words;
-                if (cost < best) {
-                    best = cost;
-                    p.gx = gx;
-                    p.gz = gz;
-                    p.lds = b;
-                    p.shape = k;
-                }
-            }
-        }
-    return best < 1e300;
-}
-
-}  // namespace
-
-// n steps from it0 of the main state, when one resident launch applies:
-// 1 launched, 0 not applicable (the caller runs the per-step kernels), < 0
-// an error.
-int run2d_steps(vti_ctx *c, int it0, int n)
-{
-    // Two steps let the write-back start after every neighbour has loaded.
-    // Below eight the call's fixed cost (a cooperative launch, the tile's
-    // coefficients, load and store) is more than the per-step kernels take
-    // (5.8 us a step and up).
-    if (c->cfg.ndim != 2 || n < 8 || c->cfg.mode == VTI_MODE_OMP_REF || !c->damp) return 0;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 0;
-    const bool tti = c->tti != nullptr;
-    if (c->run2d && c->run2d->tti != tti) {
-        if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
-        run2d_free(c);
-    }
-    if (!c->run2d) {
-        c->run2d = new (std::nothrow) Run2dPlan();
-        if (!c->run2d) return 0;
-        Run2dPlan &p = *c->run2d;
-        p.tti = tti;
-        p.ok = -1;
-        int coop = 0, cus = 0, lds = 0;
-        if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess ||
-            hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        if (!plan_tiles(c->g.nnx, c->g.nnz, tti, cus, lds, p)) return 0;
-        if (hipMalloc(&p.xbuf, 4 * c->nvol * sizeof(unsigned long long)) != hipSuccess ||
-            hipHostMalloc(&p.dead, sizeof(int), hipHostMallocMapped) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        *p.dead = 0;
-        if (launch_zero(reinterpret_cast<float *>(p.xbuf), 8 * c->nvol, c->stream) != hipSuccess)
-            return fail(VTI_ERR_HIP, "run2d: exchange planes");
-        p.ok = 1;
-    }
-    Run2dPlan &p = *c->run2d;
-    if (p.ok != 1) return 0;
-    const VtiState s = main_state(c);
-    Run2dArgs a{};
+    Run2dShot a{};
     a.nnx = c->g.nnx; a.nnz = c->g.nnz; a.ldz = c->g.ldz; a.M = c->nnmax;
-    a.u = s.f[VTI_F_U]; a.w = s.f[VTI_F_W];
-    a.px = s.f[VTI_F_PX]; a.pz = s.f[VTI_F_PZ]; a.qx = s.f[VTI_F_QX]; a.qz = s.f[VTI_F_QZ];
-    a.P = s.f[VTI_F_P]; a.Q = s.f[VTI_F_Q];
+    static const int kF[8] = {VTI_F_U, VTI_F_W, VTI_F_PX, VTI_F_PZ, VTI_F_QX, VTI_F_QZ, VTI_F_P, VTI_F_Q};
+    for (int k = 0; k < 8; ++k) a.f[k] = s.f[kF[k]];
     a.vp = c->vp; a.ep = c->ep; a.de = c->de;
     a.cth = c->tti;
-    a.sth = tti ? c->tti + c->nvol : nullptr;
+    a.sth = c->tti ? c->tti + c->nvol : nullptr;
     a.tab = c->tab;
     a.dtx = c->cfg.dt / c->cfg.dx; a.dtz = c->cfg.dt / c->cfg.dz;
     a.sv = c->cfg.sv != 0; a.svR = c->cfg.sv_R; a.cx = c->shot.sv_cx; a.cz = c->shot.sv_cz;
@@ -683,21 +829,54 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     a.rec = c->nrec > 0 ? c->rec : nullptr;
     a.nrec = c->nrec; a.rec_kind = c->cfg.rec_kind;
     a.rz = c->shot.rec_z; a.rx0 = c->shot.rec_x0; a.rdx = c->shot.rec_dx; a.rnx = c->shot.rec_nx;
+    a.split_z = a.rzi = -1;
+    a.inp = c->cfg.npml; a.inx = c->cfg.nx; a.inz = c->cfg.nz;
+    return a;
+}
+
+// n steps from it0 of the main state, when one resident launch applies:
+// 1 launched, 0 not applicable (the caller runs the per-step kernels), < 0
+// an error.
+int run2d_steps(vti_ctx *c, int it0, int n)
+{
+    // Two steps let the write-back start after every neighbour has loaded.
+    // Below eight the call's fixed cost (a cooperative launch, the tile's
+    // coefficients, load and store) is more than the per-step kernels take
+    // (5.8 us a step and up).
+    if (c->cfg.ndim != 2 || n < 8 || c->cfg.mode == VTI_MODE_OMP_REF || capturing(c->stream)) return 0;
+    const bool tti = c->tti != nullptr;
+    if (c->run2d && c->run2d->tti != tti) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
+        run2d_free(c);
+    }
+    if (!c->run2d) {
+        c->run2d = new (std::nothrow) Run2dPlan();
+        if (!c->run2d) return 0;
+        Run2dPlan &p = *c->run2d;
+        p.tti = tti;
+        p.ok = -1;
+        Device2d d;
+        p.shot.push_back(run2d_shot(c, main_state(c)));
+        if (!device_2d(c->device, d) || !plan_group(p.shot, tti, kNumShapes, d, p.shape, p.lds, p.ntile) ||
+            !alloc_group(p.shot, p.xbuf, p.dead, c->stream))
+            return 0;
+        p.ok = 1;
+    }
+    Run2dPlan &p = *c->run2d;
+    if (p.ok != 1) return 0;
+    Run2dArgs a{};
+    const Run2dShot &t = p.shot[0];
+    a.one = run2d_shot(c, main_state(c));
+    a.one.gx = t.gx; a.one.gz = t.gz;
+    a.one.xP = t.xP; a.one.xQ = t.xQ; a.one.xstride = t.xstride;
+    a.ns = 1;
     a.it0 = it0; a.n = n;
-    a.gx = p.gx; a.gz = p.gz;
-    a.xP = p.xbuf; a.xQ = p.xbuf + 2 * c->nvol;
-    a.xstride = (long long)c->nvol;
     a.base = p.base;
     a.dead = p.dead;
     const bool us = c->unsplit && c->cfg.mode == VTI_MODE_GPU_REF && !tti;
-    const KernelFn k = tti ? kernel_of<true, false>(p.shape)
-                           : (us ? kernel_of<false, true>(p.shape) : kernel_of<false, false>(p.shape));
-    void *args[] = {&a};
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) !=
-            hipSuccess ||
-        hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(p.gx * p.gz), dim3(kShapes[p.shape].nt), args,
-                                   (unsigned)p.lds, c->stream) != hipSuccess) {
-        (void)hipGetLastError();
+    const KernelFn k = tti ? kernel_of<true, false, 0>(p.shape)
+                           : (us ? kernel_of<false, true, 0>(p.shape) : kernel_of<false, false, 0>(p.shape));
+    if (!launch_coop(k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream)) {
         p.ok = -1;
         return 0;
     }
@@ -706,13 +885,152 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     return 1;
 }
 
-// after the context's stream has been waited for: an exchange that never came
-int run2d_check(vti_ctx *c)
+static int dead_check(int *dead, int &ok)
 {
-    if (!c->run2d || !c->run2d->dead || !*c->run2d->dead) return VTI_OK;
-    *c->run2d->dead = 0;
-    c->run2d->ok = -1;          // later steps take the per-step kernels
+    if (!dead || !*dead) return VTI_OK;
+    *dead = 0;
+    ok = -1;          // later steps take the per-step kernels
     return fail(VTI_ERR_HIP, "resident 2D steps: a tile's exchange did not arrive");
+}
+
+// after the context's stream has been waited for: an exchange that never came
+int run2d_check(vti_ctx *c) { return c->run2d ? dead_check(c->run2d->dead, c->run2d->ok) : VTI_OK; }
+
+// ---- groups of shots (RTM) ---------------------------------------------------
+int run2d_fit(const std::vector<Run2dShot> &shots, int first, int device)
+{
+    Device2d d;
+    if (!device_2d(device, d)) return 0;
+    int n = 0, tiles = 0;
+    std::vector<Cut> cuts;
+    for (size_t s = first; s < shots.size(); ++s, ++n) {
+        cuts_of(shots[s].nnx, shots[s].nnz, false, kRtmShapes - 1, d.cus, d.lds, cuts);
+        int least = d.cus + 1;
+        for (const Cut &c : cuts) least = std::min(least, c.tiles);
+        if ((tiles += least) > d.cus) break;
+    }
+    return n;
+}
+
+int run2d_group_make(Run2dGroup &g, const std::vector<Run2dShot> &src, const std::vector<Run2dShot> &rcv, bool us,
+                     int device, hipStream_t s)
+{
+    g.ok = 0;
+    if (src.empty() || capturing(s)) return 0;
+    Device2d d;
+    g.side[0] = src;
+    g.side[1] = rcv;
+    g.ns = (int)src.size();
+    g.us = us;
+    if (!device_2d(device, d) || !plan_group(g.side[0], false, kRtmShapes, d, g.shape, g.lds, g.ntile) ||
+        !alloc_group(g.side[0], g.xbuf, g.dead, s))
+        return 0;
+    for (int k = 0; k < g.ns; ++k) {
+        const Run2dShot &a = g.side[0][k];
+        Run2dShot &b = g.side[1][k];
+        b.gx = a.gx; b.gz = a.gz; b.tile0 = a.tile0;
+        b.xP = a.xP; b.xQ = a.xQ; b.xstride = a.xstride;
+    }
+    if (hipMalloc(&g.dev, 2 * g.ns * sizeof(Run2dShot)) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    if (hipMemcpy(g.dev, g.side[0].data(), g.ns * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(g.dev + g.ns, g.side[1].data(), g.ns * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess)
+        return fail(VTI_ERR_HIP, "run2d: descriptors");
+    g.ok = 1;
+    return 1;
+}
+
+void run2d_group_free(Run2dGroup &g)
+{
+    (void)hipFree(g.dev);
+    (void)hipFree(g.xbuf);
+    (void)hipHostFree(g.dead);
+    g.dev = nullptr;
+    g.xbuf = nullptr;
+    g.dead = nullptr;
+    g.ok = 0;
+}
+
+int run2d_group_run(Run2dGroup &g, int role, int it0, int n, bool rec, bool illum, int image_every, const long long *off,
+                    hipStream_t s)
+{
+    if (g.ok != 1 || n < 2 || n > kRun2dMax) return 0;
+    Run2dArgs a{};
+    a.many = g.dev + (role == 2 ? g.ns : 0);
+    a.ns = g.ns;
+    a.it0 = it0; a.n = n;
+    a.base = g.base;
+    a.dead = g.dead;
+    a.rec = rec; a.illum = illum;
+    a.image_every = image_every;
+    std::copy(off, off + n, a.off);
+    const KernelFn k = role == 1 ? (g.us ? kernel_of<false, true, 1>(g.shape) : kernel_of<false, false, 1>(g.shape))
+                                 : (g.us ? kernel_of<false, true, 2>(g.shape) : kernel_of<false, false, 2>(g.shape));
+    if (!launch_coop(k, g.ntile, kShapes[g.shape].nt, g.lds, a, s)) {
+        g.ok = -1;
+        return 0;
+    }
+    g.base += (unsigned)n;
+    return 1;
+}
+
+int run2d_group_check(Run2dGroup &g) { return dead_check(g.dead, g.ok); }
+
+int RtmQueue::forward(bool first, int it)
+{
+    const int k = first ? 1 : 2;
+    if (n && (kind != k || it != it0 + n || n == kRun2dMax)) {
+        const int e = flush();
+        if (e) return e;
+    }
+    if (!n) {
+        kind = k;
+        it0 = it;
+    }
+    off[n++] = 0;
+    return VTI_OK;
+}
+
+int RtmQueue::keep_last(long long o)
+{
+    if (n && kind != 3 && !off[n - 1]) {
+        off[n - 1] = o;
+        return VTI_OK;
+    }
+    const int e = flush();
+    return e ? e : keep(o);
+}
+
+int RtmQueue::receiver(int it, long long o)
+{
+    if (n && (kind != 3 || it != it0 - n || n == kRun2dMax)) {
+        const int e = flush();
+        if (e) return e;
+    }
+    if (!n) {
+        kind = 3;
+        it0 = it;
+    }
+    off[n++] = o;
+    return VTI_OK;
+}
+
+int RtmQueue::flush()
+{
+    const int m = n;
+    n = 0;
+    if (m >= kMinRun) {
+        const int e = kind == 3 ? run_receive(it0, m, off) : run_forward(kind == 1, it0, m, off);
+        if (e) return e < 0 ? e : VTI_OK;
+    }
+    for (int k = 0; k < m; ++k) {
+        int e = kind == 3 ? receive(it0 - k, off[k]) : step(kind == 1, it0 + k);
+        if (!e && kind != 3 && off[k]) e = keep(off[k]);
+        if (e) return e;
+    }
+    return VTI_OK;
 }
 
 }  // namespace vti
