@@ -443,71 +443,81 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
     op.consume_slot = [&](int k, int i) { return consume_from(rc.ck.view[i], k); };
     c->rtm_illum_mode = o->illum_mode;
 
-    // 2D: runs of steps of either side as resident launches.  The kernel
-    // images and injects inside the updated region only, so the interior and
-    // every receiver must lie in it; the TTI update and the gathers go step
-    // by step.
+    // 2D: the schedule as resident launches, one for the first sweep and one
+    // for the rest.  The kernel images and injects inside the updated region
+    // only, so the interior and every receiver must lie in it; the TTI update
+    // and the gathers go step by step.
     Run2dGroup grp;
     struct GroupGuard {
         Run2dGroup &g;
         ~GroupGuard() { run2d_group_free(g); }
     } group_guard{grp};
-    RtmQueue q;
-    if (nd == 2 && nt >= 8 && c->cfg.mode == VTI_MODE_GPU_REF && !c->tti && !c->adcig && c->cfg.npml >= 4 &&
-        c->shot.rec_x0 >= 4 && c->shot.rec_x0 + (c->shot.rec_nx - 1) * c->shot.rec_dx < c->g.nnx - 4 &&
-        c->shot.rec_z >= 4 && c->shot.rec_z < c->g.nnz - 4) {
-        Run2dShot a = run2d_shot(c, W), b = run2d_shot(c, rc.g);
+    RtmProgram q;
+    const float *P = W.f[VTI_F_P];
+    const CkSlots &ck = rc.ck;
+    auto apart = [](const float *a, const float *b) {   // floats from b to a
+        return ((long long)reinterpret_cast<intptr_t>(a) - (long long)reinterpret_cast<intptr_t>(b)) / (long long)sizeof(float);
+    };
+    const vti_shot &sh = c->shot;
+    bool same = true;   // a whole-state checkpoint is laid out as the state is
+    for (int k = 0; k < (int)(sizeof(W.f) / sizeof(W.f[0])) && !ck.compact; ++k)
+        for (int i = 0; i < nslot; ++i)
+            same = same && (!W.f[k] || apart(ck.view[i].f[k], W.f[k]) == apart(ck.mem[i], W.f[VTI_F_U]));
+    if (nd == 2 && nt >= 8 && same && c->cfg.mode == VTI_MODE_GPU_REF && !c->tti && !c->adcig && c->cfg.npml >= 4 &&
+        sh.rec_x0 >= 4 && sh.rec_x0 + (sh.rec_nx - 1) * sh.rec_dx < c->g.nnx - 4 && sh.rec_z >= 4 &&
+        sh.rec_z < c->g.nnz - 4) {
+        Run2dShot a = run2d_shot(c, W);
+        const Run2dShot b = run2d_shot(c, rc.g);
+        std::copy(b.f, b.f + 8, a.g);
         a.sv = svf;
-        b.sv = svb;
-        a.img = b.img = c->img;
-        a.illum = b.illum = c->illum;
+        a.svr = svb;
+        a.img = c->img;
+        a.illum = c->illum;
         a.clamp = clamp;
-        b.rillum = o->illum_mode == 1;
-        b.split_z = b.rzi = inj_z;
-        b.srcP = W.f[VTI_F_P];
-        if ((st = run2d_group_make(grp, {a}, {b}, c->unsplit, c->device, c->stream)) < 0) return st;
+        a.rillum = o->illum_mode == 1;
+        a.split_z = a.rzi = inj_z;
+        a.packed = ck.compact;
+        a.pxlo = ck.q.xlo; a.pxhi = ck.q.xhi; a.pzlo = ck.q.zlo; a.pzhi = ck.q.zhi;
+        a.pvol = (long long)c->nvol;
+        a.psplit = ck.q.split_n;
+        if ((st = run2d_group_make(grp, {a}, c->unsplit, c->device, c->stream)) < 0) return st;
     }
     if (grp.ok == 1) {
-        const float *P = W.f[VTI_F_P];
-        auto slot_off = [&](int i) {
-            return ((long long)reinterpret_cast<intptr_t>(rc.ck.view[i].f[VTI_F_P]) -
-                    (long long)reinterpret_cast<intptr_t>(P)) / (long long)sizeof(float);
+        if ((st = op.zero())) return st;   // the border cells, which no step changes
+        auto slot_p = [&, apart, P](int i) { return apart(rc.ck.view[i].f[VTI_F_P], P); };
+        auto slot_s = [&, apart](int i) { return apart(rc.ck.mem[i], W.f[VTI_F_U]); };
+        auto slot_of = [&, apart](long long off) {
+            for (int i = 0; i < nslot; ++i)
+                if (apart(rc.ck.mem[i], W.f[VTI_F_U]) == off) return i;
+            return -1;
         };
-        auto at = [&](long long off) {
+        auto at = [P](long long off) {
             VtiState s;
             s.f[VTI_F_P] = const_cast<float *>(P) + off;
             return s;
         };
-        q.run_forward = [&](bool first, int it0, int n, const long long *off) {
-            return run2d_group_run(grp, 1, it0, n, first, first, 1, off, c->stream);
+        const SweepOps one = op;
+        q.run = [&](const std::vector<Run2dOp> &ops, const std::vector<long long> &offs) {
+            return run2d_group_run(grp, ops, offs, o->image_every, c->stream);
         };
-        q.run_receive = [&](int it0, int n, const long long *off) {
-            return run2d_group_run(grp, 2, it0, n, false, false, o->image_every, off, c->stream);
-        };
-        const auto step1 = op.step, first1 = op.first_step;
-        q.step = [&, step1, first1](bool first, int it) { return first ? first1(it) : step1(it); };
-        q.keep = [&](long long off) {
+        q.step = [&, one](bool first, int it) { return first ? one.first_step(it) : one.step(it); };
+        q.keep = [&, at](long long off) {
             return hip(hipMemcpyAsync(at(off).f[VTI_F_P], P, c->nvol * sizeof(float), hipMemcpyDeviceToDevice, c->stream),
                        "store");
         };
-        q.receive = [&](int it, long long off) { return consume_from(at(off), it + 1); };
-        // every other operation finds the states as if each step had been
-        // taken when it was asked for
-        auto flushed = [&q](std::function<int()> f) {
-            return [&q, f]() { const int e = q.flush(); return e ? e : f(); };
+        q.receive = [&, at](int it, long long off) { return consume_from(at(off), it + 1); };
+        q.move = [&, one, slot_of](int kind, long long slot) {
+            return kind == 5 ? one.zero() : (kind == 3 ? one.store(slot_of(slot)) : one.restore(slot_of(slot)));
         };
-        auto flushed1 = [&q](std::function<int(int)> f) {
-            return [&q, f](int i) { const int e = q.flush(); return e ? e : f(i); };
-        };
-        op.zero = flushed(op.zero);
-        op.after_first = flushed(op.after_first);
-        op.store = flushed1(op.store);
-        op.restore = flushed1(op.restore);
-        op.store_light = [&, slot_off](int i) { return q.keep_last(slot_off(i)); };
+        op.zero = [&]() { return q.state(5, 0); };
+        op.after_first = [&, one]() { const int e = q.flush(); return e ? e : one.after_first(); };
+        op.store = [&, slot_s](int i) { return q.state(3, slot_s(i)); };
+        op.restore = [&, slot_s](int i) { return q.state(4, slot_s(i)); };
+        op.store_light = [&, slot_p](int i) { return q.keep_last(slot_p(i)); };
         op.step = [&](int it) { return q.forward(false, it); };
         op.first_step = [&](int it) { return q.forward(true, it); };
         op.consume = [&](int k) { return q.receiver(k - 1, 0); };
-        op.consume_slot = [&, slot_off](int k, int i) { return q.receiver(k - 1, slot_off(i)); };
+        op.consume_slot = [&, slot_p](int k, int i) { return q.receiver(k - 1, slot_p(i)); };
         if (c->unsplit) c->us_dirty = true;
     }
     if ((st = reverse_sweep(nt, nslot, op, fwd_steps))) return st;

@@ -54,17 +54,18 @@ __device__ __forceinline__ float cst(int m)
 constexpr unsigned long long kWaitTicks = 2000000000ull;
 
 struct Run2dArgs {
-    Run2dShot one;              // role 0: the shot
-    const Run2dShot *many;      // roles 1, 2: ns shots in device memory, tile0 ascending
+    Run2dShot one;              // vti_step: the shot
+    int it0, n;                 // its first time index and number of steps
+    // RTM program: ns shots in device memory (tile0 ascending), the same
+    // operations on each
+    const Run2dShot *many;
     int ns;
-    int it0, n;                 // first time index, steps (role 2: descending indices)
-    unsigned base;              // tag of the call's first step
+    const Run2dOp *ops;
+    int nops;
+    const long long *offs;
+    int image_every;
+    unsigned base;              // tag before the call's first exchange
     int *dead;                  // host-visible error word
-    int rec, illum;             // role 1: keep the record, accumulate the source illumination
-    int image_every;            // role 2
-    // role 1: where step k's P also goes, as floats from the shot's own P
-    // (0: nowhere); role 2: where step k's source P lies, from srcP
-    long long off[kRun2dMax];
 };
 
 // an opaque copy: what is derived from it inside the step loop is not hoisted
@@ -74,6 +75,14 @@ __device__ __forceinline__ int opaque(int v)
     asm volatile("" : "+v"(v));
     return v;
 }
+
+// What a launch reads and nothing in it writes (the arguments, the shots, a
+// program): scalar loads, again where they are used, instead of registers
+// held through the step loop.
+using CArgs = const __attribute__((address_space(4))) Run2dArgs;
+using CShot = const __attribute__((address_space(4))) Run2dShot;
+using COp = const __attribute__((address_space(4))) Run2dOp;
+using COff = const __attribute__((address_space(4))) long long;
 
 struct Tile {
     int x0, nx, z0, nz;         // first cell, rows; first z, cells (a multiple of 4)
@@ -153,7 +162,7 @@ __device__ __forceinline__ float await(const unsigned long long *p, unsigned lon
 }
 
 // the shot of a tile (tile0 ascending)
-__device__ __forceinline__ int find_shot2d(const Run2dShot *s, int ns, int tile)
+__device__ __forceinline__ int find_shot2d(CShot *s, int ns, int tile)
 {
     int lo = 0, hi = ns - 1;
     while (lo < hi) {
@@ -197,21 +206,29 @@ __device__ __forceinline__ float diff_z(const float *p)
 // fields of a damped one).  One cell a lane and 16 wavefronts a CU: four cells
 // a lane (16-byte LDS accesses, 8 wavefronts) took 3.8 against 3.6 us a step
 // at 400 x 400 and 14.9 against 14.1 at 2401 x 803.
-// ROLE 0: vti_step (source and record of one shot); 1: the source side of an
-// RTM, of many shots at once: record and illumination (first sweep), P into
-// checkpoints; 2: its receiver side, backward in time: the records written
-// into P and Q on the injection row before each step (only the velocity
-// update reads them: the split form of that row rebuilds P and Q), the image
-// img += P_source * P and, where asked for, the receiver illumination.
-template <bool TTI, bool US, int ROLE, int NT, int NU>
+// PROG false: vti_step (source and record of one shot).  PROG true: the
+// schedule of an RTM as a program (Run2dOp), of many shots at once: forward
+// steps (record and illumination in the first sweep, P into checkpoints),
+// receiver steps backward in time (the records written into P and Q on the
+// injection row before each step: only the velocity update reads them, the
+// split form of that row rebuilds P and Q; image img += P_source * P and,
+// where asked for, the receiver illumination), whole-state checkpoints.  The
+// state that steps is on the chip, the other side's and the checkpoints are
+// in memory; all of those are a tile's own cells, written and read by the
+// same thread, so tiles meet only in the exchange.
+template <bool TTI, bool US, bool PROG, int NT, int NU>
 __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
 {
     extern __shared__ float4 smem4[];
     float *sm = reinterpret_cast<float *>(smem4);
     __shared__ int s_dead;
     const int tid = threadIdx.x;
-    const Run2dShot &b = ROLE ? a.many[find_shot2d(a.many, a.ns, blockIdx.x)] : a.one;
-    const int tile = blockIdx.x - (ROLE ? b.tile0 : 0);
+    CArgs *ka = (CArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    CShot *many = (CShot *)a.many;
+    CShot &b = PROG ? many[find_shot2d(many, a.ns, blockIdx.x)] : ka->one;
+    COp *ops = (COp *)a.ops;
+    COff *offs = (COff *)a.offs;
+    const int tile = blockIdx.x - (PROG ? b.tile0 : 0);
     const Tile t = tile_of(b.nnx, b.nnz, b.gx, b.gz, tile / b.gz, tile % b.gz);
     const int nx = t.nx, nz = t.nz, x0 = t.x0, z0 = t.z0;
     const Lds<TTI> L(nx, nz);
@@ -280,41 +297,20 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         if (!live || i >= rows) continue;
         const int x = x0 + r0 + i, z = z0 + c;
         const long long g = (long long)x * ldz + z;
-        const float v = b.vp[g];
-        float ee = b.ep[g], dd = b.de[g];
-        s0[i] = b.f[2][g];
-        s1[i] = b.f[4][g];
-        s2[i] = b.f[3][g];
-        s3[i] = b.f[5][g];
-        const float tx1 = ax1[r0 + i], tx2 = ax2[r0 + i], tz1 = az1[c], tz2 = az2[c];
-        if (b.sv) {   // SV taper (GPU_vti2dfd_kernels.cu:260-278)
-            const int rx = x - b.cx, rz = z - b.cz, r2 = rx * rx + rz * rz;
-            if (r2 <= b.svR * b.svR) {
-                const double f = b.tap[r2];
-                ee = (float)(f * (double)ee);
-                dd = (float)(f * (double)dd);
+        if (!PROG) {
+            s0[i] = b.f[2][g];
+            s1[i] = b.f[4][g];
+            s2[i] = b.f[3][g];
+            s3[i] = b.f[5][g];
+        }
+        if (US && ax1[r0 + i] == 1.0f && ax2[r0 + i] == 1.0f && az1[c] == 1.0f && az2[c] == 1.0f) {
+            und |= 1 << i;
+            if (!PROG) {
+                s0[i] = sP[(r0 + i) * L.pp + c];
+                s1[i] = sQ[(r0 + i) * L.qp + c];
             }
         }
-        const float e2 = 1.0f + 2.0f * ee;
-        const float sd = sqrtf(1.0f + 2.0f * dd);
-        if (TTI) {   // the cos/sin terms carry dt/dx: g1 vp vp (1+2e), g1 vp vp sqrt(1+2d), g1 vp vp
-            const float g1 = tx1 * tz1;
-            c0[i] = g1 * v * v * e2;
-            c1[i] = g1 * v * v * sd;
-            c2[i] = g1 * v * v;
-            c3[i] = tx2 * tz2;
-        } else {
-            c0[i] = tx1 * v * v * e2 * b.dtx;
-            c1[i] = tx1 * v * v * sd * b.dtx;
-            c2[i] = tz1 * v * v * sd * b.dtz;
-            c3[i] = tz1 * v * v * b.dtz;
-        }
-        if (US && z != b.split_z && tx1 == 1.0f && tx2 == 1.0f && tz1 == 1.0f && tz2 == 1.0f) {
-            und |= 1 << i;
-            s0[i] = sP[(r0 + i) * L.pp + c];
-            s1[i] = sQ[(r0 + i) * L.qp + c];
-        }
-        if (ROLE != 2 && b.rec && (!ROLE || a.rec) && z == b.rz) {
+        if (b.rec && z == b.rz) {
             const int k = x - b.rx0;
             if (k >= 0 && k % b.rdx == 0 && k / b.rdx < b.rnx) {
                 if (!recs) krec = k / b.rdx;
@@ -322,44 +318,71 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
             }
         }
     }
+    // the strip's coefficients, with the SV taper or without
+    auto coefficients = [&](bool sv) {
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+            if (!live || i >= rows) continue;
+            const int x = x0 + row0 + i, z = z0 + col0;
+            const long long g = (long long)x * ldz + z;
+            const float v = b.vp[g];
+            float ee = b.ep[g], dd = b.de[g];
+            const float tx1 = ax1[row0 + i], tx2 = ax2[row0 + i], tz1 = az1[col0], tz2 = az2[col0];
+            if (sv) {   // SV taper (GPU_vti2dfd_kernels.cu:260-278)
+                const int rx = x - b.cx, rz = z - b.cz, r2 = rx * rx + rz * rz;
+                if (r2 <= b.svR * b.svR) {
+                    const double f = b.tap[r2];
+                    ee = (float)(f * (double)ee);
+                    dd = (float)(f * (double)dd);
+                }
+            }
+            const float e2 = 1.0f + 2.0f * ee;
+            const float sd = sqrtf(1.0f + 2.0f * dd);
+            if (TTI) {   // the cos/sin terms carry dt/dx: g1 vp vp (1+2e), g1 vp vp sqrt(1+2d), g1 vp vp
+                const float g1 = tx1 * tz1;
+                c0[i] = g1 * v * v * e2;
+                c1[i] = g1 * v * v * sd;
+                c2[i] = g1 * v * v;
+                c3[i] = tx2 * tz2;
+            } else {
+                c0[i] = tx1 * v * v * e2 * b.dtx;
+                c1[i] = tx1 * v * v * sd * b.dtx;
+                c2[i] = tz1 * v * v * sd * b.dtz;
+                c3[i] = tz1 * v * v * b.dtz;
+            }
+        }
+    };
+    if (!PROG) coefficients(b.sv != 0);
 
     // images: interior cell (r0 + i, c) at img[io + i * inz]
-    const bool inz_ok = ROLE && live && z0 + c >= b.inp && z0 + c < b.inp + b.inz;
+    const bool inz_ok = PROG && live && z0 + c >= b.inp && z0 + c < b.inp + b.inz;
     const long long io = (long long)(x0 + row0 - b.inp) * b.inz + (z0 + col0 - b.inp);
-    const bool lit = ROLE == 1 ? a.illum != 0 : (ROLE == 2 && b.rillum);
     int inn = 0;                               // rows of the strip in the interior
-    float il[ROLE ? NU : 1], im[ROLE == 2 ? NU : 1];
-    if (ROLE) {
+    float il[PROG ? NU : 1], im[PROG ? NU : 1];
+    if (PROG) {
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
             const int jx = x0 + row0 + i - b.inp;
-            il[i] = 0.0f;
-            if (ROLE == 2) im[i] = 0.0f;
+            il[i] = im[i] = 0.0f;
             if (!inz_ok || i >= rows || jx < 0 || jx >= b.inx) continue;
             inn |= 1 << i;
-            if (lit) il[i] = b.illum[io + (long long)i * b.inz];
-            if (ROLE == 2) im[i] = b.img[io + (long long)i * b.inz];
+            il[i] = b.illum[io + (long long)i * b.inz];
+            im[i] = b.img[io + (long long)i * b.inz];
         }
 #pragma unroll
-        for (int i = 0; i < NU; ++i) {
-            asm volatile("" : "+v"(il[i]));
-            if (ROLE == 2) asm volatile("" : "+v"(im[i]));
-        }
+        for (int i = 0; i < NU; ++i) asm volatile("" : "+v"(il[i]), "+v"(im[i]));
     }
-    const bool clamp = ROLE == 1 && b.clamp;
     // receiver samples of this lane's row of the injection row (tile and halo)
-    const int zi = ROLE == 2 ? b.rzi - z0 : 0;
-    const bool inj_p = ROLE == 2 && zi >= 0 && zi < nz, inj_q = ROLE == 2 && zi >= -8 && zi < nz + 8;
+    const int zi = PROG ? b.rzi - z0 : 0;
+    const bool inj_p = PROG && zi >= 0 && zi < nz, inj_q = PROG && zi >= -8 && zi < nz + 8;
     int kinj = -1;
     if (inj_q && tid < nx + 14) {
         const int k = x0 + tid - 7 - b.rx0;
         if (k >= 0 && k % b.rdx == 0 && k / b.rdx < b.rnx) kinj = k / b.rdx;
     }
-    const float *srcP = b.srcP;
-    float *ownP = b.f[6];
     const int srow = b.sx - x0, scol = b.sz - z0;
-    const bool src_p = ROLE != 2 && b.point && srow >= -7 && srow < nx + 7 && scol >= (TTI ? -8 : 0) && scol < nz + (TTI ? 8 : 0);
-    const bool src_q = ROLE != 2 && b.point && srow >= (TTI ? -7 : 0) && srow < nx + (TTI ? 7 : 0) && scol >= -8 && scol < nz + 8;
+    const bool src_p = b.point && srow >= -7 && srow < nx + 7 && scol >= (TTI ? -8 : 0) && scol < nz + (TTI ? 8 : 0);
+    const bool src_q = b.point && srow >= (TTI ? -7 : 0) && srow < nx + (TTI ? 7 : 0) && scol >= -8 && scol < nz + 8;
 
     // the strip is in registers before the step loop, whose waits would
     // otherwise count these loads as possibly still on their way
@@ -368,29 +391,176 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         asm volatile("" : "+v"(s0[i]), "+v"(s1[i]), "+v"(s2[i]), "+v"(s3[i]), "+v"(c0[i]), "+v"(c1[i]), "+v"(c2[i]), "+v"(c3[i]));
     if (US) __syncthreads();   // P and Q are in s0 and s1 before the source is added to them in LDS
     float amps = 0.0f;   // lane k: the gain of step k of the current 64
-    for (int s = 0; s < a.n; ++s) {
-        const int it = ROLE == 2 ? a.it0 - s : a.it0 + s;
-        if (ROLE != 2 && (s & 63) == 0) {
-            amps = b.amp[a.it0 + min(s + (tid & 63), a.n - 1)];
+    unsigned tag = a.base;
+    int cur = PROG ? 0 : 1;   // whose state is on the chip: 1 source, 2 receiver
+    bool fresh = false;       // PROG: the halos are not those of the state on the chip
+    const int nops = PROG ? a.nops : 1;
+    for (int o = 0; o < nops; ++o) {
+    Run2dOp op{};
+    if (PROG) {
+        op.kind = ops[o].kind;
+        op.it0 = ops[o].it0;
+        op.n = ops[o].n;
+        op.first = ops[o].first;
+        op.link = ops[o].link;
+        op.off0 = ops[o].off0;
+        op.slot = ops[o].slot;
+    } else {
+        op.kind = 1;
+        op.first = 1;
+        op.it0 = a.it0;
+        op.n = a.n;
+    }
+    const bool rcv = PROG && op.kind == 2;
+    if (PROG) {
+        const int role = rcv ? 2 : 1;
+        const bool sw = cur != role;
+        // cell (row0 + i, col0) of a packed checkpoint's split fields
+        auto packed = [&](int i) {
+            const int x = x0 + row0 + i, z = z0 + col0;
+            const bool whole = x < b.pxlo || x >= b.pxhi;
+            const long long full = (long long)min(x, b.pxlo) + max(0, x - b.pxhi);
+            return full * b.nnz + (x - full) * (long long)(b.pzlo + b.nnz - b.pzhi) +
+                   (whole || z < b.pzlo ? z : b.pzlo + (z - b.pzhi));
+        };
+        if ((sw && cur) || op.kind == 3) {   // the state on the chip to its home, or to a checkpoint
+            const bool pk = op.kind == 3 && b.packed;
+            const long long off = op.kind == 3 ? op.slot : 0;
+            float *F[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) F[k] = (cur == 2 ? b.g[k] : b.f[k]) + off;
+            if (pk) {
+                F[0] = b.f[0] + off;
+                F[1] = F[0] + b.pvol; F[6] = F[1] + b.pvol; F[7] = F[6] + b.pvol;
+                F[2] = F[7] + b.pvol; F[3] = F[2] + b.psplit; F[4] = F[3] + b.psplit; F[5] = F[4] + b.psplit;
+            }
+            const int ub = cur == 2 && z0 + col0 == b.split_z ? 0 : und;
+#pragma unroll
+            for (int i = 0; i < NU; ++i) {
+                asm volatile("" ::: "memory");
+                if (!live || i >= rows) continue;
+                const int r = row0 + i, c = col0;
+                const long long g = (long long)(x0 + r) * ldz + z0 + c;
+                F[0][g] = sU[r * L.up + c];
+                F[1][g] = sW[r * L.wp + c];
+                F[6][g] = sP[r * L.pp + c];
+                F[7][g] = sQ[r * L.qp + c];
+                if (US && (ub >> i & 1)) continue;
+                const long long h = pk ? packed(i) : g;
+                F[2][h] = s0[i];
+                F[4][h] = s1[i];
+                F[3][h] = s2[i];
+                F[5][h] = s3[i];
+            }
+        }
+        if (sw || op.kind >= 4) {            // another state onto the chip: a home, a checkpoint, zero
+            const bool pk = op.kind == 4 && b.packed;
+            const long long off = op.kind == 4 ? op.slot : 0;
+            const float *F[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) F[k] = (rcv ? b.g[k] : b.f[k]) + off;
+            if (pk) {
+                F[0] = b.f[0] + off;
+                F[1] = F[0] + b.pvol; F[6] = F[1] + b.pvol; F[7] = F[6] + b.pvol;
+                F[2] = F[7] + b.pvol; F[3] = F[2] + b.psplit; F[4] = F[3] + b.psplit; F[5] = F[4] + b.psplit;
+            }
+            const bool zero = op.kind == 5;
+            const int ub = rcv && z0 + col0 == b.split_z ? 0 : und;
+#pragma unroll
+            for (int i = 0; i < NU; ++i) {
+                asm volatile("" ::: "memory");
+                if (!live || i >= rows) continue;
+                const int r = row0 + i, c = col0;
+                const long long g = (long long)(x0 + r) * ldz + z0 + c;
+                const float P = zero ? 0.0f : F[6][g], Q = zero ? 0.0f : F[7][g];
+                sU[r * L.up + c] = zero ? 0.0f : F[0][g];
+                sW[r * L.wp + c] = zero ? 0.0f : F[1][g];
+                sP[r * L.pp + c] = P;
+                sQ[r * L.qp + c] = Q;
+                if (US && (ub >> i & 1)) {
+                    s0[i] = P;
+                    s1[i] = Q;
+                    continue;
+                }
+                const long long h = pk ? packed(i) : g;
+                s0[i] = zero ? 0.0f : F[2][h];
+                s1[i] = zero ? 0.0f : F[4][h];
+                s2[i] = zero ? 0.0f : F[3][h];
+                s3[i] = zero ? 0.0f : F[5][h];
+            }
+            if (sw) coefficients(rcv ? b.svr != 0 : b.sv != 0);
+#pragma unroll
+            for (int i = 0; i < NU; ++i)
+                asm volatile("" : "+v"(s0[i]), "+v"(s1[i]), "+v"(s2[i]), "+v"(s3[i]), "+v"(c0[i]), "+v"(c1[i]), "+v"(c2[i]), "+v"(c3[i]));
+            cur = role;
+            fresh = true;
+            __syncthreads();
+        }
+        if (op.kind >= 3) continue;
+    }
+    const bool lit = PROG && (rcv ? b.rillum != 0 : op.first != 0), clamp = PROG && !rcv && b.clamp;
+    for (int s = 0; s < op.n; ++s) {
+        const int it = rcv ? op.it0 - s : op.it0 + s;
+        if (!rcv && (s & 63) == 0) {
+            amps = b.amp[op.it0 + min(s + (tid & 63), op.n - 1)];
             // taken here: waited for at the top of each step, the load would
             // hold the step until the stores before it are acknowledged too
             asm volatile("" : "+v"(amps));
         }
-        const float amp = ROLE == 2 ? 0.0f : __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(amps), s & 63));
+        const float amp = rcv ? 0.0f : __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(amps), s & 63));
         const int vt = opaque(tid), r0 = opaque(row0), c = opaque(col0);
         // what this step reads from memory: its latency passes behind the exchange
-        float inj = 0.0f, sp[ROLE == 2 ? NU : 1];
-        const bool imaged = ROLE == 2 && it % a.image_every == 0;
-        if (ROLE == 2) {
+        float inj = 0.0f, sp[PROG ? NU : 1];
+        const bool imaged = rcv && it % a.image_every == 0;
+        if (rcv) {
             if (kinj >= 0) inj = b.rec[(long long)it * b.nrec + kinj];
-            const float *src = srcP + a.off[s] + (long long)(x0 + r0) * ldz + z0 + c;
+            const float *src = b.f[6] + offs[op.off0 + s] + (long long)(x0 + r0) * ldz + z0 + c;
 #pragma unroll
             for (int i = 0; i < NU; ++i) sp[i] = imaged && (inn >> i & 1) ? src[(long long)i * ldz] : 0.0f;
         }
-        if (s > 0) {
+        if (PROG && fresh) {
+            // ---- a state just put on the chip: its outer rows and columns of
+            // all four fields to the neighbours, theirs taken ----
+            ++tag;
+            const long long par = (tag & 1) * b.xstride;
+            unsigned long long *gP = b.xP + par, *gQ = b.xQ + par, *gU = b.xU + par, *gW = b.xW + par;
+            if (live) {
+#pragma unroll
+                for (int i = 0; i < NU; ++i) {
+                    if (i >= rows) continue;
+                    const int r = r0 + i;
+                    const long long g = (long long)(x0 + r) * ldz + z0 + c;
+                    if (r < 7 || r >= nx - 7) put(gP + g, sP[r * L.pp + c], tag);
+                    if (c < 7 || c >= nz - 7) put(gQ + g, sQ[r * L.qp + c], tag);
+                    if (r < 4 || r >= nx - 4) put(gU + g, sU[r * L.up + c], tag);
+                    if (c < 4 || c >= nz - 4) put(gW + g, sW[r * L.wp + c], tag);
+                }
+            }
+            for (int k = vt; k < 21 * nz + 21 * nx; k += NT) {
+                const bool q = k >= 21 * nz;
+                int r, cc;
+                if (!q) divmod(k, nz, inv_z, r, cc);
+                else divmod(k - 21 * nz, 21, 1.0f / 21.0f, r, cc);
+                int &w = q ? cc : r;            // 0-13: P (Q), 14-20: u (w)
+                const int n = q ? nz : nx;
+                const bool vel = w >= 14;
+                w = vel ? (w < 18 ? w - 18 : n + w - 18) : (w < 7 ? w - 7 : n + w - 7);
+                const int x = x0 + r, z = z0 + cc;
+                if (x < 4 || x >= xend || z < 4 || z >= zend) continue;
+                const unsigned long long *p = (q ? (vel ? gW : gQ) : (vel ? gU : gP)) + (long long)x * ldz + z;
+                float *d = q ? (vel ? sW + r * L.wp + cc : sQ + r * L.qp + cc) : (vel ? sU + r * L.up + cc : sP + r * L.pp + cc);
+                *d = await(p, peek(p), tag, &s_dead);
+            }
+            fresh = false;
+            __syncthreads();
+            if (s_dead) {
+                if (tid == 0) *a.dead = 1;
+                return;
+            }
+        } else if (PROG || s > 0) {
             // ---- the neighbours' outer rows and columns of the last step ----
-            const unsigned tag = a.base + s;
-            const unsigned long long *gP = b.xP + (s & 1) * b.xstride, *gQ = b.xQ + (s & 1) * b.xstride;
+            ++tag;
+            const unsigned long long *gP = b.xP + (tag & 1) * b.xstride, *gQ = b.xQ + (tag & 1) * b.xstride;
             const int nrow = 14 * nz;
             const int wide = 14 * (nz + 14), nget = (TTI ? wide : nrow) + 14 * nx;
             const int total = TTI ? 2 * nget : nget;
@@ -430,7 +600,7 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 return;
             }
         }
-        if (ROLE == 2 && inj_q) {   // shot_record(load) Toa_gpu2DvtiFdRtmAdcigsLaplace.cu:525-528
+        if (rcv && inj_q) {   // shot_record(load) Toa_gpu2DvtiFdRtmAdcigsLaplace.cu:525-528
             if (kinj >= 0) {
                 const int r = tid - 7;
                 if (inj_p) sP[r * L.pp + zi] = inj;
@@ -438,7 +608,7 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
             }
             __syncthreads();
         }
-        if (ROLE != 2 && amp != 0.0f && (src_p || src_q)) {   // P[src] += amp, Q[src] += amp before the update (add_source2d :204-205)
+        if (amp != 0.0f && (src_p || src_q)) {   // P[src] += amp, Q[src] += amp before the update (add_source2d :204-205)
             if (tid == 0) {
                 if (src_p) sP[srow * L.pp + scol] += amp;
                 if (src_q) sQ[srow * L.qp + scol] += amp;
@@ -512,11 +682,16 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
 
         // ---- stress update of the tile ----
         if (live) {
-            const int nr = opaque(rows), ub = opaque(und), rb = opaque(recs), in_ = ROLE ? opaque(inn) : 0;
-            float *keep = ROLE == 1 && a.off[s] ? ownP + a.off[s] : nullptr;
-            const bool foot = ROLE == 0 && !b.point && amp != 0.0f, more = s + 1 < a.n;
-            unsigned long long *gP = b.xP + ((s + 1) & 1) * b.xstride, *gQ = b.xQ + ((s + 1) & 1) * b.xstride;
-            const unsigned tag = a.base + s + 1;
+            const int nr = opaque(rows), rb = opaque(recs), in_ = PROG ? opaque(inn) : 0;
+            const int ub = opaque(rcv && z0 + c == b.split_z ? 0 : und);
+            float *keep = nullptr;
+            if (PROG && !rcv) {
+                const long long off = offs[op.off0 + s];
+                if (off) keep = b.f[6] + off;
+            }
+            const bool foot = !PROG && !b.point && amp != 0.0f, more = s + 1 < op.n || op.link, note = !rcv && op.first;
+            const unsigned next = tag + 1;
+            unsigned long long *gP = b.xP + (next & 1) * b.xstride, *gQ = b.xQ + (next & 1) * b.xstride;
             const bool ez = c < 7 || c >= nz - 7;
             const float *pu = sU + r0 * L.up + c, *pw = sW + r0 * L.wp + c;
             float f[NU + 7], h[TTI ? NU + 7 : 1];
@@ -564,18 +739,18 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 if (more) {   // the outer 7 rows and columns, to the neighbours
                     const bool ex = r < 7 || r >= nx - 7;
                     const long long g = (long long)(x0 + r) * ldz + z0 + c;
-                    if (ex || (TTI && ez)) put(gP + g, Pn, tag);
-                    if (ez || (TTI && ex)) put(gQ + g, Qn, tag);
+                    if (ex || (TTI && ez)) put(gP + g, Pn, next);
+                    if (ez || (TTI && ex)) put(gQ + g, Qn, next);
                 }
-                if (ROLE && (in_ >> i & 1)) {
+                if (PROG && (in_ >> i & 1)) {
                     if (lit) {   // cal_illumination :654-677
                         il[i] += Pn * Pn + Qn * Qn;
                         if (clamp && il[i] <= 0.0f) il[i] = 1.0f;
                     }
-                    if (ROLE == 2 && imaged) im[i] += sp[i] * Pn;   // cal_migration :679-698
+                    if (imaged) im[i] += sp[i] * Pn;   // cal_migration :679-698
                 }
-                if (ROLE == 1 && keep) keep[(long long)(x0 + r) * ldz + z0 + c] = Pn;
-                if (ROLE != 2 && (rb >> i & 1)) {
+                if (PROG && keep) keep[(long long)(x0 + r) * ldz + z0 + c] = Pn;
+                if (note && (rb >> i & 1)) {
                     const int k = krec + __popc(rb & ((1 << i) - 1));
                     b.rec[(long long)it * b.nrec + k] = b.rec_kind == 0 ? Pn : (b.rec_kind == 1 ? Pn + Pn : Pn + Qn);
                 }
@@ -583,18 +758,18 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         }
         __syncthreads();
     }
+    }   // operations
 
-    // ---- write the tile back (n >= 2: every neighbour has loaded its halo) ----
+    // ---- write the tile back (n >= 2: every neighbour has loaded its halo;
+    // PROG: none reads another's cells in memory) ----
     // the field pointers come from memory again: held through the loop they
     // would cost the registers that it needs
-    using KArgs = const __attribute__((address_space(4))) Run2dArgs;
-    KArgs *ka = (KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(ka));
-    const Run2dShot *bm = ROLE ? &b : nullptr;
+    CShot *bm = &b;
     asm volatile("" : "+s"(bm));
     float *gf[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) gf[k] = ROLE ? bm->f[k] : ka->one.f[k];
+    for (int k = 0; k < 8; ++k) gf[k] = cur == 2 ? bm->g[k] : bm->f[k];
+    const int ub = cur == 2 && z0 + c == b.split_z ? 0 : und;
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
@@ -605,11 +780,11 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
         gf[1][g] = sW[r * L.wp + c];
         gf[6][g] = sP[r * L.pp + c];
         gf[7][g] = sQ[r * L.qp + c];
-        if (ROLE && (inn >> i & 1)) {
-            if (lit) b.illum[io + (long long)i * b.inz] = il[i];
-            if (ROLE == 2) b.img[io + (long long)i * b.inz] = im[i];
+        if (PROG && (inn >> i & 1)) {
+            b.illum[io + (long long)i * b.inz] = il[i];
+            b.img[io + (long long)i * b.inz] = im[i];
         }
-        if (US && (und >> i & 1)) continue;   // no split fields there
+        if (US && (ub >> i & 1)) continue;   // no split fields there
         gf[2][g] = s0[i];
         gf[4][g] = s1[i];
         gf[3][g] = s2[i];
@@ -625,19 +800,19 @@ struct Shape2d {
 };
 constexpr Shape2d kShapes[] = {{512, 1}, {1024, 1}, {1024, 2}, {1024, 3}, {1024, 4}, {1024, 6}, {1024, 8}};
 constexpr int kNumShapes = (int)(sizeof(kShapes) / sizeof(kShapes[0]));
-constexpr int kRtmShapes = kNumShapes - 1;   // the RTM roles' images leave no registers for strips of 8
+constexpr int kRtmShapes = kNumShapes - 1;   // the RTM program's images leave no registers for strips of 8
 
-template <bool TTI, bool US, int ROLE>
+template <bool TTI, bool US, bool PROG>
 KernelFn kernel_of(int shape)
 {
     switch (shape) {
-    case 0: return run2d_kernel<TTI, US, ROLE, 512, 1>;
-    case 1: return run2d_kernel<TTI, US, ROLE, 1024, 1>;
-    case 2: return run2d_kernel<TTI, US, ROLE, 1024, 2>;
-    case 3: return run2d_kernel<TTI, US, ROLE, 1024, 3>;
-    case 4: return run2d_kernel<TTI, US, ROLE, 1024, 4>;
-    case 5: return run2d_kernel<TTI, US, ROLE, 1024, 6>;
-    default: return run2d_kernel<TTI, US, ROLE, 1024, ROLE ? 6 : 8>;
+    case 0: return run2d_kernel<TTI, US, PROG, 512, 1>;
+    case 1: return run2d_kernel<TTI, US, PROG, 1024, 1>;
+    case 2: return run2d_kernel<TTI, US, PROG, 1024, 2>;
+    case 3: return run2d_kernel<TTI, US, PROG, 1024, 3>;
+    case 4: return run2d_kernel<TTI, US, PROG, 1024, 4>;
+    case 5: return run2d_kernel<TTI, US, PROG, 1024, 6>;
+    default: return run2d_kernel<TTI, US, PROG, 1024, PROG ? 6 : 8>;
     }
 }
 
@@ -746,10 +921,10 @@ bool plan_group(std::vector<Run2dShot> &shots, bool tti, int nshape, const Devic
 size_t plane_of(const Run2dShot &s) { return (size_t)s.ldz * s.nnx; }
 
 // the exchange planes of every shot, zeroed, and the error word
-bool alloc_group(std::vector<Run2dShot> &shots, unsigned long long *&xbuf, int *&dead, hipStream_t s)
+bool alloc_group(std::vector<Run2dShot> &shots, int nfield, unsigned long long *&xbuf, int *&dead, hipStream_t s)
 {
     size_t n = 0;
-    for (const Run2dShot &b : shots) n += 4 * plane_of(b);
+    for (const Run2dShot &b : shots) n += 2 * nfield * plane_of(b);
     if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess ||
         hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess ||
         launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) != hipSuccess) {
@@ -762,7 +937,9 @@ bool alloc_group(std::vector<Run2dShot> &shots, unsigned long long *&xbuf, int *
         b.xstride = (long long)plane_of(b);
         b.xP = p;
         b.xQ = p + 2 * plane_of(b);
-        p += 4 * plane_of(b);
+        b.xU = nfield > 2 ? p + 4 * plane_of(b) : nullptr;
+        b.xW = nfield > 2 ? p + 6 * plane_of(b) : nullptr;
+        p += 2 * nfield * plane_of(b);
     }
     return true;
 }
@@ -858,7 +1035,7 @@ int run2d_steps(vti_ctx *c, int it0, int n)
         Device2d d;
         p.shot.push_back(run2d_shot(c, main_state(c)));
         if (!device_2d(c->device, d) || !plan_group(p.shot, tti, kNumShapes, d, p.shape, p.lds, p.ntile) ||
-            !alloc_group(p.shot, p.xbuf, p.dead, c->stream))
+            !alloc_group(p.shot, 2, p.xbuf, p.dead, c->stream))
             return 0;
         p.ok = 1;
     }
@@ -874,8 +1051,8 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     a.base = p.base;
     a.dead = p.dead;
     const bool us = c->unsplit && c->cfg.mode == VTI_MODE_GPU_REF && !tti;
-    const KernelFn k = tti ? kernel_of<true, false, 0>(p.shape)
-                           : (us ? kernel_of<false, true, 0>(p.shape) : kernel_of<false, false, 0>(p.shape));
+    const KernelFn k = tti ? kernel_of<true, false, false>(p.shape)
+                           : (us ? kernel_of<false, true, false>(p.shape) : kernel_of<false, false, false>(p.shape));
     if (!launch_coop(k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream)) {
         p.ok = -1;
         return 0;
@@ -912,31 +1089,21 @@ int run2d_fit(const std::vector<Run2dShot> &shots, int first, int device)
     return n;
 }
 
-int run2d_group_make(Run2dGroup &g, const std::vector<Run2dShot> &src, const std::vector<Run2dShot> &rcv, bool us,
-                     int device, hipStream_t s)
+int run2d_group_make(Run2dGroup &g, const std::vector<Run2dShot> &shots, bool us, int device, hipStream_t s)
 {
     g.ok = 0;
-    if (src.empty() || capturing(s)) return 0;
+    if (shots.empty() || capturing(s)) return 0;
     Device2d d;
-    g.side[0] = src;
-    g.side[1] = rcv;
-    g.ns = (int)src.size();
+    g.shots = shots;
     g.us = us;
-    if (!device_2d(device, d) || !plan_group(g.side[0], false, kRtmShapes, d, g.shape, g.lds, g.ntile) ||
-        !alloc_group(g.side[0], g.xbuf, g.dead, s))
+    if (!device_2d(device, d) || !plan_group(g.shots, false, kRtmShapes, d, g.shape, g.lds, g.ntile) ||
+        !alloc_group(g.shots, 4, g.xbuf, g.dead, s))
         return 0;
-    for (int k = 0; k < g.ns; ++k) {
-        const Run2dShot &a = g.side[0][k];
-        Run2dShot &b = g.side[1][k];
-        b.gx = a.gx; b.gz = a.gz; b.tile0 = a.tile0;
-        b.xP = a.xP; b.xQ = a.xQ; b.xstride = a.xstride;
-    }
-    if (hipMalloc(&g.dev, 2 * g.ns * sizeof(Run2dShot)) != hipSuccess) {
+    if (hipMalloc(&g.dev, g.shots.size() * sizeof(Run2dShot)) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
     }
-    if (hipMemcpy(g.dev, g.side[0].data(), g.ns * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(g.dev + g.ns, g.side[1].data(), g.ns * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess)
+    if (hipMemcpy(g.dev, g.shots.data(), g.shots.size() * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess)
         return fail(VTI_ERR_HIP, "run2d: descriptors");
     g.ok = 1;
     return 1;
@@ -946,88 +1113,113 @@ void run2d_group_free(Run2dGroup &g)
 {
     (void)hipFree(g.dev);
     (void)hipFree(g.xbuf);
+    (void)hipFree(g.prog);
     (void)hipHostFree(g.dead);
-    g.dev = nullptr;
-    g.xbuf = nullptr;
-    g.dead = nullptr;
-    g.ok = 0;
+    g = Run2dGroup{};
 }
 
-int run2d_group_run(Run2dGroup &g, int role, int it0, int n, bool rec, bool illum, int image_every, const long long *off,
+// The per-step kernels can start a schedule but not go on with one: the
+// checkpoints that a launch wrote have no border cells.
+static int unavailable(Run2dGroup &g)
+{
+    g.ok = -1;
+    return g.ran ? fail(VTI_ERR_HIP, "run2d: launch") : 0;
+}
+
+// prog: the operations, then the offsets
+int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::vector<long long> &offs, int image_every,
                     hipStream_t s)
 {
-    if (g.ok != 1 || n < 2 || n > kRun2dMax) return 0;
+    if (g.ok != 1) return 0;
+    const size_t nb = ops.size() * sizeof(Run2dOp), need = nb + std::max<size_t>(offs.size(), 1) * sizeof(long long);
+    if (need > g.prog_bytes) {
+        if (hipStreamSynchronize(s) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
+        (void)hipFree(g.prog);
+        g.prog = nullptr;
+        g.prog_bytes = 0;
+        if (hipMalloc(&g.prog, 2 * need) != hipSuccess) {
+            (void)hipGetLastError();
+            return unavailable(g);
+        }
+        g.prog_bytes = 2 * need;
+    }
+    static_assert(sizeof(Run2dOp) % sizeof(long long) == 0, "the offsets follow the operations");
+    char *p = static_cast<char *>(g.prog);
+    if (hipMemcpyAsync(p, ops.data(), nb, hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(p + nb, offs.data(), offs.size() * sizeof(long long), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return fail(VTI_ERR_HIP, "run2d: program");
     Run2dArgs a{};
-    a.many = g.dev + (role == 2 ? g.ns : 0);
-    a.ns = g.ns;
-    a.it0 = it0; a.n = n;
+    a.many = g.dev;
+    a.ns = (int)g.shots.size();
+    a.ops = reinterpret_cast<const Run2dOp *>(p);
+    a.nops = (int)ops.size();
+    a.offs = reinterpret_cast<const long long *>(p + nb);
+    a.image_every = image_every;
     a.base = g.base;
     a.dead = g.dead;
-    a.rec = rec; a.illum = illum;
-    a.image_every = image_every;
-    std::copy(off, off + n, a.off);
-    const KernelFn k = role == 1 ? (g.us ? kernel_of<false, true, 1>(g.shape) : kernel_of<false, false, 1>(g.shape))
-                                 : (g.us ? kernel_of<false, true, 2>(g.shape) : kernel_of<false, false, 2>(g.shape));
-    if (!launch_coop(k, g.ntile, kShapes[g.shape].nt, g.lds, a, s)) {
-        g.ok = -1;
-        return 0;
-    }
-    g.base += (unsigned)n;
+    const KernelFn k = g.us ? kernel_of<false, true, true>(g.shape) : kernel_of<false, false, true>(g.shape);
+    if (!launch_coop(k, g.ntile, kShapes[g.shape].nt, g.lds, a, s)) return unavailable(g);
+    g.ran = true;
+    g.base += (unsigned)(offs.size() + 2);   // one exchange a step
     return 1;
 }
 
 int run2d_group_check(Run2dGroup &g) { return dead_check(g.dead, g.ok); }
 
-int RtmQueue::forward(bool first, int it)
+int RtmProgram::steps(int kind, bool first, int it, long long off)
 {
-    const int k = first ? 1 : 2;
-    if (n && (kind != k || it != it0 + n || n == kRun2dMax)) {
-        const int e = flush();
-        if (e) return e;
+    const int d = kind == 2 ? -1 : 1;
+    if (!ops.empty()) {
+        Run2dOp &l = ops.back();
+        if (l.kind == kind && l.first == (int)first && it == l.it0 + d * l.n) {
+            ++l.n;
+            offs.push_back(off);
+            return VTI_OK;
+        }
     }
-    if (!n) {
-        kind = k;
-        it0 = it;
+    // the run goes on from the state on the chip, a forward one over checkpoints
+    for (size_t k = ops.size(); k-- > 0;) {
+        if (kind == 1 && ops[k].kind == 3) continue;
+        if (ops[k].kind == kind) ops[k].link = 1;
+        break;
     }
-    off[n++] = 0;
+    ops.push_back(Run2dOp{kind, it, 1, (int)first, 0, (int)offs.size(), 0});
+    offs.push_back(off);
     return VTI_OK;
 }
 
-int RtmQueue::keep_last(long long o)
+int RtmProgram::keep_last(long long off)
 {
-    if (n && kind != 3 && !off[n - 1]) {
-        off[n - 1] = o;
-        return VTI_OK;
-    }
-    const int e = flush();
-    return e ? e : keep(o);
-}
-
-int RtmQueue::receiver(int it, long long o)
-{
-    if (n && (kind != 3 || it != it0 - n || n == kRun2dMax)) {
-        const int e = flush();
-        if (e) return e;
-    }
-    if (!n) {
-        kind = 3;
-        it0 = it;
-    }
-    off[n++] = o;
+    if (ops.empty() || ops.back().kind != 1 || offs.back()) return fail(VTI_ERR_STATE, "RTM program: no step to keep");
+    offs.back() = off;
     return VTI_OK;
 }
 
-int RtmQueue::flush()
+int RtmProgram::state(int kind, long long slot)
 {
-    const int m = n;
-    n = 0;
-    if (m >= kMinRun) {
-        const int e = kind == 3 ? run_receive(it0, m, off) : run_forward(kind == 1, it0, m, off);
-        if (e) return e < 0 ? e : VTI_OK;
-    }
-    for (int k = 0; k < m; ++k) {
-        int e = kind == 3 ? receive(it0 - k, off[k]) : step(kind == 1, it0 + k);
-        if (!e && kind != 3 && off[k]) e = keep(off[k]);
+    // a checkpoint is written from the chip
+    if (kind == 3 && (ops.empty() || ops.back().kind != 1)) return fail(VTI_ERR_STATE, "RTM program: no step to store");
+    ops.push_back(Run2dOp{kind, 0, 0, 0, 0, 0, slot});
+    return VTI_OK;
+}
+
+int RtmProgram::flush()
+{
+    std::vector<Run2dOp> o;
+    std::vector<long long> f;
+    o.swap(ops);
+    f.swap(offs);
+    if (o.empty()) return VTI_OK;
+    int e = run(o, f);
+    if (e) return e < 0 ? e : VTI_OK;
+    for (const Run2dOp &op : o) {
+        if (op.kind >= 3) e = move(op.kind, op.slot);
+        else
+            for (int k = 0; k < op.n && !e; ++k) {
+                if (op.kind == 2) e = receive(op.it0 - k, f[op.off0 + k]);
+                else if (!(e = step(op.first != 0, op.it0 + k)) && f[op.off0 + k]) e = keep(f[op.off0 + k]);
+            }
         if (e) return e;
     }
     return VTI_OK;
