@@ -37,5 +37,7 @@ hipError_t launch_image(vti_ctx *c, const float *sP, const float *gP, float *img
 hipError_t launch_illum(vti_ctx *c, const float *P, const float *Q, float *illum, int clamp);
 hipError_t launch_divide(vti_ctx *c, float *img, const float *illum, size_t n, int guard);
 void laplace_adj(int nz, int nx, int ny, const float *in, float *out);
+int fetch_image(hipStream_t s, const float *dimg, const float *dillum, int nz, int nx, int ny, int finalize, bool guard,
+                float *img, float *illum, const char *what);
 
 }  // namespace vti

@@ -211,11 +211,14 @@ struct CkSlots {
     CkGeom q{};
     int nbase = 0, nsplit = 0;
     long long slot_floats = 0;
-    std::vector<float *> mem;      // one allocation per slot
+    // one allocation for all slots (600 x 300, 32 slots: 32 pairs of hipMalloc
+    // and hipFree took ~6 of a shot's 14.6 ms)
+    float *base = nullptr;
+    std::vector<float *> mem;      // each slot's share
     std::vector<VtiState> view;    // whole-volume fields of each slot (split fields: full slots only)
     ~CkSlots()
     {
-        for (float *p : mem) (void)hipFree(p);
+        (void)hipFree(base);
     }
 };
 
@@ -269,11 +272,14 @@ int ck_alloc(vti_ctx *c, CkSlots &k, int nslot)
 {
     k.mem.assign(nslot, nullptr);
     k.view.assign(nslot, VtiState{});
+    const size_t pitch = ((size_t)k.slot_floats + 63) / 64 * 64;
+    if (nslot > 0 && hipMalloc(&k.base, (size_t)nslot * pitch * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        k.base = nullptr;
+        return fail(VTI_ERR_ALLOC, "checkpoint slots");
+    }
     for (int i = 0; i < nslot; ++i) {
-        if (hipMalloc(&k.mem[i], (size_t)k.slot_floats * sizeof(float)) != hipSuccess) {
-            k.mem[i] = nullptr;
-            return fail(VTI_ERR_ALLOC, "checkpoint slots");
-        }
+        k.mem[i] = k.base + (size_t)i * pitch;
         if (!k.compact) {   // a full state, laid out as state_alloc lays it out
             static const int order3[11] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10};
             static const int order2[8] = {0, 2, 3, 5, 6, 8, 9, 10};
@@ -480,7 +486,7 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
         a.pxlo = ck.q.xlo; a.pxhi = ck.q.xhi; a.pzlo = ck.q.zlo; a.pzhi = ck.q.zhi;
         a.pvol = (long long)c->nvol;
         a.psplit = ck.q.split_n;
-        if ((st = run2d_group_make(grp, {a}, c->unsplit, c->device, c->stream)) < 0) return st;
+        if ((st = run2d_group_make(grp, run2d_parts({a}, c->device), {a}, c->unsplit, nt, c->stream)) < 0) return st;
     }
     if (grp.ok == 1) {
         if ((st = op.zero())) return st;   // the border cells, which no step changes
@@ -523,8 +529,33 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
     if ((st = reverse_sweep(nt, nslot, op, fwd_steps))) return st;
     if (grp.ok && (st = q.flush())) return st;
     if ((st = hip(hipStreamSynchronize(c->stream), "sync"))) return st;
-    return run2d_group_check(grp);
+    return run2d_group_check(grp, c->stream);
 }
+
+}  // extern "C"
+
+// The interior image and illumination to the host (either may be null), the
+// raw ones straight into the caller's arrays.
+int vti::fetch_image(hipStream_t s, const float *dimg, const float *dillum, int nz, int nx, int ny, int finalize, bool guard,
+                     float *img, float *illum, const char *what)
+{
+    const size_t n = (size_t)nz * nx * ny;
+    const bool fin = finalize && img;
+    std::vector<float> hi(fin ? n : 0), hl(fin && !illum ? n : 0);
+    float *pi = fin ? hi.data() : img, *pl = fin && !illum ? hl.data() : illum;
+    if (hipStreamSynchronize(s) != hipSuccess ||
+        (pi && hipMemcpy(pi, dimg, n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess) ||
+        (pl && hipMemcpy(pl, dillum, n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess))
+        return fail(VTI_ERR_HIP, what);
+    if (!fin) return VTI_OK;
+    // migration_illum then laplace_filter(adj=1) (:1486-1493)
+    for (size_t i = 0; i < n; ++i)
+        if (!guard || pl[i] != 0.0f) pi[i] /= pl[i];
+    laplace_adj(nz, nx, ny, pi, img);
+    return VTI_OK;
+}
+
+extern "C" {
 
 // One imaging step of a caller-driven RTM (cal_migration
 // Toa_gpu2DvtiFdRtmAdcigsLaplace.cu:679-698, 3D
@@ -558,24 +589,8 @@ int vti_image_accumulate(vti_ctx *src, vti_ctx *rcv, float *img, float *illum, i
 int vti_rtm_image(vti_ctx *c, int finalize, float *img, float *illum)
 {
     if (!c || !c->img) return fail(VTI_ERR_STATE, "vti_rtm_image: no image");
-    const size_t n = c->nint;
-    std::vector<float> hi(n), hl(n);
-    if (hipStreamSynchronize(c->stream) != hipSuccess ||
-        hipMemcpy(hi.data(), c->img, n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(hl.data(), c->illum, n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(VTI_ERR_HIP, "vti_rtm_image: copy");
-    if (illum) std::memcpy(illum, hl.data(), n * sizeof(float));
-    if (!img) return VTI_OK;
-    if (!finalize) {
-        std::memcpy(img, hi.data(), n * sizeof(float));
-        return VTI_OK;
-    }
-    // migration_illum then laplace_filter(adj=1) (:1486-1493)
-    const bool guard = c->rtm_illum_mode == 1;
-    for (size_t i = 0; i < n; ++i)
-        if (!guard || hl[i] != 0.0f) hi[i] /= hl[i];
-    laplace_adj(c->cfg.nz, c->cfg.nx, c->cfg.ndim == 3 ? c->cfg.ny : 1, hi.data(), img);
-    return VTI_OK;
+    return fetch_image(c->stream, c->img, c->illum, c->cfg.nz, c->cfg.nx, c->cfg.ndim == 3 ? c->cfg.ny : 1, finalize,
+                       c->rtm_illum_mode == 1, img, illum, "vti_rtm_image: copy");
 }
 
 }  // extern "C"

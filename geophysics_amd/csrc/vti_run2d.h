@@ -57,32 +57,41 @@ struct Run2dOp {
     long long slot;  // 3, 4: floats from the state to the checkpoint (packed: from u to its start)
 };
 
-// Shots that step together in one launch.
+// The parts of a list of shots: consecutive ones step together in one launch.
+struct Run2dPart {
+    int first, n;               // shots
+    int shape, ntile;
+    size_t lds;
+};
+struct Run2dParts {
+    std::vector<Run2dPart> part;   // empty: not available, the per-step kernels run all of them
+    std::vector<int> gx, gz, tile0;
+};
+
 struct Run2dGroup {
     int ok = 0;                 // 1: usable
     bool ran = false;           // a program has run
-    int ntile = 0, shape = 0;
-    size_t lds = 0;
     bool us = false;
-    std::vector<Run2dShot> shots;
+    Run2dParts parts;
+    void *mem = nullptr, *more = nullptr;   // more: a program larger than mem's share
     Run2dShot *dev = nullptr;
-    unsigned long long *xbuf = nullptr;
     void *prog = nullptr;
-    size_t prog_bytes = 0;
+    size_t prog_bytes = 0, words = 0;       // words: exchange planes
     unsigned base = 1;          // tag before the next run's first exchange; the planes start with tag 0
-    int *dead = nullptr;        // pinned, mapped
+    int *dead = nullptr;        // on the device: an exchange that never came
 };
 
-// Most consecutive shots from `first` on that one group can hold (0: not
-// even one; the per-step kernels run it).
-int run2d_fit(const std::vector<Run2dShot> &shots, int first, int device);
+Run2dParts run2d_parts(const std::vector<Run2dShot> &shots, int device);
 // 1: made, 0: not available here, < 0: error
-int run2d_group_make(Run2dGroup &g, const std::vector<Run2dShot> &shots, bool us, int device, hipStream_t s);
+int run2d_group_make(Run2dGroup &g, const Run2dParts &p, std::vector<Run2dShot> shots, bool us, int nt, hipStream_t s);
+// other shots on the same grids (their pointers, source and receivers)
+int run2d_group_set(Run2dGroup &g, std::vector<Run2dShot> shots, hipStream_t s);
 void run2d_group_free(Run2dGroup &g);
-// 1: launched, 0: not available, < 0: error
+// the program on every part; 1: launched, 0: not available, < 0: error
 int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::vector<long long> &offs, int image_every,
                     hipStream_t s);
-int run2d_group_check(Run2dGroup &g);
+// waits for the stream
+int run2d_group_check(Run2dGroup &g, hipStream_t s);
 
 // Collects the operations that an RTM's schedule asks for one by one, so that
 // flush() runs them as one resident launch: a cooperative launch costs ~100 us

@@ -65,7 +65,7 @@ struct Run2dArgs {
     const long long *offs;
     int image_every;
     unsigned base;              // tag before the call's first exchange
-    int *dead;                  // host-visible error word
+    int *dead;                  // error word
 };
 
 // an opaque copy: what is derived from it inside the step loop is not hoisted
@@ -828,25 +828,37 @@ struct Cut {
     size_t lds;
     double cost;
 };
+// out: by ascending tiles, each cheaper than all with fewer
 void cuts_of(int nnx, int nnz, bool tti, int shape, int cus, int lds_max, std::vector<Cut> &out)
 {
     out.clear();
     const int ux = nnx - 8, uq = (nnz - 8 + 3) / 4;
     if (uq < 2) return;
     const int nt = kShapes[shape].nt, nu = kShapes[shape].nu;
-    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); ++gx)
-        for (int gz = 1; gz <= std::min(cus / gx, std::max(1, uq / 2)); ++gz) {
-            const int nx = (ux + gx - 1) / gx, nz = 4 * ((uq + gz - 1) / gz);
-            const int strips = (nx + nu - 1) / nu * nz;
-            if (strips > nt || nx + 14 > nt) continue;
+    std::vector<Cut> best(cus + 1, Cut{0, 0, 0, 0, 1e300});   // by tiles
+    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); ++gx) {
+        const int nx = (ux + gx - 1) / gx, rows = (nx + nu - 1) / nu;
+        if (nx + 14 > nt || 8 * rows > nt) continue;
+        const int widest = nt / rows / 4;   // units of 4 columns that leave a thread one strip
+        for (int gz = (uq + widest - 1) / widest; gz <= std::min(cus / gx, std::max(1, uq / 2)); ++gz) {
+            const int nz = 4 * ((uq + gz - 1) / gz);
+            const int strips = rows * nz;
             const size_t b = 4 * (size_t)(tti ? Lds<true>(nx, nz).total : Lds<false>(nx, nz).total);
             if (b + 64 > (size_t)lds_max) continue;
-            const int us = (nx + 7 + nu - 1) / nu * (tti ? nz + 8 : nz), ws = tti ? 0 : (nx + nu - 1) / nu * (nz + 8);
+            const int us = (nx + 7 + nu - 1) / nu * (tti ? nz + 8 : nz), ws = tti ? 0 : rows * (nz + 8);
             const double f = tti ? 2.0 : 1.0;
             const double issue = f * nu * (20.0 * us + 26.0 * ws + 50.0 * strips) / 64.0;
             const double wait = f * ((us + ws + nt - 1) / nt * (350.0 + 60.0 * nu) + 300.0 + 90.0 * nu);
             const double words = (tti ? 2.0 : 1.0) * 14.0 * (nx + nz + (tti ? 14 : 0));
-            out.push_back(Cut{gx, gz, gx * gz, b, std::max(issue, wait) + 0.25 * words});
+            const double cost = std::max(issue, wait) + 0.25 * words;
+            if (cost < best[gx * gz].cost) best[gx * gz] = Cut{gx, gz, gx * gz, b, cost};
+        }
+    }
+    double least = 1e300;
+    for (const Cut &c : best)
+        if (c.cost < least) {
+            least = c.cost;
+            out.push_back(c);
         }
 }
 
@@ -865,31 +877,46 @@ bool device_2d(int device, Device2d &d)
     return true;
 }
 
-// One tile per CU for all shots together, the same launch shape: the shape
-// and the cuts with the least cost of the slowest tile.
-bool plan_group(std::vector<Run2dShot> &shots, bool tti, int nshape, const Device2d &d, int &shape, size_t &lds, int &ntile)
+// One tile per CU for n shots together, the same launch shape: the shape and
+// the cuts with the least cost of the slowest tile.  cuts: [shape][shot].
+struct Plan2d {
+    double cost = 1e300;
+    int shape = 0;
+    std::vector<Cut> cut;
+};
+using Cuts2d = std::vector<std::vector<std::vector<Cut>>>;
+Cuts2d cuts_of_all(const std::vector<Run2dShot> &shots, bool tti, int nshape, const Device2d &d)
 {
-    const int ns = (int)shots.size();
-    double best = 1e300;
-    std::vector<Cut> pick(ns), chosen;
+    Cuts2d cuts(nshape);
     for (int k = 0; k < nshape; ++k) {
-        std::vector<std::vector<Cut>> cuts(ns);
+        cuts[k].resize(shots.size());
+        for (size_t s = 0; s < shots.size(); ++s) cuts_of(shots[s].nnx, shots[s].nnz, tti, k, d.cus, d.lds, cuts[k][s]);
+    }
+    return cuts;
+}
+Plan2d plan_group(const Cuts2d &cuts, int first, int n, const Device2d &d)
+{
+    Plan2d best;
+    std::vector<Cut> pick(n);
+    for (size_t k = 0; k < cuts.size(); ++k) {
         std::vector<double> costs;
         bool all = true;
-        for (int s = 0; s < ns && all; ++s) {
-            cuts_of(shots[s].nnx, shots[s].nnz, tti, k, d.cus, d.lds, cuts[s]);
-            all = !cuts[s].empty();
-            for (const Cut &c : cuts[s]) costs.push_back(c.cost);
+        for (int s = 0; s < n && all; ++s) {
+            all = !cuts[k][first + s].empty();
+            for (const Cut &c : cuts[k][first + s]) costs.push_back(c.cost);
         }
         if (!all) continue;
         std::sort(costs.begin(), costs.end());
         auto fits = [&](double c) {   // fewest tiles of every shot within cost c
-            int n = 0;
-            for (int s = 0; s < ns; ++s) {
+            int tiles = 0;
+            for (int s = 0; s < n; ++s) {
                 const Cut *b = nullptr;
-                for (const Cut &x : cuts[s])
-                    if (x.cost <= c && (!b || x.tiles < b->tiles || (x.tiles == b->tiles && x.cost < b->cost))) b = &x;
-                if (!b || (n += b->tiles) > d.cus) return false;
+                for (const Cut &x : cuts[k][first + s])
+                    if (x.cost <= c) {
+                        b = &x;
+                        break;
+                    }
+                if (!b || (tiles += b->tiles) > d.cus) return false;
                 pick[s] = *b;
             }
             return true;
@@ -900,40 +927,27 @@ bool plan_group(std::vector<Run2dShot> &shots, bool tti, int nshape, const Devic
             if (fits(costs[mid])) hi = mid;
             else lo = mid + 1;
         }
-        if (lo == costs.size() || costs[lo] >= best || !fits(costs[lo])) continue;
-        best = costs[lo];
-        shape = k;
-        chosen = pick;
+        if (lo == costs.size() || costs[lo] >= best.cost || !fits(costs[lo])) continue;
+        best.cost = costs[lo];
+        best.shape = (int)k;
+        best.cut = pick;
     }
-    if (best == 1e300) return false;
-    lds = 0;
-    ntile = 0;
-    for (int s = 0; s < ns; ++s) {
-        shots[s].gx = chosen[s].gx;
-        shots[s].gz = chosen[s].gz;
-        shots[s].tile0 = ntile;
-        ntile += chosen[s].tiles;
-        lds = std::max(lds, chosen[s].lds);
-    }
-    return true;
+    return best;
 }
 
 size_t plane_of(const Run2dShot &s) { return (size_t)s.ldz * s.nnx; }
 
-// the exchange planes of every shot, zeroed, and the error word
-bool alloc_group(std::vector<Run2dShot> &shots, int nfield, unsigned long long *&xbuf, int *&dead, hipStream_t s)
+// words of the exchange planes, two a field
+size_t plane_words(const Run2dShot *shots, int n, int nfield)
 {
-    size_t n = 0;
-    for (const Run2dShot &b : shots) n += 2 * nfield * plane_of(b);
-    if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess ||
-        launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    *dead = 0;
-    unsigned long long *p = xbuf;
-    for (Run2dShot &b : shots) {
+    size_t w = 0;
+    for (int k = 0; k < n; ++k) w += 2 * nfield * plane_of(shots[k]);
+    return w;
+}
+void place_planes(Run2dShot *shots, int n, int nfield, unsigned long long *p)
+{
+    for (int k = 0; k < n; ++k) {
+        Run2dShot &b = shots[k];
         b.xstride = (long long)plane_of(b);
         b.xP = p;
         b.xQ = p + 2 * plane_of(b);
@@ -941,6 +955,20 @@ bool alloc_group(std::vector<Run2dShot> &shots, int nfield, unsigned long long *
         b.xW = nfield > 2 ? p + 6 * plane_of(b) : nullptr;
         p += 2 * nfield * plane_of(b);
     }
+}
+
+// a context's exchange planes, zeroed, and its host-visible error word
+bool alloc_plan(std::vector<Run2dShot> &shots, unsigned long long *&xbuf, int *&dead, hipStream_t s)
+{
+    const size_t n = plane_words(shots.data(), 1, 2);
+    if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess ||
+        launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    *dead = 0;
+    place_planes(shots.data(), 1, 2, xbuf);
     return true;
 }
 
@@ -1034,9 +1062,14 @@ int run2d_steps(vti_ctx *c, int it0, int n)
         p.ok = -1;
         Device2d d;
         p.shot.push_back(run2d_shot(c, main_state(c)));
-        if (!device_2d(c->device, d) || !plan_group(p.shot, tti, kNumShapes, d, p.shape, p.lds, p.ntile) ||
-            !alloc_group(p.shot, 2, p.xbuf, p.dead, c->stream))
-            return 0;
+        if (!device_2d(c->device, d)) return 0;
+        const Plan2d one = plan_group(cuts_of_all(p.shot, tti, kNumShapes, d), 0, 1, d);
+        if (one.cut.empty() || !alloc_plan(p.shot, p.xbuf, p.dead, c->stream)) return 0;
+        p.shape = one.shape;
+        p.lds = one.cut[0].lds;
+        p.ntile = one.cut[0].tiles;
+        p.shot[0].gx = one.cut[0].gx;
+        p.shot[0].gz = one.cut[0].gz;
         p.ok = 1;
     }
     Run2dPlan &p = *c->run2d;
@@ -1074,47 +1107,93 @@ static int dead_check(int *dead, int &ok)
 int run2d_check(vti_ctx *c) { return c->run2d ? dead_check(c->run2d->dead, c->run2d->ok) : VTI_OK; }
 
 // ---- groups of shots (RTM) ---------------------------------------------------
-int run2d_fit(const std::vector<Run2dShot> &shots, int first, int device)
+// Consecutive shots to a part while that lowers the time a cell: the slowest
+// tile's cost and what a step costs besides (exchange, barriers: ~2 us).
+Run2dParts run2d_parts(const std::vector<Run2dShot> &shots, int device)
 {
+    Run2dParts r;
     Device2d d;
-    if (!device_2d(device, d)) return 0;
-    int n = 0, tiles = 0;
-    std::vector<Cut> cuts;
-    for (size_t s = first; s < shots.size(); ++s, ++n) {
-        cuts_of(shots[s].nnx, shots[s].nnz, false, kRtmShapes - 1, d.cus, d.lds, cuts);
-        int least = d.cus + 1;
-        for (const Cut &c : cuts) least = std::min(least, c.tiles);
-        if ((tiles += least) > d.cus) break;
+    if (!device_2d(device, d)) return r;
+    const int ns = (int)shots.size();
+    Cuts2d cuts = cuts_of_all(shots, false, kRtmShapes, d);
+    // strips of 6 spill ~95 registers with the images: for shots that fit no
+    // other way (24 shots of 0.1 to 1 M cells: 46 ms in parts of strips of 6
+    // taken at their plain cost, 39 with parts of 4)
+    for (auto &c : cuts[kRtmShapes - 1])
+        for (Cut &x : c) x.cost *= 2.0;
+    for (int first = 0; first < ns;) {
+        Plan2d best;
+        double rate = 1e300, cells = 0.0;
+        for (int n = 1; first + n <= ns; ++n) {
+            cells += (double)shots[first + n - 1].nnx * shots[first + n - 1].nnz;
+            const Plan2d p = plan_group(cuts, first, n, d);
+            if (p.cut.empty()) break;
+            if ((p.cost + 4000.0) / cells >= rate) continue;
+            rate = (p.cost + 4000.0) / cells;
+            best = p;
+        }
+        if (best.cut.empty()) return Run2dParts{};
+        Run2dPart q{first, (int)best.cut.size(), best.shape, 0, 0};
+        for (const Cut &c : best.cut) {
+            r.gx.push_back(c.gx);
+            r.gz.push_back(c.gz);
+            r.tile0.push_back(q.ntile);
+            q.ntile += c.tiles;
+            q.lds = std::max(q.lds, c.lds);
+        }
+        r.part.push_back(q);
+        first += q.n;
     }
-    return n;
+    return r;
 }
 
-int run2d_group_make(Run2dGroup &g, const std::vector<Run2dShot> &shots, bool us, int device, hipStream_t s)
+// one allocation: exchange planes (tag 0; the parts run one after the other
+// and share them), error word, shots, program
+int run2d_group_make(Run2dGroup &g, const Run2dParts &p, std::vector<Run2dShot> shots, bool us, int nt, hipStream_t s)
 {
     g.ok = 0;
-    if (shots.empty() || capturing(s)) return 0;
-    Device2d d;
-    g.shots = shots;
+    if (p.part.empty() || capturing(s)) return 0;
+    g.parts = p;
     g.us = us;
-    if (!device_2d(device, d) || !plan_group(g.shots, false, kRtmShapes, d, g.shape, g.lds, g.ntile) ||
-        !alloc_group(g.shots, 4, g.xbuf, g.dead, s))
-        return 0;
-    if (hipMalloc(&g.dev, g.shots.size() * sizeof(Run2dShot)) != hipSuccess) {
+    g.words = 0;
+    for (const Run2dPart &q : p.part) g.words = std::max(g.words, plane_words(&shots[q.first], q.n, 4));
+    const size_t head = (g.words + 32) * 8, desc = (shots.size() * sizeof(Run2dShot) + 255) / 256 * 256;
+    g.prog_bytes = 128 * (size_t)nt + 65536;
+    if (hipMalloc(&g.mem, head + desc + g.prog_bytes) != hipSuccess) {
         (void)hipGetLastError();
+        g.mem = nullptr;
         return 0;
     }
-    if (hipMemcpy(g.dev, g.shots.data(), g.shots.size() * sizeof(Run2dShot), hipMemcpyHostToDevice) != hipSuccess)
-        return fail(VTI_ERR_HIP, "run2d: descriptors");
+    char *m = static_cast<char *>(g.mem);
+    g.dead = reinterpret_cast<int *>(m + g.words * 8);
+    g.dev = reinterpret_cast<Run2dShot *>(m + head);
+    g.prog = m + head + desc;
+    if (launch_zero(static_cast<float *>(g.mem), head / 4, s) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: planes");
+    const int e = run2d_group_set(g, std::move(shots), s);
+    if (e) return e;
     g.ok = 1;
     return 1;
 }
 
+int run2d_group_set(Run2dGroup &g, std::vector<Run2dShot> shots, hipStream_t s)
+{
+    const Run2dParts &p = g.parts;
+    for (size_t k = 0; k < shots.size(); ++k) {
+        shots[k].gx = p.gx[k];
+        shots[k].gz = p.gz[k];
+        shots[k].tile0 = p.tile0[k];
+    }
+    for (const Run2dPart &q : p.part) place_planes(&shots[q.first], q.n, 4, static_cast<unsigned long long *>(g.mem));
+    if (hipMemcpyAsync(g.dev, shots.data(), shots.size() * sizeof(Run2dShot), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return fail(VTI_ERR_HIP, "run2d: descriptors");
+    return VTI_OK;
+}
+
 void run2d_group_free(Run2dGroup &g)
 {
-    (void)hipFree(g.dev);
-    (void)hipFree(g.xbuf);
-    (void)hipFree(g.prog);
-    (void)hipHostFree(g.dead);
+    (void)hipFree(g.mem);
+    (void)hipFree(g.more);
     g = Run2dGroup{};
 }
 
@@ -1134,13 +1213,13 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
     const size_t nb = ops.size() * sizeof(Run2dOp), need = nb + std::max<size_t>(offs.size(), 1) * sizeof(long long);
     if (need > g.prog_bytes) {
         if (hipStreamSynchronize(s) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
-        (void)hipFree(g.prog);
-        g.prog = nullptr;
-        g.prog_bytes = 0;
-        if (hipMalloc(&g.prog, 2 * need) != hipSuccess) {
+        (void)hipFree(g.more);
+        g.more = nullptr;
+        if (hipMalloc(&g.more, 2 * need) != hipSuccess) {
             (void)hipGetLastError();
             return unavailable(g);
         }
+        g.prog = g.more;
         g.prog_bytes = 2 * need;
     }
     static_assert(sizeof(Run2dOp) % sizeof(long long) == 0, "the offsets follow the operations");
@@ -1149,23 +1228,33 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         hipMemcpyAsync(p + nb, offs.data(), offs.size() * sizeof(long long), hipMemcpyHostToDevice, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return fail(VTI_ERR_HIP, "run2d: program");
-    Run2dArgs a{};
-    a.many = g.dev;
-    a.ns = (int)g.shots.size();
-    a.ops = reinterpret_cast<const Run2dOp *>(p);
-    a.nops = (int)ops.size();
-    a.offs = reinterpret_cast<const long long *>(p + nb);
-    a.image_every = image_every;
-    a.base = g.base;
-    a.dead = g.dead;
-    const KernelFn k = g.us ? kernel_of<false, true, true>(g.shape) : kernel_of<false, false, true>(g.shape);
-    if (!launch_coop(k, g.ntile, kShapes[g.shape].nt, g.lds, a, s)) return unavailable(g);
-    g.ran = true;
-    g.base += (unsigned)(offs.size() + 2);   // one exchange a step
+    for (const Run2dPart &q : g.parts.part) {
+        Run2dArgs a{};
+        a.many = g.dev + q.first;
+        a.ns = q.n;
+        a.ops = reinterpret_cast<const Run2dOp *>(p);
+        a.nops = (int)ops.size();
+        a.offs = reinterpret_cast<const long long *>(p + nb);
+        a.image_every = image_every;
+        a.base = g.base;
+        a.dead = g.dead;
+        const KernelFn k = g.us ? kernel_of<false, true, true>(q.shape) : kernel_of<false, false, true>(q.shape);
+        if (!launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s)) return unavailable(g);
+        g.ran = true;
+        g.base += (unsigned)(offs.size() + 2);   // one exchange a step
+    }
     return 1;
 }
 
-int run2d_group_check(Run2dGroup &g) { return dead_check(g.dead, g.ok); }
+int run2d_group_check(Run2dGroup &g, hipStream_t s)
+{
+    if (!g.ran) return VTI_OK;
+    int dead = 0;
+    if (hipMemcpyAsync(&dead, g.dead, sizeof dead, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return fail(VTI_ERR_HIP, "run2d: check");
+    return dead_check(&dead, g.ok);
+}
 
 int RtmProgram::steps(int kind, bool first, int it, long long off)
 {

@@ -95,6 +95,39 @@ def test_resident_rtm_equals_per_step_kernels(unsplit, illum_mode, every, modell
         assert np.array_equal(f0[k], f1[k]), k
 
 
+@pytest.mark.parametrize("unsplit", [False, True])
+@pytest.mark.parametrize("large", [(2401, 403), (2401, 1003)])
+def test_resident_batch_in_parts_equals_single_shots(unsplit, large):
+    """More shots than one launch holds, with one of strips of six rows or
+    one that fits no launch (per-step kernels for all)."""
+    sizes, nt = [(900, 301), (333, 71), (1200, 500), (16, 17), (60, 50), large, (700, 301)], 12
+    rng = np.random.default_rng(11)
+    cfgs, shots, models, obs = [], [], [], []
+    for k, (nx, nz) in enumerate(sizes):
+        cfgs.append(vti.cfg_ref2d(vti.MODE_GPU_REF, nx, nz, 10, 10, 4 + k, k % 2, 20, nt, 1000))
+        shots.append(vti.shot_ref2d(cfgs[k], 1, nx // 2, 0, 3))
+        ep = (0.2 * rng.random((nx, nz))).astype(np.float32)
+        models.append(((2200.0 + 600.0 * rng.random((nx, nz))).astype(np.float32), ep, (0.5 * ep).astype(np.float32)))
+        obs.append(rng.standard_normal((shots[k].rec_nx, nt)).astype(np.float32))
+    o = vti.rtm_defaults(2)
+    o.nsnap = 2
+    with vti.Batch(cfgs, shots, models) as B:
+        B.set_unsplit(unsplit)
+        for _ in range(2):
+            B.rtm(o, obs)
+        got = [B.image(k) for k in range(len(sizes))]
+    for k, (cfg, shot, m) in enumerate(zip(cfgs, shots, models)):
+        with vti.Propagator(cfg, *m) as p:
+            p.set_unsplit(unsplit)
+            p.adcig_config(2)             # step by step
+            p.set_shot(shot)
+            p.rtm_reset()
+            p.rtm_shot(o, obs[k])
+            img, ill = p.rtm_image(finalize=False)
+        assert np.abs(img).max() > 0
+        assert np.array_equal(got[k][1], ill) and np.array_equal(got[k][0], img), k
+
+
 def test_resident_steps_of_several_contexts_and_threads():
     """Contexts on streams of their own, stepped from four threads at once."""
     import threading
