@@ -39,6 +39,7 @@
 
 #include "vti_internal.h"
 #include "vti_rtm.h"
+#include "vti_run2d.h"
 
 namespace vti {
 namespace {
@@ -188,34 +189,46 @@ __global__ void gcoef(GGrid g, const T *vp, const T *ep, const T *de, const T *t
 }
 
 // ---- adjoint --------------------------------------------------------------
-template <typename T>
-__global__ void gadj_rec(GGrid g, Fields<T> a, const T *r, int rkind, int rz, int rx0, int rdx, int rnx,
-                         int ry0, int rdy, int rny)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= rnx * rny) return;
-    const int ix = rx0 + (k % rnx) * rdx, iy = g.three ? ry0 + (k / rnx) * rdy : 0;
-    const long long c = rz + (long long)ix * g.ldz + (long long)iy * g.ldxy;
-    const T v = r[k];
-    if (rkind == 0) a.P[c] += v;
-    else if (rkind == 1) a.P[c] += v + v;
-    else { a.P[c] += v; a.Q[c] += v; }
-}
+// Two passes a step, each up to a point where neighbours' values are needed:
+// memory traffic (2D: 28 values a cell and step) and, on small grids, the
+// launches bound it.  Residual, P~/Q~, source gradient and the four halves of
+// the transposed updates as passes of their own moved 40 and took six
+// launches: 1040 x 340 cells, 400 steps: 10.1 -> 5.2 ms of adjoint kernels.
 
-// stress^T, phase A: distribute P~, Q~ to the splits, accumulate the
-// gradient against the forward state fw (after the step), form F.
+// The rest of vel^T of step n+1 (P~ += D- Hx (+ D- Hy), Q~ += D- Hz; P~ and
+// Q~ were 0) with its source gradient, then step n's residual and the first
+// half of stress^T: distribute P~, Q~ to the splits (P~ = Q~ = 0 again, so
+// neither is stored), accumulate the gradient against the forward state fw
+// (after the step), form F.  sg: step n+1's source gradient, nullptr: n is
+// the last step; r: step n's residual, nullptr: n + 1 was the first step.
 template <typename T>
-__global__ __launch_bounds__(256) void gadj_stress_a(GGrid g, Fields<T> a, Fields<T> fw, Coef<T> c, T *Fx,
-                                                     T *Fy, T *Fz, T *grad)
+__global__ __launch_bounds__(256) void gadj_p(GGrid g, Fields<T> a, const T *Hx, const T *Hy, const T *Hz, Fields<T> fw,
+                                              Coef<T> c, T *Fx, T *Fy, T *Fz, T *grad, long long src, T *sg, const T *r,
+                                              int rkind, int rz, int rx0, int rdx, int rnx, int ry0, int rdy, int rny)
 {
     int ix, iy, iz;
     long long id;
     if (!cell(g, ix, iy, iz, id)) return;
     const long long sx = g.ldz, sy = g.ldxy;
-    const T Pa = a.P[id], Qa = a.Q[id];
+    T p = 0, q = 0, py = 0;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        p += cm<T>(m) * (Hx[id + m * sx] - Hx[id - (m + 1) * sx]);
+        q += cm<T>(m) * (Hz[id + m] - Hz[id - m - 1]);
+        if (g.three) py += cm<T>(m) * (Hy[id + m * sy] - Hy[id - (m + 1) * sy]);
+    }
+    T Pa = T(0) + (g.three ? p + py : p), Qa = T(0) + q;
+    if (sg && id == src) *sg = Pa + Qa;
+    if (!r) return;
+    if (iz == rz) {
+        const int k = ix - rx0, j = g.three ? iy - ry0 : 0;
+        if (k >= 0 && k % rdx == 0 && k / rdx < rnx && j >= 0 && j % rdy == 0 && j / rdy < rny) {
+            const T v = r[k / rdx + (long long)rnx * (j / rdy)];
+            Pa += rkind == 1 ? v + v : v;
+            if (rkind != 0 && rkind != 1) Qa += v;
+        }
+    }
     const T spx = a.px[id] + Pa, spz = a.pz[id] + Pa, sqx = a.qx[id] + Qa, sqz = a.qz[id] + Qa;
-    a.P[id] = 0;
-    a.Q[id] = 0;
     T xx = 0, yy = 0, zz = 0;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -243,9 +256,11 @@ __global__ __launch_bounds__(256) void gadj_stress_a(GGrid g, Fields<T> a, Field
     grad[id] += gsum;
 }
 
-// stress^T, phase B: u~ += D+ F (gather form of the transpose of D-).
+// The rest of stress^T, u~ += D+ F (gather form of the transpose of D-), and
+// the first half of vel^T: H = coff1*dt/dx * u~, u~ *= coff2.
 template <typename T>
-__global__ __launch_bounds__(256) void gadj_stress_b(GGrid g, Fields<T> a, const T *Fx, const T *Fy, const T *Fz)
+__global__ __launch_bounds__(256) void gadj_u(GGrid g, Fields<T> a, Coef<T> c, const T *Fx, const T *Fy, const T *Fz,
+                                              T *Hx, T *Hy, T *Hz)
 {
     int ix, iy, iz;
     long long id;
@@ -258,55 +273,18 @@ __global__ __launch_bounds__(256) void gadj_stress_b(GGrid g, Fields<T> a, const
         wz += cm<T>(m) * (Fz[id + m + 1] - Fz[id - m]);
         if (g.three) vy += cm<T>(m) * (Fy[id + (m + 1) * sy] - Fy[id - m * sy]);
     }
-    a.u[id] += ux;
-    a.w[id] += wz;
-    if (g.three) a.v[id] += vy;
-}
-
-// vel^T, phase A: H = coff1*dt/dx * u~, u~ *= coff2.
-template <typename T>
-__global__ __launch_bounds__(256) void gadj_vel_a(GGrid g, Fields<T> a, Coef<T> c, T *Hx, T *Hy, T *Hz)
-{
-    int ix, iy, iz;
-    long long id;
-    if (!cell(g, ix, iy, iz, id)) return;
     const T *t = c.tab;
     const int M = c.M;
-    const T ua = a.u[id], wa = a.w[id];
+    const T ua = a.u[id] + ux, wa = a.w[id] + wz;
     Hx[id] = t[0 * M + ix] * c.dtx * ua;
     Hz[id] = t[4 * M + iz] * c.dtz * wa;
     a.u[id] = t[1 * M + ix] * ua;
     a.w[id] = t[5 * M + iz] * wa;
     if (g.three) {
-        const T va = a.v[id];
+        const T va = a.v[id] + vy;
         Hy[id] = t[2 * M + iy] * c.dty * va;
         a.v[id] = t[3 * M + iy] * va;
     }
-}
-
-// vel^T, phase B: P~ += D- Hx (+ D- Hy), Q~ += D- Hz.
-template <typename T>
-__global__ __launch_bounds__(256) void gadj_vel_b(GGrid g, Fields<T> a, const T *Hx, const T *Hy, const T *Hz)
-{
-    int ix, iy, iz;
-    long long id;
-    if (!cell(g, ix, iy, iz, id)) return;
-    const long long sx = g.ldz, sy = g.ldxy;
-    T p = 0, q = 0, py = 0;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        p += cm<T>(m) * (Hx[id + m * sx] - Hx[id - (m + 1) * sx]);
-        q += cm<T>(m) * (Hz[id + m] - Hz[id - m - 1]);
-        if (g.three) py += cm<T>(m) * (Hy[id + m * sy] - Hy[id - (m + 1) * sy]);
-    }
-    a.P[id] += g.three ? p + py : p;
-    a.Q[id] += q;
-}
-
-template <typename T>
-__global__ void gsrc_grad(const T *P, const T *Q, long long src, T *out)
-{
-    if (threadIdx.x == 0) *out = P[src] + Q[src];
 }
 
 template <typename T>
@@ -397,7 +375,7 @@ struct Grad : vti_grad {
     hipStream_t stream = nullptr;
     T *arena = nullptr;
     T *vp = nullptr, *ep = nullptr, *de = nullptr, *C[6] = {}, *tab = nullptr, *grad = nullptr;
-    T *tmp[3] = {};
+    T *tmp[3] = {}, *hy = nullptr;
     Fields<T> f{}, a{};
     std::vector<T> htab, amp;
     std::vector<double> hvp;     // interior vp (host) for the final scaling
@@ -407,6 +385,9 @@ struct Grad : vti_grad {
     T *rec = nullptr, *res = nullptr, *sgrad = nullptr;
     double *dtap = nullptr;
     std::vector<T *> slots;
+    Run2dGroup res2d;            // 2D, FP32: the resident first sweep
+    float *damp = nullptr;       // its source gains
+    int res2d_state = 0;         // 1: made, -1: not available
 
     ~Grad() override
     {
@@ -418,6 +399,8 @@ struct Grad : vti_grad {
         (void)hipFree(res);
         (void)hipFree(sgrad);
         (void)hipFree(dtap);
+        (void)hipFree(damp);
+        run2d_group_free(res2d);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -452,7 +435,7 @@ struct Grad : vti_grad {
         g.ldxy = (long long)g.ldz * g.nnx;
         nvol = (size_t)g.ldxy * g.nny;
         M = std::max(g.nnx, std::max(g.nny, g.nnz));
-        const int nf = 3 + 6 + 1 + 3 + 2 * nstate();   // model, C, grad, tmp, fwd, adj
+        const int nf = 3 + 6 + 1 + 3 + 2 * nstate() + (three ? 1 : 0);   // model, C, grad, tmp, fwd, adj, hy
         if (hipMalloc(&arena, (size_t)nf * nvol * sizeof(T)) != hipSuccess) return fail(VTI_ERR_ALLOC, "vti_grad: arena");
         if (hipMalloc(&tab, 12 * (size_t)M * sizeof(T)) != hipSuccess) return fail(VTI_ERR_ALLOC, "vti_grad: tables");
         if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return fail(VTI_ERR_HIP, "stream");
@@ -462,7 +445,8 @@ struct Grad : vti_grad {
         grad = p; p += nvol;
         for (int k = 0; k < 3; ++k) { tmp[k] = p; p += nvol; }
         set_fields(f, p, nvol, three); p += nstate() * nvol;
-        set_fields(a, p, nvol, three);
+        set_fields(a, p, nvol, three); p += nstate() * nvol;
+        if (three) hy = p;
         zero(arena, (size_t)nf * nvol);
         htab.assign(12 * (size_t)M, T(1));
         return sync();
@@ -605,20 +589,71 @@ struct Grad : vti_grad {
                            shot.rec_x0, shot.rec_dx, shot.rec_nx, shot.rec_y0, shot.rec_dy, shot.rec_ny);
     }
 
-    void adj_step(int it, const Fields<T> &fw)
+    // H lies where P~ and Q~ (and, in 3D, one more volume) would: the passes
+    // keep neither.  last: the step before in reverse time (-1: none), whose
+    // P~ the pass completes; it < 0: only that.
+    void adj_step(int it, int last, const Fields<T> &fw)
     {
         const Coef<T> c = coef();
-        hipLaunchKernelGGL(gadj_rec<T>, dim3((nrec + 255) / 256), dim3(256), 0, stream, g, a, res + (size_t)it * nrec,
-                           cfg.rec_kind, shot.rec_z, shot.rec_x0, shot.rec_dx, shot.rec_nx, shot.rec_y0,
-                           shot.rec_dy, shot.rec_ny);
-        hipLaunchKernelGGL(gadj_stress_a<T>, grid(), dim3(TZ, TX), 0, stream, g, a, fw, c, tmp[0], tmp[1], tmp[2], grad);
-        hipLaunchKernelGGL(gadj_stress_b<T>, grid(), dim3(TZ, TX), 0, stream, g, a, (const T *)tmp[0],
-                           (const T *)tmp[1], (const T *)tmp[2]);
-        hipLaunchKernelGGL(gadj_vel_a<T>, grid(), dim3(TZ, TX), 0, stream, g, a, c, tmp[0], tmp[1], tmp[2]);
-        hipLaunchKernelGGL(gadj_vel_b<T>, grid(), dim3(TZ, TX), 0, stream, g, a, (const T *)tmp[0],
-                           (const T *)tmp[1], (const T *)tmp[2]);
-        hipLaunchKernelGGL(gsrc_grad<T>, dim3(1), dim3(64), 0, stream, (const T *)a.P, (const T *)a.Q, src_index(),
-                           sgrad + it);
+        hipLaunchKernelGGL(gadj_p<T>, grid(), dim3(TZ, TX), 0, stream, g, a, (const T *)a.P, (const T *)hy, (const T *)a.Q,
+                           fw, c, tmp[0], tmp[1], tmp[2], grad, src_index(), last >= 0 ? sgrad + last : (T *)nullptr,
+                           it >= 0 ? res + (size_t)it * nrec : (T *)nullptr, cfg.rec_kind, shot.rec_z, shot.rec_x0,
+                           shot.rec_dx, shot.rec_nx, shot.rec_y0, shot.rec_dy, shot.rec_ny);
+        if (it < 0) return;
+        hipLaunchKernelGGL(gadj_u<T>, grid(), dim3(TZ, TX), 0, stream, g, a, c, (const T *)tmp[0], (const T *)tmp[1],
+                           (const T *)tmp[2], a.P, hy, a.Q);
+    }
+
+    // The forward sweep with its record as one resident launch (FP32, 2D):
+    // q collects the steps and checkpoints.  1040 x 340, 400 steps: 4.4 ms
+    // step by step, 1.6 so; recomputation runs of ~10 steps between adjoint
+    // steps stay with the per-step kernels (a resident launch costs ~100 us).
+    // 1: q is set up, 0: not available, < 0: error
+    int resident(RtmProgram &q)
+    {
+        if constexpr (sizeof(T) == 4) {
+            if (g.three || cfg.nt < 8 || res2d_state < 0) return 0;
+            Run2dShot b{};
+            b.nnx = g.nnx; b.nnz = g.nnz; b.ldz = g.ldz; b.M = M;
+            T *const fl[8] = {f.u, f.w, f.px, f.pz, f.qx, f.qz, f.P, f.Q};
+            std::copy(fl, fl + 8, b.f);
+            b.vp = vp; b.ep = ep; b.de = de; b.tab = tab;
+            b.dtx = coef().dtx; b.dtz = coef().dtz;
+            b.sv = cfg.sv != 0; b.svR = cfg.sv_R; b.cx = shot.sv_cx; b.cz = shot.sv_cz;
+            b.tap = dtap;
+            b.point = 1; b.sx = shot.sx; b.sz = shot.sz;
+            b.rec = rec; b.nrec = nrec; b.rec_kind = cfg.rec_kind;
+            b.rz = shot.rec_z; b.rx0 = shot.rec_x0; b.rdx = shot.rec_dx; b.rnx = shot.rec_nx;
+            b.split_z = b.rzi = -1;   // no receiver side, no images
+            if (!damp && hipMalloc(&damp, (size_t)cfg.nt * sizeof(float)) != hipSuccess) {
+                (void)hipGetLastError();
+                damp = nullptr;
+                return 0;
+            }
+            b.amp = damp;
+            int e;
+            if (!res2d_state) {
+                int device = 0;
+                if (hipGetDevice(&device) != hipSuccess) return fail(VTI_ERR_HIP, "device");
+                e = run2d_group_make(res2d, run2d_parts({b}, device), {b}, false, cfg.nt, stream);
+                res2d_state = e == 1 ? 1 : -1;
+                if (e < 1) return e;
+            } else if ((e = run2d_group_set(res2d, {b}, stream))) {
+                return e;
+            }
+            if (hipMemcpyAsync(damp, amp.data(), amp.size() * sizeof(float), hipMemcpyHostToDevice, stream) != hipSuccess ||
+                hipStreamSynchronize(stream) != hipSuccess)
+                return fail(VTI_ERR_HIP, "source gains");
+            q.run = [this](const std::vector<Run2dOp> &o, const std::vector<long long> &off) {
+                return run2d_group_run(res2d, o, off, 1, stream);
+            };
+            q.step = [this](bool first, int it) {
+                fwd_step(it, first);
+                return hipGetLastError() == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "launch");
+            };
+            return 1;
+        }
+        return 0;
     }
 
     T *state_base(const Fields<T> &F) const { return F.u; }
@@ -627,8 +662,16 @@ struct Grad : vti_grad {
     {
         if (!have_model || !have_shot) return fail(VTI_ERR_STATE, "vti_grad: model and shot first");
         zero(state_base(f), (size_t)nstate() * nvol);
-        for (int it = 0; it < cfg.nt; ++it) fwd_step(it, true);
-        int st = sync();
+        RtmProgram q;
+        int st = resident(q);
+        if (st < 0) return st;
+        if (st) {
+            for (int it = 0; it < cfg.nt; ++it) q.forward(true, it);
+            if ((st = q.flush()) || (st = run2d_group_check(res2d, stream))) return st;
+        } else {
+            for (int it = 0; it < cfg.nt; ++it) fwd_step(it, true);
+        }
+        st = sync();
         if (st || !d_out) return st;
         return fetch_record(d_out);
     }
@@ -655,10 +698,12 @@ struct Grad : vti_grad {
             if (hipMalloc(&s, (size_t)nstate() * nvol * sizeof(T)) != hipSuccess)
                 return fail(VTI_ERR_ALLOC, "vti_grad: checkpoint slots");
             slots.push_back(s);
+            zero(s, (size_t)nstate() * nvol);   // the border cells, which the resident steps do not store
         }
         zero(state_base(a), (size_t)nstate() * nvol);
         zero(grad, nvol);
         zero(tmp[0], 3 * nvol);
+        if (hy) zero(hy, nvol);
         auto hip_ok = []() { return hipGetLastError() == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "launch"); };
         const size_t sbytes = (size_t)nstate() * nvol * sizeof(T);
         SweepOps op;
@@ -693,18 +738,51 @@ struct Grad : vti_grad {
         };
         // the adjoint reads u, v and w of the forward state, from a slot too;
         // a checkpoint that no step starts from keeps those alone
-        op.consume = [&](int k) { adj_step(k - 1, f); return hip_ok(); };
+        int last = -1;   // step whose adjoint is under way
+        op.consume = [&](int k) { adj_step(k - 1, last, f); last = k - 1; return hip_ok(); };
         op.consume_slot = [&](int k, int i) {
             Fields<T> s{};
             set_fields(s, slots[i], nvol, g.three);
-            adj_step(k - 1, s);
+            adj_step(k - 1, last, s);
+            last = k - 1;
             return hip_ok();
         };
         op.store_light = [&](int i) {   // u, v, w (2D: u, w) lead the state
             return hipMemcpyAsync(slots[i], state_base(f), (g.three ? 3 : 2) * nvol * sizeof(T), hipMemcpyDeviceToDevice,
                                   stream) == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "store");
         };
-        int st = reverse_sweep(nt, nslot, op, steps);
+        RtmProgram q;
+        int st = resident(q);
+        if (st < 0) return st;
+        if (st) {
+            const SweepOps one = op;
+            bool swept = false;
+            auto apart = [this](int i) {
+                return ((long long)reinterpret_cast<intptr_t>(slots[i]) -
+                        (long long)reinterpret_cast<intptr_t>(state_base(f))) / (long long)sizeof(T);
+            };
+            q.move = [&, one](int, long long off) {
+                int i = 0;
+                while (i + 1 < nslot && apart(i) != off) ++i;
+                return one.store(i);
+            };
+            op.first_step = [&](int it) { return q.forward(true, it); };
+            op.store = [&, one](int i) { return swept ? one.store(i) : q.state(3, apart(i)); };
+            op.store_light = [&, one](int i) { return swept ? one.store_light(i) : q.state(3, apart(i)); };
+            op.after_first = [&, one]() {
+                swept = true;
+                int e = q.flush();
+                if (!e) e = run2d_group_check(res2d, stream);
+                return e ? e : one.after_first();
+            };
+            st = reverse_sweep(nt, nslot, op, steps);
+        } else {
+            st = reverse_sweep(nt, nslot, op, steps);
+        }
+        if (!st) {
+            adj_step(-1, last, f);
+            st = hip_ok();
+        }
         if (st || (st = sync())) return st;
         if (misfit) *misfit = J;
         if (grad_src) {

@@ -128,6 +128,42 @@ def test_resident_batch_in_parts_equals_single_shots(unsplit, large):
         assert np.array_equal(got[k][1], ill) and np.array_equal(got[k][0], img), k
 
 
+@pytest.mark.parametrize("nx,nz,npml,nt", [(11, 13, 5, 8), (16, 17, 4, 40), (333, 71, 20, 60), (700, 301, 20, 24),
+                                           (2401, 1003, 20, 9)])
+def test_gradient_with_resident_first_sweep(nx, nz, npml, nt):
+    """FP32 gradients of two shots of one object: the record bit for bit that
+    of the per-step kernels, the gradient the same from any checkpoints
+    (restored ones too) and within FP32 rounding of the FP64 one: 6e-8 times
+    ~50 operations a step, bounded by 1e-4 for at most 60 steps."""
+    rng = np.random.default_rng(2)
+    cfg = vti.cfg_ref2d(vti.MODE_GPU_REF, nx, nz, 10, 10, npml, 1, 20, nt, 1000)
+    vp = (2200.0 + 600.0 * rng.random((nx, nz))).astype(np.float32)
+    ep = (0.2 * rng.random((nx, nz))).astype(np.float32)
+    dl = (0.5 * ep).astype(np.float32)
+    shots = [vti.shot_ref2d(cfg, 1, nx // 2 - k, 0, nz // 2, rec_depth=nz // 2 + 2 * k) for k in range(2)]
+    with vti.Gradient(cfg, fp64=False) as G, vti.Gradient(cfg, fp64=True) as D, vti.Propagator(cfg, vp, ep, dl) as p:
+        for H in (G, D):
+            H.set_model(vp, ep, dl)
+        for shot in shots:
+            p.set_shot(shot)
+            p.reset()
+            for it in range(nt):
+                p.update_vel(it)
+                p.update_stress(it)
+            G.set_shot(shot)
+            D.set_shot(shot)
+            assert np.array_equal(G.forward().astype(np.float32), p.record())
+            r = rng.standard_normal((G.nrec, nt))
+            out = [G.run(resid=r, nsnap=s) for s in (0, 1, 3)]
+            for o in out[1:]:
+                assert np.array_equal(o["grad_vp"], out[0]["grad_vp"])
+                assert np.array_equal(o["grad_src"], out[0]["grad_src"])
+            d = D.run(resid=r, nsnap=3)
+            for k in ("grad_vp", "grad_src"):
+                assert np.abs(d[k]).max() > 0
+                assert np.linalg.norm(out[0][k] - d[k]) <= 1e-4 * np.linalg.norm(d[k]), k
+
+
 def test_resident_steps_of_several_contexts_and_threads():
     """Contexts on streams of their own, stepped from four threads at once."""
     import threading
