@@ -337,12 +337,33 @@ __global__ void copy_kernel(const float4 *__restrict__ src, float4 *__restrict__
 }  // namespace
 
 // ---------------------------------------------------------- launchers ----
-// 3D launches march y in chunks of 16 planes per workgroup (36x more
-// workgroups than whole-column marching at 512^3, so the tail of the
-// launch is short; 8 halo planes of one field re-read per chunk) with
-// non-temporal access to the fields touched once.  Measured at 572^3:
-// chunks of 16 beat 64 by 1 % (stress) and 3 % (velocity).
-constexpr int kYChunk = 16;
+// 3D launches march y in chunks per workgroup: many workgroups, so that the
+// tail of the launch is short and small grids fill the chip; 8 halo planes
+// of one field are read again per chunk, from the caches.  Velocity: 16
+// planes (160^3 .. 572^3: chunks of 8 and 4 are 1 to 3 % slower; 64 3 %).
+// Stress: 4 planes (steps of 104^3: 42 -> 40 us split, 50 -> 38 unsplit;
+// 200^3: 181 -> 175, 165 -> 160; 572^3 0.5 % faster than 16).
+constexpr int kVelChunk = 16, kStressChunk = 4;
+
+// Non-temporal access to what a step touches once keeps the rest in the 256 MB
+// memory-side cache, and loses where all of it would stay there until the
+// next step.  Velocity: u, v, w bypass it unless u, v, w, P and Q together
+// fit (split, us a step, bypassing / not: 184^3, 130 MB 137 / 131; 216^3, 200
+// MB 221 / 216; 232^3, 250 MB 282 / 288; 296^3 636 / 672).  Stress: the model
+// and the split fields unless all that a step touches fits: 14 fields, in the
+// unsplit interior 8 and about a quarter of the 6 split ones (split: 136^3,
+// 140 MB 59 / 50; 168^3, 270 MB 102 / 110; unsplit: 168^3, 200 MB 81 / 72;
+// 184^3, 245 MB 103 / 96; 200^3, 300 MB 137 / 155).  P and Q of the unsplit
+// interior unless the two leave room for the rest of the velocity update
+// (232^3, 110 MB 228 / 200; 264^3, 150 MB 323 / 319; 296^3, 210 MB 443 / 449;
+// 572^3 3.10 / 3.28 ms).
+inline double field_mb(const Grid &g) { return 4e-6 * (double)g.ldxy * g.nny; }
+inline bool stream_vel(const Grid &g) { return 5.0 * field_mb(g) > 224.0; }
+inline int stream_stress(const Grid &g, bool us)
+{
+    if ((us ? 9.5 : 14.0) * field_mb(g) <= 250.0) return 0;
+    return us && 2.0 * field_mb(g) > 160.0 ? 2 : 1;
+}
 
 hipError_t launch_vel(int ndim, const VelArgs &a, hipStream_t s)
 {
@@ -356,8 +377,10 @@ hipError_t launch_vel(int ndim, const VelArgs &a, hipStream_t s)
         else hipLaunchKernelGGL(vel2d_kernel<false>, grd, blk, 0, s, a);
     } else {
         int nzt, nt, ntp;
-        const int grd = s3d::grid3d(a.g, kYChunk, nzt, nt, ntp);
-        hipLaunchKernelGGL((s3d::vel3d<kYChunk, true>), dim3(grd), dim3(s3d::TZ, s3d::TX), 0, s, a, nzt, nt, ntp);
+        const int grd = s3d::grid3d(a.g, kVelChunk, nzt, nt, ntp);
+        const dim3 blk(s3d::TZ, s3d::TX);
+        if (stream_vel(a.g)) hipLaunchKernelGGL((s3d::vel3d<kVelChunk, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+        else hipLaunchKernelGGL((s3d::vel3d<kVelChunk, false>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
     }
     return hipGetLastError();
 }
@@ -374,6 +397,16 @@ hipError_t launch_fused(const FusedArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+template <int NT>
+void stress3d_form(const StressArgs &a, bool us, int grd, int nzt, int nt, int ntp, hipStream_t s)
+{
+    const dim3 blk(s3d::TZ, s3d::TX);
+    if (a.snap && us) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, true, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+    else if (a.snap) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, false, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+    else if (us) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+    else hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+}
+
 hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s)
 {
     if (ndim == 2) {
@@ -384,13 +417,13 @@ hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s)
         else hipLaunchKernelGGL((stress2d_kernel<false, false>), grd, blk, 0, s, a);
     } else {
         int nzt, nt, ntp;
-        const int grd = s3d::grid3d(a.g, kYChunk, nzt, nt, ntp);
-        const dim3 blk(s3d::TZ, s3d::TX);
+        const int grd = s3d::grid3d(a.g, kStressChunk, nzt, nt, ntp);
         const bool us = a.unsplit && !a.gsrc;
-        if (a.snap && us) hipLaunchKernelGGL((s3d::stress3d<kYChunk, true, true, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-        else if (a.snap) hipLaunchKernelGGL((s3d::stress3d<kYChunk, true, false, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-        else if (us) hipLaunchKernelGGL((s3d::stress3d<kYChunk, true, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-        else hipLaunchKernelGGL((s3d::stress3d<kYChunk, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+        switch (stream_stress(a.g, us)) {
+        case 0: stress3d_form<0>(a, us, grd, nzt, nt, ntp, s); break;
+        case 1: stress3d_form<1>(a, us, grd, nzt, nt, ntp, s); break;
+        default: stress3d_form<2>(a, us, grd, nzt, nt, ntp, s);
+        }
     }
     return hipGetLastError();
 }

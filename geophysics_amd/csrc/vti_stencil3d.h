@@ -155,6 +155,8 @@ __global__ __launch_bounds__(256) void vel3d(VelArgs a, int nzt, int ntile, int 
 }
 
 // ------------------------------------------------------------- stress ----
+// NT (launch_stress): 1: the model and the split fields, which a step touches
+// once, bypass the caches; 2: P and Q of the unsplit interior as well.
 // US (reduced split): where every damping factor of the cell is exactly 1
 // (outside the absorbing layer) the split fields are redundant: P and Q are
 // updated directly, P -= (tx + ty + tz), Q likewise, with the same
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(256) void vel3d(VelArgs a, int nzt, int ntile, int 
 // the undamped (tx ..) axes (56 or 72 bytes per cell).  Corners (three damped
 // axes) and row a.split_z keep the full split form.  Point-source
 // (load-time) form only.
-template <int YCHUNK, bool NT, bool US = false, bool SNAP = false>
+template <int YCHUNK, int NT, bool US = false, bool SNAP = false>
 __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile, int ntile_p)
 {
     const Grid g = a.g;
@@ -200,8 +202,8 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
         for (int k = 0; k < 8; ++k) ux[k] = u[id + (long long)(k - 4) * LZ];   // x-4 .. x+3
 #pragma unroll
         for (int k = 0; k < 8; ++k) wz[k] = w[id + (k - 4)];                   // z-4 .. z+3
-        const float vv = ld<NT>(a.vp + id);
-        float ee = ld<NT>(a.ep + id), dd = ld<NT>(a.de + id);
+        const float vv = ld<(NT > 0)>(a.vp + id);
+        float ee = ld<(NT > 0)>(a.ep + id), dd = ld<(NT > 0)>(a.de + id);
         const float ay1 = a.ay1[iy], ay2 = a.ay2[iy];
         const bool dy = !(ay1 == 1.0f && ay2 == 1.0f);
         const bool un = col_int && !dy;
@@ -209,10 +211,10 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
         const bool full = col_full || (dxc && dy && dzc);
         const bool fx = full || dxc, fy = full || dy, fz = full || dzc;
         float opx = 0.0f, opy = 0.0f, opz = 0.0f, oqx = 0.0f, oqy = 0.0f, oqz = 0.0f, oP = 0.0f, oQ = 0.0f;
-        if (fx) { opx = ld<NT>(a.px + id); oqx = ld<NT>(a.qx + id); }
-        if (fy) { opy = ld<NT>(a.py + id); oqy = ld<NT>(a.qy + id); }
-        if (fz) { opz = ld<NT>(a.pz + id); oqz = ld<NT>(a.qz + id); }
-        if (!full) { oP = ld<NT>(a.P + id); oQ = ld<NT>(a.Q + id); }
+        if (fx) { opx = ld<(NT > 0)>(a.px + id); oqx = ld<(NT > 0)>(a.qx + id); }
+        if (fy) { opy = ld<(NT > 0)>(a.py + id); oqy = ld<(NT > 0)>(a.qy + id); }
+        if (fz) { opz = ld<(NT > 0)>(a.pz + id); oqz = ld<(NT > 0)>(a.qz + id); }
+        if (!full) { oP = ld<(NT > 1)>(a.P + id); oQ = ld<(NT > 1)>(a.Q + id); }
         const float vn = iy + 1 < c.y1 ? v[id + 4 * L] : 0.0f;
         compiler_fence();
         float xx = 0.0f, yy = 0.0f, zz = 0.0f;
@@ -237,8 +239,8 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
             const float aa = vv * vv;
             const float Pn = oP - (aa * e2 * dtx * xx + aa * e2 * dty * yy + aa * sd * dtz * zz);
             const float Qn = oQ - (aa * sd * dtx * xx + aa * sd * dty * yy + aa * dtz * zz);
-            st<NT>(a.P + id, Pn);
-            st<NT>(a.Q + id, Qn);
+            st<(NT > 1)>(a.P + id, Pn);
+            st<(NT > 1)>(a.Q + id, Qn);
             illum_add(a, ix, iy, iz, Pn, Qn);
             snap_put<SNAP>(a, ix, iy, iz, Pn);
             if (rk >= 0) {
@@ -256,9 +258,9 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
             const float qx = fx ? ax2 * oqx - ax1 * vv * vv * sd * dtx * xx : 0.0f;
             const float qy = fy ? ay2 * oqy - ay1 * vv * vv * sd * dty * yy : 0.0f;
             const float qz = fz ? az2 * oqz - az1 * vv * vv * dtz * zz : 0.0f;
-            if (fx) { st<NT>(a.px + id, px); st<NT>(a.qx + id, qx); }
-            if (fy) { st<NT>(a.py + id, py); st<NT>(a.qy + id, qy); }
-            if (fz) { st<NT>(a.pz + id, pz); st<NT>(a.qz + id, qz); }
+            if (fx) { st<(NT > 0)>(a.px + id, px); st<(NT > 0)>(a.qx + id, qx); }
+            if (fy) { st<(NT > 0)>(a.py + id, py); st<(NT > 0)>(a.qy + id, qy); }
+            if (fz) { st<(NT > 0)>(a.pz + id, pz); st<(NT > 0)>(a.qz + id, qz); }
             const float rp = ((oP - opx) - opy) - opz;   // unkept components are 0
             const float rq = ((oQ - oqx) - oqy) - oqz;
             const float tp = ((fx ? 0.0f : aa * e2 * dtx * xx) + (fy ? 0.0f : aa * e2 * dty * yy)) +
@@ -267,8 +269,8 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
                              (fz ? 0.0f : aa * dtz * zz);
             const float Pn = ((px + py) + pz) + (rp - tp);
             const float Qn = ((qx + qy) + qz) + (rq - tq);
-            st<NT>(a.P + id, Pn);
-            st<NT>(a.Q + id, Qn);
+            st<(NT > 1)>(a.P + id, Pn);
+            st<(NT > 1)>(a.Q + id, Qn);
             illum_add(a, ix, iy, iz, Pn, Qn);
             snap_put<SNAP>(a, ix, iy, iz, Pn);
             if (rk >= 0) {
@@ -285,8 +287,8 @@ __global__ __launch_bounds__(256) void stress3d(StressArgs a, int nzt, int ntile
             const float qx = ax2 * oqx - ax1 * vv * vv * sd * dtx * xx;
             const float qy = ay2 * oqy - ay1 * vv * vv * sd * dty * yy;
             const float qz = az2 * oqz - az1 * vv * vv * dtz * zz;
-            st<NT>(a.px + id, px); st<NT>(a.py + id, py); st<NT>(a.pz + id, pz);
-            st<NT>(a.qx + id, qx); st<NT>(a.qy + id, qy); st<NT>(a.qz + id, qz);
+            st<(NT > 0)>(a.px + id, px); st<(NT > 0)>(a.py + id, py); st<(NT > 0)>(a.pz + id, pz);
+            st<(NT > 0)>(a.qx + id, qx); st<(NT > 0)>(a.qy + id, qy); st<(NT > 0)>(a.qz + id, qz);
             float Pn = px + py + pz, Qn = qx + qy + qz;
             if (src_col && iy == a.gy) {
                 const float s = (float)((double)a.gamp * a.gw[(ix - a.gx + 3) * 7 + (iz - a.gz + 3)]);
