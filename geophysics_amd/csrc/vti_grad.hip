@@ -87,8 +87,11 @@ struct Coef {
 };
 
 // ---- forward --------------------------------------------------------------
+// keep: floats from u (v, w) to where the new value also goes, 0: nowhere (the
+// checkpoint that the adjoint reads; a copy of its own took 3.2 us and a
+// launch gap a step at 1040 x 340)
 template <typename T>
-__global__ __launch_bounds__(256) void gvel(GGrid g, Fields<T> f, Coef<T> c, long long src, T amp)
+__global__ __launch_bounds__(256) void gvel(GGrid g, Fields<T> f, Coef<T> c, long long src, T amp, long long keep)
 {
     int ix, iy, iz;
     long long id;
@@ -105,9 +108,19 @@ __global__ __launch_bounds__(256) void gvel(GGrid g, Fields<T> f, Coef<T> c, lon
     }
     const T *t = c.tab;
     const int M = c.M;
-    f.u[id] = t[1 * M + ix] * f.u[id] - t[0 * M + ix] * c.dtx * xx;
-    if (g.three) f.v[id] = t[3 * M + iy] * f.v[id] - t[2 * M + iy] * c.dty * yy;
-    f.w[id] = t[5 * M + iz] * f.w[id] - t[4 * M + iz] * c.dtz * zz;
+    const T u = t[1 * M + ix] * f.u[id] - t[0 * M + ix] * c.dtx * xx;
+    const T w = t[5 * M + iz] * f.w[id] - t[4 * M + iz] * c.dtz * zz;
+    f.u[id] = u;
+    f.w[id] = w;
+    if (keep) {
+        f.u[id + keep] = u;
+        f.w[id + keep] = w;
+    }
+    if (g.three) {
+        const T v = t[3 * M + iy] * f.v[id] - t[2 * M + iy] * c.dty * yy;
+        f.v[id] = v;
+        if (keep) f.v[id + keep] = v;
+    }
 }
 
 template <typename T>
@@ -579,11 +592,11 @@ struct Grad : vti_grad {
 
     long long src_index() const { return shot.sz + (long long)shot.sx * g.ldz + (long long)shot.sy * g.ldxy; }
 
-    void fwd_step(int it, bool record)
+    void fwd_step(int it, bool record, long long keep = 0)
     {
         const Coef<T> c = coef();
         const long long src = amp[it] != T(0) ? src_index() : -1;
-        hipLaunchKernelGGL(gvel<T>, grid(), dim3(TZ, TX), 0, stream, g, f, c, src, amp[it]);
+        hipLaunchKernelGGL(gvel<T>, grid(), dim3(TZ, TX), 0, stream, g, f, c, src, amp[it], keep);
         hipLaunchKernelGGL(gstress<T>, grid(), dim3(TZ, TX), 0, stream, g, f, c,
                            record ? rec + (size_t)it * nrec : (T *)nullptr, cfg.rec_kind, shot.rec_z,
                            shot.rec_x0, shot.rec_dx, shot.rec_nx, shot.rec_y0, shot.rec_dy, shot.rec_ny);
@@ -606,7 +619,7 @@ struct Grad : vti_grad {
 
     // The forward sweep with its record as one resident launch (FP32, 2D):
     // q collects the steps and checkpoints.  1040 x 340, 400 steps: 4.4 ms
-    // step by step, 1.6 so; recomputation runs of ~10 steps between adjoint
+    // step by step, 1.7 so; recomputation runs of ~10 steps between adjoint
     // steps stay with the per-step kernels (a resident launch costs ~100 us).
     // 1: q is set up, 0: not available, < 0: error
     int resident(RtmProgram &q)
@@ -706,22 +719,37 @@ struct Grad : vti_grad {
         if (hy) zero(hy, nvol);
         auto hip_ok = []() { return hipGetLastError() == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "launch"); };
         const size_t sbytes = (size_t)nstate() * nvol * sizeof(T);
+        // the sweep's last step waits for what comes next: a checkpoint that
+        // keeps u, v, w alone is written by the step that leads to it (its
+        // border cells are zero, as f's)
+        int next = -1;
+        bool first = false;
+        auto apart = [this](int i) {
+            return ((long long)reinterpret_cast<intptr_t>(slots[i]) -
+                    (long long)reinterpret_cast<intptr_t>(state_base(f))) / (long long)sizeof(T);
+        };
+        auto step_now = [&](long long keep) {
+            if (next >= 0) fwd_step(next, first, keep);
+            next = -1;
+            return hip_ok();
+        };
         SweepOps op;
-        op.zero = [&]() { zero(state_base(f), (size_t)nstate() * nvol); return hip_ok(); };
+        op.zero = [&]() { next = -1; zero(state_base(f), (size_t)nstate() * nvol); return hip_ok(); };
         op.store = [&](int i) {
+            const int e = step_now(0);
+            if (e) return e;
             return hipMemcpyAsync(slots[i], state_base(f), sbytes, hipMemcpyDeviceToDevice, stream) == hipSuccess
                        ? VTI_OK : fail(VTI_ERR_HIP, "store");
         };
         op.restore = [&](int i) {
+            next = -1;
             return hipMemcpyAsync(state_base(f), slots[i], sbytes, hipMemcpyDeviceToDevice, stream) == hipSuccess
                        ? VTI_OK : fail(VTI_ERR_HIP, "restore");
         };
-        op.step = [&](int it) { fwd_step(it, false); return hip_ok(); };
-        op.first_step = [&](int it) { fwd_step(it, true); return hip_ok(); };
         double J = 0;
         op.after_first = [&]() {
-            int st = sync();
-            if (st) return st;
+            int st = step_now(0);
+            if (st || (st = sync())) return st;
             std::vector<T> h((size_t)nrec * nt);
             if (hipMemcpy(h.data(), rec, h.size() * sizeof(T), hipMemcpyDeviceToHost) != hipSuccess)
                 return fail(VTI_ERR_HIP, "record copy");
@@ -739,7 +767,13 @@ struct Grad : vti_grad {
         // the adjoint reads u, v and w of the forward state, from a slot too;
         // a checkpoint that no step starts from keeps those alone
         int last = -1;   // step whose adjoint is under way
-        op.consume = [&](int k) { adj_step(k - 1, last, f); last = k - 1; return hip_ok(); };
+        op.consume = [&](int k) {
+            const int e = step_now(0);
+            if (e) return e;
+            adj_step(k - 1, last, f);
+            last = k - 1;
+            return hip_ok();
+        };
         op.consume_slot = [&](int k, int i) {
             Fields<T> s{};
             set_fields(s, slots[i], nvol, g.three);
@@ -747,20 +781,21 @@ struct Grad : vti_grad {
             last = k - 1;
             return hip_ok();
         };
-        op.store_light = [&](int i) {   // u, v, w (2D: u, w) lead the state
-            return hipMemcpyAsync(slots[i], state_base(f), (g.three ? 3 : 2) * nvol * sizeof(T), hipMemcpyDeviceToDevice,
-                                  stream) == hipSuccess ? VTI_OK : fail(VTI_ERR_HIP, "store");
+        op.store_light = [&](int i) { return step_now(apart(i)); };
+        auto ahead = [&](int it, bool f1) {
+            const int e = step_now(0);
+            next = it;
+            first = f1;
+            return e;
         };
+        op.step = [&](int it) { return ahead(it, false); };
+        op.first_step = [&](int it) { return ahead(it, true); };
         RtmProgram q;
         int st = resident(q);
         if (st < 0) return st;
         if (st) {
             const SweepOps one = op;
             bool swept = false;
-            auto apart = [this](int i) {
-                return ((long long)reinterpret_cast<intptr_t>(slots[i]) -
-                        (long long)reinterpret_cast<intptr_t>(state_base(f))) / (long long)sizeof(T);
-            };
             q.move = [&, one](int, long long off) {
                 int i = 0;
                 while (i + 1 < nslot && apart(i) != off) ++i;
