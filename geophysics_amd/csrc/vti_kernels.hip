@@ -342,8 +342,12 @@ __global__ void copy_kernel(const float4 *__restrict__ src, float4 *__restrict__
 // of one field are read again per chunk, from the caches.  Velocity: 16
 // planes (160^3 .. 572^3: chunks of 8 and 4 are 1 to 3 % slower; 64 3 %).
 // Stress: 4 planes (steps of 104^3: 42 -> 40 us split, 50 -> 38 unsplit;
-// 200^3: 181 -> 175, 165 -> 160; 572^3 0.5 % faster than 16).
-constexpr int kVelChunk = 16, kStressChunk = 4;
+// 200^3: 181 -> 175, 165 -> 160; 400^3 1577 -> 1553; unsplit 552^3 2840 -> 2800
+// and no slower up to 680^3).  The split update of the largest grids streams
+// so much between a chunk and the next that the halo planes leave the
+// memory-side cache: 16 planes (chunks of 4 / 16: 480^3, 442 MB a field 2645
+// / 2679 us; 520^3, 560 MB 3508 / 3479; 552^3 4135 / 4060).
+constexpr int kVelChunk = 16, kStressChunk = 4, kSplitChunk = 16;
 
 // Non-temporal access to what a step touches once keeps the rest in the 256 MB
 // memory-side cache, and loses where all of it would stay there until the
@@ -397,14 +401,15 @@ hipError_t launch_fused(const FusedArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-template <int NT>
-void stress3d_form(const StressArgs &a, bool us, int grd, int nzt, int nt, int ntp, hipStream_t s)
+template <int CH, int NT>
+void stress3d_form(const StressArgs &a, bool us, hipStream_t s)
 {
-    const dim3 blk(s3d::TZ, s3d::TX);
-    if (a.snap && us) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, true, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-    else if (a.snap) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, false, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-    else if (us) hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT, true>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
-    else hipLaunchKernelGGL((s3d::stress3d<kStressChunk, NT>), dim3(grd), blk, 0, s, a, nzt, nt, ntp);
+    int nzt, nt, ntp;
+    const dim3 grd(s3d::grid3d(a.g, CH, nzt, nt, ntp)), blk(s3d::TZ, s3d::TX);
+    if (a.snap && us) hipLaunchKernelGGL((s3d::stress3d<CH, NT, true, true>), grd, blk, 0, s, a, nzt, nt, ntp);
+    else if (a.snap) hipLaunchKernelGGL((s3d::stress3d<CH, NT, false, true>), grd, blk, 0, s, a, nzt, nt, ntp);
+    else if (us) hipLaunchKernelGGL((s3d::stress3d<CH, NT, true>), grd, blk, 0, s, a, nzt, nt, ntp);
+    else hipLaunchKernelGGL((s3d::stress3d<CH, NT>), grd, blk, 0, s, a, nzt, nt, ntp);
 }
 
 hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s)
@@ -416,13 +421,14 @@ hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s)
         else if (a.unsplit && !a.gsrc) hipLaunchKernelGGL((stress2d_kernel<true, false>), grd, blk, 0, s, a);
         else hipLaunchKernelGGL((stress2d_kernel<false, false>), grd, blk, 0, s, a);
     } else {
-        int nzt, nt, ntp;
-        const int grd = s3d::grid3d(a.g, kStressChunk, nzt, nt, ntp);
         const bool us = a.unsplit && !a.gsrc;
         switch (stream_stress(a.g, us)) {
-        case 0: stress3d_form<0>(a, us, grd, nzt, nt, ntp, s); break;
-        case 1: stress3d_form<1>(a, us, grd, nzt, nt, ntp, s); break;
-        default: stress3d_form<2>(a, us, grd, nzt, nt, ntp, s);
+        case 0: stress3d_form<kStressChunk, 0>(a, us, s); break;
+        case 1:
+            if (us || field_mb(a.g) <= 500.0) stress3d_form<kStressChunk, 1>(a, us, s);
+            else stress3d_form<kSplitChunk, 1>(a, us, s);
+            break;
+        default: stress3d_form<kStressChunk, 2>(a, us, s);
         }
     }
     return hipGetLastError();
