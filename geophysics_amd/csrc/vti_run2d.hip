@@ -978,6 +978,8 @@ bool capturing(hipStream_t s)
     return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
+thread_local long long t_launches = 0;   // vti_resident_launches
+
 bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     void *args[] = {&a};
@@ -988,6 +990,7 @@ bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStre
         (void)hipGetLastError();
         return false;
     }
+    ++t_launches;
     return true;
 }
 
@@ -1315,3 +1318,5 @@ int RtmProgram::flush()
 }
 
 }  // namespace vti
+
+extern "C" long long vti_resident_launches(void) { return vti::t_launches; }

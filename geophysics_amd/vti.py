@@ -95,6 +95,7 @@ def _declare(L):
         "vti_update_vel": (C.c_int, [VP, C.c_int]),
         "vti_update_stress": (C.c_int, [VP, C.c_int]),
         "vti_step": (C.c_int, [VP, C.c_int, C.c_int]),
+        "vti_resident_launches": (C.c_longlong, []),
         "vti_run": (C.c_int, [VP]),
         "vti_nrec": (C.c_int, [VP]),
         "vti_mute": (C.c_int, [VP] + [C.c_int] * 5),
@@ -255,6 +256,11 @@ def sweep_check(nt, nslot):
     steps, slots = C.c_longlong(), C.c_int()
     check(lib().vti_sweep_check(nt, nslot, C.byref(steps), C.byref(slots)), "sweep_check")
     return steps.value, slots.value
+
+
+def resident_launches():
+    """Launches of the resident 2D kernel that this thread's calls have made."""
+    return lib().vti_resident_launches()
 
 
 def learned_defaults():

@@ -158,6 +158,11 @@ int vti_update_vel(vti_ctx *ctx, int it);
 int vti_update_stress(vti_ctx *ctx, int it);
 /* nsteps full steps starting at it0. */
 int vti_step(vti_ctx *ctx, int it0, int nsteps);
+/* Launches of the resident 2D kernel (many steps in one launch: vti_step /
+ * vti_run of 8 steps or more, vti_rtm_shot, vti_batch_rtm, vti_grad_*) that
+ * calls of this thread have made so far; where it does not apply or cannot be
+ * launched, the per-step kernels run and the count stays. */
+long long vti_resident_launches(void);
 /* reset + all nt steps. */
 int vti_run(vti_ctx *ctx);
 
