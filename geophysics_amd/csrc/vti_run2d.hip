@@ -793,6 +793,8 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
 }
 
 // ---- host side --------------------------------------------------------------
+constexpr size_t kStaticLds = 64;   // s_dead, rounded up
+
 using KernelFn = void (*)(Run2dArgs);
 // Launch shapes: threads, rows a strip.
 struct Shape2d {
@@ -844,7 +846,7 @@ void cuts_of(int nnx, int nnz, bool tti, int shape, int cus, int lds_max, std::v
             const int nz = 4 * ((uq + gz - 1) / gz);
             const int strips = rows * nz;
             const size_t b = 4 * (size_t)(tti ? Lds<true>(nx, nz).total : Lds<false>(nx, nz).total);
-            if (b + 64 > (size_t)lds_max) continue;
+            if (b + kStaticLds > (size_t)lds_max) continue;
             const int us = (nx + 7 + nu - 1) / nu * (tti ? nz + 8 : nz), ws = tti ? 0 : rows * (nz + 8);
             const double f = tti ? 2.0 : 1.0;
             const double issue = f * nu * (20.0 * us + 26.0 * ws + 50.0 * strips) / 64.0;
@@ -983,8 +985,17 @@ thread_local long long t_launches = 0;   // vti_resident_launches
 bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     void *args[] = {&a};
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-            hipSuccess ||
+    // The function's own limit, which its callers in all threads share: always
+    // the same value, what a workgroup can have, never this launch's need.
+    static const int lds_max = [] {
+        int device = 0, n = 0;
+        if (hipGetDevice(&device) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
+            (void)hipGetLastError();
+        return n;
+    }();
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            std::max((int)lds, lds_max - (int)kStaticLds)) != hipSuccess ||
         hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s) !=
             hipSuccess) {
         (void)hipGetLastError();

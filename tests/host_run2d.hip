@@ -1,0 +1,140 @@
+// The host side of the resident 2D steps (vti_run2d.hip) over a runtime that
+// is made up here: allocations are host memory, launches are only recorded and
+// refused as the scenario asks.  No device is touched and no kernel runs.
+// test_host_run2d.py builds it with the device passes left out and runs one
+// scenario (argv[1]) a time; a failed condition names itself and ends it.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+
+#include "../geophysics_amd/csrc/vti_run2d.hip"
+
+#define CHECK(x)                                        \
+    do {                                                \
+        if (!(x)) {                                     \
+            std::printf("line %d: %s\n", __LINE__, #x); \
+            std::exit(1);                               \
+        }                                               \
+    } while (0)
+
+// ---- the runtime ------------------------------------------------------------
+struct Launched {
+    const void *kernel;
+    int grid, block;
+    size_t lds;
+};
+static std::vector<Launched> g_launched;
+static std::map<const void *, int> g_lds_max;       // the attribute of each function
+static std::function<void()> g_after_attribute;     // what another thread does after this one's set
+static int g_cus = 256, g_lds = 163840;
+
+extern "C" {
+char __hip_fatbin[64];
+void **__hipRegisterFatBinary(const void *) { return nullptr; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipFree(void *p)
+{
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
+{
+    *c = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d)
+{
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int)
+{
+    *v = a == hipDeviceAttributeMultiprocessorCount ? g_cus : (a == hipDeviceAttributeMaxSharedMemoryPerBlock ? g_lds : 1);
+    return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v)
+{
+    g_lds_max[f] = v;
+    std::function<void()> other;
+    other.swap(g_after_attribute);
+    if (other) other();
+    return hipSuccess;
+}
+hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3 b, void **, unsigned lds, hipStream_t)
+{
+    if (!g_lds_max.count(f) || (int)lds > g_lds_max[f] || (int)lds > g_lds) return hipErrorInvalidValue;
+    if ((int)g.x > g_cus) return hipErrorCooperativeLaunchTooLarge;
+    g_launched.push_back({f, (int)g.x, (int)b.x, lds});
+    return hipSuccess;
+}
+}
+
+namespace vti {
+int fail(int code, const std::string &) { return code; }
+hipError_t launch_zero(float *p, size_t n, hipStream_t)
+{
+    std::memset(p, 0, n * sizeof(float));
+    return hipSuccess;
+}
+VtiState main_state(vti_ctx *c)
+{
+    VtiState s;
+    for (int k = 0; k < 11; ++k) s.f[k] = c->f[k];
+    return s;
+}
+
+// ---- scenarios --------------------------------------------------------------
+struct Ctx : vti_ctx {   // a 2D context, its padded size
+    Ctx(int nnx, int nnz)
+    {
+        cfg.ndim = 2;
+        cfg.mode = VTI_MODE_GPU_REF;
+        cfg.dt = 1e-3f;
+        cfg.dx = cfg.dy = cfg.dz = 10.0f;
+        g = Grid{nnx, 1, nnz, (nnz + 31) / 32 * 32, 0};
+        g.ldxy = (long long)g.ldz * nnx;
+        nvol = (size_t)g.ldxy;
+        nnmax = std::max(nnx, nnz);
+    }
+    ~Ctx() { run2d_free(this); }
+};
+
+// Two threads whose tiles of one kernel need different amounts of LDS: the
+// smaller one's launch comes between the larger one's attribute and launch.
+void lds_attribute()
+{
+    Ctx large(1440, 543), small(1340, 543);
+    int r = -1;
+    g_after_attribute = [&] { r = run2d_steps(&small, 0, 16); };
+    const int q = run2d_steps(&large, 0, 16);
+    CHECK(r == 1 && g_launched.size() >= 1);
+    CHECK(q == 1 && g_launched.size() == 2);
+    CHECK(g_launched[0].kernel == g_launched[1].kernel && g_launched[0].lds < g_launched[1].lds);
+}
+
+}  // namespace vti
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}};
+    const auto s = all.find(argc > 1 ? argv[1] : "");
+    CHECK(s != all.end());
+    s->second();
+    std::printf("ok\n");
+    return 0;
+}

@@ -127,7 +127,7 @@ def test_threads_of_one_launch_shape():
     """Four threads whose grids share a launch shape (threads and rows a strip)
     and need different amounts of LDS: every call is a resident launch, and the
     fields are those of each context alone."""
-    sizes = [(1401, 503), (1300, 480), (1200, 500), (1350, 450)]
+    sizes = [(1400, 503), (1300, 503), (1150, 503), (1400, 503)]
     alone, got, count = {}, {}, {}
 
     def work(k, into):
