@@ -982,7 +982,7 @@ bool capturing(hipStream_t s)
 
 thread_local long long t_launches = 0;   // vti_resident_launches
 
-bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
+hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     void *args[] = {&a};
     // The function's own limit, which its callers in all threads share: always
@@ -994,15 +994,13 @@ bool launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStre
             (void)hipGetLastError();
         return n;
     }();
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            std::max((int)lds, lds_max - (int)kStaticLds)) != hipSuccess ||
-        hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    ++t_launches;
-    return true;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       std::max((int)lds, lds_max - (int)kStaticLds));
+    if (e == hipSuccess)
+        e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s);
+    if (e != hipSuccess) (void)hipGetLastError();
+    else ++t_launches;
+    return e;
 }
 
 }  // namespace
@@ -1100,8 +1098,11 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     const bool us = c->unsplit && c->cfg.mode == VTI_MODE_GPU_REF && !tti;
     const KernelFn k = tti ? kernel_of<true, false, false>(p.shape)
                            : (us ? kernel_of<false, true, false>(p.shape) : kernel_of<false, false, false>(p.shape));
-    if (!launch_coop(k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream)) {
-        p.ok = -1;
+    const hipError_t e = launch_coop(k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream);
+    if (e != hipSuccess) {
+        // a launch that the device cannot hold never will be; another cause
+        // (scratch or queue memory) may be gone at the next call
+        if (e == hipErrorCooperativeLaunchTooLarge) p.ok = -1;
         return 0;
     }
     p.base += (unsigned)n;
@@ -1253,7 +1254,7 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         a.base = g.base;
         a.dead = g.dead;
         const KernelFn k = g.us ? kernel_of<false, true, true>(q.shape) : kernel_of<false, false, true>(q.shape);
-        if (!launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s)) return unavailable(g);
+        if (launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s) != hipSuccess) return unavailable(g);
         g.ran = true;
         g.base += (unsigned)(offs.size() + 2);   // one exchange a step
     }

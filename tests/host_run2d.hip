@@ -28,6 +28,7 @@ struct Launched {
 static std::vector<Launched> g_launched;
 static std::map<const void *, int> g_lds_max;       // the attribute of each function
 static std::function<void()> g_after_attribute;     // what another thread does after this one's set
+static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
 static int g_cus = 256, g_lds = 163840;
 
 extern "C" {
@@ -77,6 +78,11 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v)
 }
 hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3 b, void **, unsigned lds, hipStream_t)
 {
+    if (!g_refuse.empty()) {
+        const hipError_t e = g_refuse.front();
+        g_refuse.erase(g_refuse.begin());
+        if (e != hipSuccess) return e;
+    }
     if (!g_lds_max.count(f) || (int)lds > g_lds_max[f] || (int)lds > g_lds) return hipErrorInvalidValue;
     if ((int)g.x > g_cus) return hipErrorCooperativeLaunchTooLarge;
     g_launched.push_back({f, (int)g.x, (int)b.x, lds});
@@ -127,11 +133,24 @@ void lds_attribute()
     CHECK(g_launched[0].kernel == g_launched[1].kernel && g_launched[0].lds < g_launched[1].lds);
 }
 
+// A refused launch leaves that call to the per-step kernels and no later one,
+// unless the device can never hold it.
+void refused_step()
+{
+    Ctx c(440, 440);
+    g_refuse = {hipErrorOutOfMemory};
+    CHECK(run2d_steps(&c, 0, 16) == 0);
+    CHECK(run2d_steps(&c, 16, 16) == 1 && g_launched.size() == 1);
+    g_refuse = {hipErrorCooperativeLaunchTooLarge};
+    CHECK(run2d_steps(&c, 0, 16) == 0);
+    CHECK(run2d_steps(&c, 16, 16) == 0 && g_launched.size() == 1);
+}
+
 }  // namespace vti
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}};
+    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step}};
     const auto s = all.find(argc > 1 ? argv[1] : "");
     CHECK(s != all.end());
     s->second();
