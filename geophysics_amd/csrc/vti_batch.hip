@@ -781,32 +781,17 @@ int vti_batch_autotune(vti_batch *B, int steps, double *best_ms)
     return hipStreamSynchronize(B->stream) == hipSuccess ? bs : bfail(VTI_ERR_HIP, "sync");
 }
 
-// RTM of every shot of the batch in lockstep.  obs: per-shot observed
-// records [irec][it] (host), or NULL to migrate the modelled records.
-int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, long long *fwd_steps)
+}  // extern "C"
+
+namespace {
+
+// One pass over the schedule.  resident: with the resident kernel where the
+// shots fit; a launch refused when shots have moved on without it (refused is
+// set then) ends the pass.
+int rtm_pass(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, int nslot, long long *fwd_steps, bool resident,
+             bool &refused)
 {
-    if (!B || !o || o->image_every < 1 || o->nsnap < 0 || o->illum_mode != 0)
-        return bfail(VTI_ERR_ARG, "vti_batch_rtm: bad arguments (the batch images with source illumination, illum_mode 0)");
     const int nt = B->nt;
-    // the taper switches and the imaging interval hold for this call only:
-    // vti_batch_forward keeps the batch's own (SV taper on in the forward
-    // propagation); illum_mode stays, vti_batch_image reads it
-    struct Restore {
-        vti_batch *B;
-        int sf, sb, ie;
-        ~Restore() { B->sv_fwd = sf; B->sv_bwd = sb; B->image_every = ie; }
-    } restore{B, B->sv_fwd, B->sv_bwd, B->image_every};
-    B->image_every = o->image_every;
-    B->illum_mode = o->illum_mode;
-    B->sv_fwd = o->sv_forward;
-    B->sv_bwd = o->sv_backward;
-    const int nslot = std::max(0, o->nsnap > 0 ? std::min(o->nsnap, nt - 1) : nt - 1);
-    while ((int)B->slots.size() < nslot) {
-        float *p = nullptr;
-        if (hipMalloc(&p, B->state_floats * sizeof(float)) != hipSuccess)
-            return bfail(VTI_ERR_ALLOC, "vti_batch_rtm: checkpoint slots");
-        B->slots.push_back(p);
-    }
     // zero receiver states, images, illuminations
     zero_floats(B, B->rstate_base, B->state_floats);
     for (auto &b : B->hb) {
@@ -912,7 +897,7 @@ int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, 
         ~GroupGuard() { run2d_group_free(g); }
     } group_guard{grp};
     RtmProgram q;
-    bool inside = nt >= 8;
+    bool inside = resident && nt >= 8;
     for (const vti_cfg &c : B->cfgs) inside = inside && c.npml >= 4;
     if (inside) {
         std::vector<Run2dShot> shots;
@@ -939,7 +924,9 @@ int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, 
         };
         const SweepOps one = op;
         q.run = [&](const std::vector<Run2dOp> &ops, const std::vector<long long> &offs) {
-            return run2d_group_run(grp, ops, offs, o->image_every, B->stream);
+            const int r = run2d_group_run(grp, ops, offs, o->image_every, B->stream);
+            refused = r == 2 || (r == 0 && grp.ran);
+            return refused ? VTI_ERR_HIP : r;
         };
         q.step = [one](bool first, int it) { return first ? one.first_step(it) : one.step(it); };
         q.keep = [one, slot_of](long long off) { return one.store_light(slot_of(off)); };
@@ -973,6 +960,42 @@ int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, 
     if (st) return st;
     if (hipStreamSynchronize(B->stream) != hipSuccess) return fail(VTI_ERR_HIP, "sync");
     return run2d_group_check(grp, B->stream);
+}
+
+}  // namespace
+
+extern "C" {
+
+// RTM of every shot of the batch in lockstep.  obs: per-shot observed
+// records [irec][it] (host), or NULL to migrate the modelled records.
+int vti_batch_rtm(vti_batch *B, const vti_rtm_opts *o, const float *const *obs, long long *fwd_steps)
+{
+    if (!B || !o || o->image_every < 1 || o->nsnap < 0 || o->illum_mode != 0)
+        return bfail(VTI_ERR_ARG, "vti_batch_rtm: bad arguments (the batch images with source illumination, illum_mode 0)");
+    const int nt = B->nt;
+    // the taper switches and the imaging interval hold for this call only:
+    // vti_batch_forward keeps the batch's own (SV taper on in the forward
+    // propagation); illum_mode stays, vti_batch_image reads it
+    struct Restore {
+        vti_batch *B;
+        int sf, sb, ie;
+        ~Restore() { B->sv_fwd = sf; B->sv_bwd = sb; B->image_every = ie; }
+    } restore{B, B->sv_fwd, B->sv_bwd, B->image_every};
+    B->image_every = o->image_every;
+    B->illum_mode = o->illum_mode;
+    B->sv_fwd = o->sv_forward;
+    B->sv_bwd = o->sv_backward;
+    const int nslot = std::max(0, o->nsnap > 0 ? std::min(o->nsnap, nt - 1) : nt - 1);
+    while ((int)B->slots.size() < nslot) {
+        float *p = nullptr;
+        if (hipMalloc(&p, B->state_floats * sizeof(float)) != hipSuccess)
+            return bfail(VTI_ERR_ALLOC, "vti_batch_rtm: checkpoint slots");
+        B->slots.push_back(p);
+    }
+    bool refused = false;
+    const int st = rtm_pass(B, o, obs, nslot, fwd_steps, true, refused);
+    // from the start on the per-step kernels: a pass sets all that it reads
+    return refused ? rtm_pass(B, o, obs, nslot, fwd_steps, false, refused) : st;
 }
 
 int vti_batch_image(vti_batch *B, int shot, int finalize, float *img, float *illum)

@@ -316,6 +316,19 @@ hipError_t ck_copy(vti_ctx *c, const CkSlots &k, int i, const VtiState &W, bool 
     return hipGetLastError();
 }
 
+// The cells of a 2D state that no step changes (four around the grid, and the
+// pitch): zero, as from the start.
+__global__ void border_zero_kernel(Grid g, VtiState p)
+{
+    const int ix = blockIdx.x;
+    const bool row = ix < 4 || ix >= g.nnx - 4;
+    for (int k = 0; k < 11; ++k) {
+        if (!p.f[k]) continue;
+        for (int iz = threadIdx.x; iz < g.ldz; iz += blockDim.x)
+            if (row || iz < 4 || iz >= g.nnz - 4) p.f[k][(long long)ix * g.ldz + iz] = 0.0f;
+    }
+}
+
 struct RtmCache {
     VtiState g;                  // receiver wavefield
     CkSlots ck;                  // checkpoints of the source state
@@ -513,7 +526,12 @@ int vti_rtm_shot(vti_ctx *c, const vti_rtm_opts *o, const float *obs, long long 
         };
         q.receive = [&, at](int it, long long off) { return consume_from(at(off), it + 1); };
         q.move = [&, one, slot_of](int kind, long long slot) {
-            return kind == 5 ? one.zero() : (kind == 3 ? one.store(slot_of(slot)) : one.restore(slot_of(slot)));
+            if (kind != 4) return kind == 5 ? one.zero() : one.store(slot_of(slot));
+            const int e = one.restore(slot_of(slot));
+            if (e) return e;
+            // a resident launch leaves them out of its checkpoints
+            hipLaunchKernelGGL(border_zero_kernel, dim3(c->g.nnx), dim3(256), 0, c->stream, c->g, W);
+            return hip(hipGetLastError(), "restore");
         };
         op.zero = [&]() { return q.state(5, 0); };
         op.after_first = [&, one]() { const int e = q.flush(); return e ? e : one.after_first(); };

@@ -70,6 +70,7 @@ struct Run2dParts {
 
 struct Run2dGroup {
     int ok = 0;                 // 1: usable
+    bool refused = false;       // a launch was refused: no further one until run2d_group_set
     bool ran = false;           // a program has run
     bool us = false;
     Run2dParts parts;
@@ -87,7 +88,10 @@ int run2d_group_make(Run2dGroup &g, const Run2dParts &p, std::vector<Run2dShot> 
 // other shots on the same grids (their pointers, source and receivers)
 int run2d_group_set(Run2dGroup &g, std::vector<Run2dShot> shots, hipStream_t s);
 void run2d_group_free(Run2dGroup &g);
-// the program on every part; 1: launched, 0: not available, < 0: error
+// the program on every part; 1: launched, 0: not available, nothing launched
+// (the states lie where the programs before it left them; their checkpoints
+// have no border cells), 2: refused after some of the parts have run it, < 0:
+// error
 int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::vector<long long> &offs, int image_every,
                     hipStream_t s);
 // waits for the stream

@@ -981,9 +981,11 @@ bool capturing(hipStream_t s)
 }
 
 thread_local long long t_launches = 0;   // vti_resident_launches
+thread_local long long t_left = -1;      // vti_resident_limit
 
 hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
+    if (t_left == 0) return hipErrorOutOfMemory;
     void *args[] = {&a};
     // The function's own limit, which its callers in all threads share: always
     // the same value, what a workgroup can have, never this launch's need.
@@ -998,8 +1000,12 @@ hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, h
                                        std::max((int)lds, lds_max - (int)kStaticLds));
     if (e == hipSuccess)
         e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s);
-    if (e != hipSuccess) (void)hipGetLastError();
-    else ++t_launches;
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return e;
+    }
+    ++t_launches;
+    if (t_left > 0) --t_left;
     return e;
 }
 
@@ -1192,6 +1198,7 @@ int run2d_group_make(Run2dGroup &g, const Run2dParts &p, std::vector<Run2dShot> 
 
 int run2d_group_set(Run2dGroup &g, std::vector<Run2dShot> shots, hipStream_t s)
 {
+    g.refused = false;
     const Run2dParts &p = g.parts;
     for (size_t k = 0; k < shots.size(); ++k) {
         shots[k].gx = p.gx[k];
@@ -1212,19 +1219,11 @@ void run2d_group_free(Run2dGroup &g)
     g = Run2dGroup{};
 }
 
-// The per-step kernels can start a schedule but not go on with one: the
-// checkpoints that a launch wrote have no border cells.
-static int unavailable(Run2dGroup &g)
-{
-    g.ok = -1;
-    return g.ran ? fail(VTI_ERR_HIP, "run2d: launch") : 0;
-}
-
 // prog: the operations, then the offsets
 int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::vector<long long> &offs, int image_every,
                     hipStream_t s)
 {
-    if (g.ok != 1) return 0;
+    if (g.ok != 1 || g.refused) return 0;
     const size_t nb = ops.size() * sizeof(Run2dOp), need = nb + std::max<size_t>(offs.size(), 1) * sizeof(long long);
     if (need > g.prog_bytes) {
         if (hipStreamSynchronize(s) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
@@ -1232,7 +1231,10 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         g.more = nullptr;
         if (hipMalloc(&g.more, 2 * need) != hipSuccess) {
             (void)hipGetLastError();
-            return unavailable(g);
+            g.more = nullptr;
+            g.prog_bytes = 0;
+            g.refused = true;
+            return 0;
         }
         g.prog = g.more;
         g.prog_bytes = 2 * need;
@@ -1254,7 +1256,12 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         a.base = g.base;
         a.dead = g.dead;
         const KernelFn k = g.us ? kernel_of<false, true, true>(q.shape) : kernel_of<false, false, true>(q.shape);
-        if (launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s) != hipSuccess) return unavailable(g);
+        const hipError_t e = launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s);
+        if (e != hipSuccess) {
+            g.refused = true;
+            if (e == hipErrorCooperativeLaunchTooLarge) g.ok = -1;
+            return &q == &g.parts.part.front() ? 0 : 2;
+        }
         g.ran = true;
         g.base += (unsigned)(offs.size() + 2);   // one exchange a step
     }
@@ -1332,3 +1339,5 @@ int RtmProgram::flush()
 }  // namespace vti
 
 extern "C" long long vti_resident_launches(void) { return vti::t_launches; }
+
+extern "C" void vti_resident_limit(long long n) { vti::t_left = n < 0 ? -1 : n; }

@@ -96,6 +96,7 @@ def _declare(L):
         "vti_update_stress": (C.c_int, [VP, C.c_int]),
         "vti_step": (C.c_int, [VP, C.c_int, C.c_int]),
         "vti_resident_launches": (C.c_longlong, []),
+        "vti_resident_limit": (None, [C.c_longlong]),
         "vti_run": (C.c_int, [VP]),
         "vti_nrec": (C.c_int, [VP]),
         "vti_mute": (C.c_int, [VP] + [C.c_int] * 5),
@@ -261,6 +262,11 @@ def sweep_check(nt, nslot):
 def resident_launches():
     """Launches of the resident 2D kernel that this thread's calls have made."""
     return lib().vti_resident_launches()
+
+
+def resident_limit(n):
+    """At most n further resident launches by this thread (None: no limit)."""
+    lib().vti_resident_limit(-1 if n is None else n)
 
 
 def learned_defaults():

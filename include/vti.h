@@ -163,6 +163,10 @@ int vti_step(vti_ctx *ctx, int it0, int nsteps);
  * calls of this thread have made so far; where it does not apply or cannot be
  * launched, the per-step kernels run and the count stays. */
 long long vti_resident_launches(void);
+/* At most n further ones (n < 0, the default: no limit): a launch above that
+ * is refused as the runtime may refuse any, and the call goes on with the
+ * per-step kernels, from the middle of an RTM's schedule too. */
+void vti_resident_limit(long long n);
 /* reset + all nt steps. */
 int vti_run(vti_ctx *ctx);
 

@@ -29,6 +29,7 @@ static std::vector<Launched> g_launched;
 static std::map<const void *, int> g_lds_max;       // the attribute of each function
 static std::function<void()> g_after_attribute;     // what another thread does after this one's set
 static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
+static bool g_no_memory = false;
 static int g_cus = 256, g_lds = 163840;
 
 extern "C" {
@@ -39,7 +40,7 @@ void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipMalloc(void **p, size_t n) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipMalloc(void **p, size_t n) { return !g_no_memory && (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipFree(void *p)
 {
     std::free(p);
@@ -146,11 +147,52 @@ void refused_step()
     CHECK(run2d_steps(&c, 16, 16) == 0 && g_launched.size() == 1);
 }
 
+struct Group : Run2dGroup {   // shots of two parts
+    std::vector<Run2dShot> shots;
+    std::vector<Run2dOp> ops{Run2dOp{1, 0, 8, 1, 0, 0, 0}};
+    std::vector<long long> offs = std::vector<long long>(8, 0);
+    Group()
+    {
+        for (int nnx : {2441, 2401}) {
+            Run2dShot b{};
+            b.nnx = b.M = nnx;
+            b.nnz = 543;
+            b.ldz = 544;
+            shots.push_back(b);
+        }
+        CHECK(run2d_group_make(*this, run2d_parts(shots, 0), shots, false, 8, nullptr) == 1);
+        CHECK(parts.part.size() == 2);
+    }
+    ~Group() { run2d_group_free(*this); }
+    int run() { return run2d_group_run(*this, ops, offs, 1, nullptr); }
+};
+
+// A program refused before its first part has run nothing, one refused later
+// has; both leave the group alone until the next set of shots.
+void refused_program()
+{
+    Group g;
+    CHECK(g.run() == 1 && g_launched.size() == 2);
+    g_refuse = {hipErrorOutOfMemory};
+    CHECK(g.run() == 0 && g.run() == 0 && g_launched.size() == 2);
+    CHECK(run2d_group_set(g, g.shots, nullptr) == VTI_OK && g.run() == 1 && g_launched.size() == 4);
+    g_refuse = {hipSuccess, hipErrorOutOfMemory};
+    CHECK(g.run() == 2 && g.run() == 0 && g_launched.size() == 5);
+    g.offs.resize(1 << 16);   // a program larger than the group's share of memory, and none to be had
+    g.ops[0].n = 1 << 16;
+    CHECK(run2d_group_set(g, g.shots, nullptr) == VTI_OK);
+    g_no_memory = true;
+    CHECK(g.run() == 0 && g.run() == 0 && g_launched.size() == 5);
+    g_no_memory = false;
+    CHECK(run2d_group_set(g, g.shots, nullptr) == VTI_OK && g.run() == 1 && g_launched.size() == 7);
+}
+
 }  // namespace vti
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step}};
+    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step},
+                                                       {"refused_program", vti::refused_program}};
     const auto s = all.find(argc > 1 ? argv[1] : "");
     CHECK(s != all.end());
     s->second();
