@@ -71,7 +71,7 @@ struct Run2dParts {
 struct Run2dGroup {
     int ok = 0;                 // 1: usable
     bool refused = false;       // a launch was refused: no further one until run2d_group_set
-    bool ran = false;           // a program has run
+    bool ran = false;           // a program has run since the last check
     bool us = false;
     Run2dParts parts;
     void *mem = nullptr, *more = nullptr;   // more: a program larger than mem's share
@@ -94,7 +94,7 @@ void run2d_group_free(Run2dGroup &g);
 // error
 int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::vector<long long> &offs, int image_every,
                     hipStream_t s);
-// waits for the stream
+// waits for the stream; reports an exchange that never came, once
 int run2d_group_check(Run2dGroup &g, hipStream_t s);
 
 // Collects the operations that an RTM's schedule asks for one by one, so that

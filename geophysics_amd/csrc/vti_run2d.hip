@@ -1271,10 +1271,12 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
 int run2d_group_check(Run2dGroup &g, hipStream_t s)
 {
     if (!g.ran) return VTI_OK;
+    g.ran = false;
     int dead = 0;
     if (hipMemcpyAsync(&dead, g.dead, sizeof dead, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return fail(VTI_ERR_HIP, "run2d: check");
+    if (dead && launch_zero(reinterpret_cast<float *>(g.dead), 1, s) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: check");
     return dead_check(&dead, g.ok);
 }
 

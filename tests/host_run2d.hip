@@ -187,12 +187,26 @@ void refused_program()
     CHECK(run2d_group_set(g, g.shots, nullptr) == VTI_OK && g.run() == 1 && g_launched.size() == 7);
 }
 
+// An exchange that never came is reported once, by the check after the program
+// that missed it; the object then keeps the per-step kernels.
+void missed_exchange()
+{
+    Group g;
+    CHECK(g.run() == 1 && run2d_group_check(g, nullptr) == VTI_OK);
+    CHECK(g.run() == 1);
+    *g.dead = 1;   // as a workgroup does
+    CHECK(run2d_group_check(g, nullptr) == VTI_ERR_HIP);
+    CHECK(run2d_group_set(g, g.shots, nullptr) == VTI_OK && g.run() == 0);
+    CHECK(run2d_group_check(g, nullptr) == VTI_OK);
+}
+
 }  // namespace vti
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step},
-                                                       {"refused_program", vti::refused_program}};
+                                                       {"refused_program", vti::refused_program},
+                                                       {"missed_exchange", vti::missed_exchange}};
     const auto s = all.find(argc > 1 ? argv[1] : "");
     CHECK(s != all.end());
     s->second();
