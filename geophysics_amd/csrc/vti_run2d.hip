@@ -30,8 +30,9 @@
 // CPU_vti2dfd_kernels.c:78-177, Toa_gpu_2dtti_fd_1orderfunction.cu:81-183).
 //
 // Launch: cooperative (all workgroups resident, or the launch fails and the
-// per-step kernels run).  Every wait ends: a sample that does not come within
-// kWaitTicks raises the error word and the workgroup leaves its loop.
+// per-step kernels run).  Every wait ends: a tile that misses a sample for
+// kWaitTicks raises the error word and leaves its loop, and the others, which
+// look at the word while they wait, follow it within milliseconds.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -50,8 +51,10 @@ __device__ __forceinline__ float cst(int m)
     return m == 0 ? 1.196289f : (m == 1 ? -0.0797526f : (m == 2 ? 0.009570313f : -0.0006975447f));
 }
 
-// 100 MHz ticks a neighbour's sample may take before the call is given up (20 s)
-constexpr unsigned long long kWaitTicks = 2000000000ull;
+// 100 MHz ticks that a tile may wait for a neighbour's sample before the call is
+// given up (20 s); and those after which it looks whether another thread or tile
+// has (1 ms)
+constexpr unsigned kWaitTicks = 2000000000u, kLookTicks = 100000u;
 
 struct Run2dArgs {
     Run2dShot one;              // vti_step: the shot
@@ -65,6 +68,7 @@ struct Run2dArgs {
     const long long *offs;
     int image_every;
     unsigned base;              // tag before the call's first exchange
+    unsigned wait;              // ticks that a sample may take
     int *dead;                  // error word
 };
 
@@ -145,17 +149,32 @@ __device__ __forceinline__ unsigned long long peek(const unsigned long long *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The wait for one word is over when it began too long ago or, looked at only
+// after a while (at every poll it cost 0.14 us a step at 60 x 50), another
+// thread of the tile or another tile has given up.
+struct Wait {
+    unsigned limit;
+    int *dead;                  // the tile's (LDS)
+    const int *gone;            // the launch's error word
+    __device__ __forceinline__ bool over(unsigned t0) const
+    {
+        const unsigned d = (unsigned)wall_clock64() - t0;
+        if (d < min(kLookTicks, limit)) return false;
+        if (d <= limit && !__hip_atomic_load(dead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) &&
+            !__hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
+            return false;
+        *dead = 1;
+        return true;
+    }
+};
 // the word's sample once it carries the tag (w: an earlier look at it)
-__device__ __forceinline__ float await(const unsigned long long *p, unsigned long long w, unsigned tag, int *dead)
+__device__ __forceinline__ float await(const unsigned long long *p, unsigned long long w, unsigned tag, const Wait &x)
 {
     if ((unsigned)(w >> 32) != tag) {
-        const unsigned long long t0 = wall_clock64();
+        const unsigned t0 = (unsigned)wall_clock64();
         do {
             w = peek(p);
-            if (wall_clock64() - t0 > kWaitTicks) {
-                *dead = 1;
-                break;
-            }
+            if (x.over(t0)) break;   // asked while the load is on its way
         } while ((unsigned)(w >> 32) != tag);
     }
     return __uint_as_float((unsigned)w);
@@ -536,6 +555,7 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                     if (c < 4 || c >= nz - 4) put(gW + g, sW[r * L.wp + c], tag);
                 }
             }
+            const Wait wait{a.wait, &s_dead, a.dead};
             for (int k = vt; k < 21 * nz + 21 * nx; k += NT) {
                 const bool q = k >= 21 * nz;
                 int r, cc;
@@ -549,12 +569,12 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 if (x < 4 || x >= xend || z < 4 || z >= zend) continue;
                 const unsigned long long *p = (q ? (vel ? gW : gQ) : (vel ? gU : gP)) + (long long)x * ldz + z;
                 float *d = q ? (vel ? sW + r * L.wp + cc : sQ + r * L.qp + cc) : (vel ? sU + r * L.up + cc : sP + r * L.pp + cc);
-                *d = await(p, peek(p), tag, &s_dead);
+                *d = await(p, peek(p), tag, wait);
             }
             fresh = false;
             __syncthreads();
             if (s_dead) {
-                if (tid == 0) *a.dead = 1;
+                if (tid == 0) __hip_atomic_store(a.dead, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return;
             }
         } else if (PROG || s > 0) {
@@ -564,6 +584,7 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
             const int nrow = 14 * nz;
             const int wide = 14 * (nz + 14), nget = (TTI ? wide : nrow) + 14 * nx;
             const int total = TTI ? 2 * nget : nget;
+            const Wait wait{a.wait, &s_dead, a.dead};
             constexpr int B = NU == 1 && !TTI ? 1 : (NU < 4 ? 2 : 4);   // words looked at before the first wait
             for (int k0 = vt; k0 < total; k0 += B * NT) {
                 const unsigned long long *p[B];
@@ -592,11 +613,11 @@ __global__ __launch_bounds__(NT) void run2d_kernel(Run2dArgs a)
                 }
 #pragma unroll
                 for (int j = 0; j < B; ++j)
-                    if (at[j] >= 0) sm[at[j]] = await(p[j], w[j], tag, &s_dead);
+                    if (at[j] >= 0) sm[at[j]] = await(p[j], w[j], tag, wait);
             }
             __syncthreads();
             if (s_dead) {   // the same for every thread: written before the barrier only
-                if (tid == 0) *a.dead = 1;
+                if (tid == 0) __hip_atomic_store(a.dead, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return;
             }
         }
@@ -982,10 +1003,12 @@ bool capturing(hipStream_t s)
 
 thread_local long long t_launches = 0;   // vti_resident_launches
 thread_local long long t_left = -1;      // vti_resident_limit
+thread_local unsigned t_wait = kWaitTicks;   // vti_resident_wait
 
 hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     if (t_left == 0) return hipErrorOutOfMemory;
+    a.wait = t_wait;
     void *args[] = {&a};
     // The function's own limit, which its callers in all threads share: always
     // the same value, what a workgroup can have, never this launch's need.
@@ -1343,3 +1366,8 @@ int RtmProgram::flush()
 extern "C" long long vti_resident_launches(void) { return vti::t_launches; }
 
 extern "C" void vti_resident_limit(long long n) { vti::t_left = n < 0 ? -1 : n; }
+
+extern "C" void vti_resident_wait(long long us)
+{
+    vti::t_wait = us < 0 ? vti::kWaitTicks : (unsigned)std::min(us, (long long)vti::kWaitTicks / 100) * 100;
+}

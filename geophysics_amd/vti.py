@@ -97,6 +97,7 @@ def _declare(L):
         "vti_step": (C.c_int, [VP, C.c_int, C.c_int]),
         "vti_resident_launches": (C.c_longlong, []),
         "vti_resident_limit": (None, [C.c_longlong]),
+        "vti_resident_wait": (None, [C.c_longlong]),
         "vti_run": (C.c_int, [VP]),
         "vti_nrec": (C.c_int, [VP]),
         "vti_mute": (C.c_int, [VP] + [C.c_int] * 5),
@@ -267,6 +268,11 @@ def resident_launches():
 def resident_limit(n):
     """At most n further resident launches by this thread (None: no limit)."""
     lib().vti_resident_limit(-1 if n is None else n)
+
+
+def resident_wait(us):
+    """Microseconds that a resident launch by this thread may wait in an exchange (None: 20 s)."""
+    lib().vti_resident_wait(-1 if us is None else us)
 
 
 def learned_defaults():

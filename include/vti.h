@@ -167,6 +167,10 @@ long long vti_resident_launches(void);
  * is refused as the runtime may refuse any, and the call goes on with the
  * per-step kernels, from the middle of an RTM's schedule too. */
 void vti_resident_limit(long long n);
+/* Microseconds that a resident launch of this thread's calls may wait for a
+ * neighbouring tile's samples (us < 0, the default, and at most: 20 s); one
+ * that waits longer ends, and the call that waits for it returns VTI_ERR_HIP. */
+void vti_resident_wait(long long us);
 /* reset + all nt steps. */
 int vti_run(vti_ctx *ctx);
 
