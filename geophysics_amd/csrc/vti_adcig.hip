@@ -235,6 +235,8 @@ int vti_adcig_accumulate(vti_ctx *src, vti_ctx *rcv)
     if (a.ndim != b.ndim || a.nx != b.nx || a.nz != b.nz || (a.ndim == 3 && a.ny != b.ny) || a.npml != b.npml)
         return fail(VTI_ERR_ARG, "vti_adcig_accumulate: the contexts' grids differ");
     if (rcv->adcig_na <= 0) return fail(VTI_ERR_STATE, "vti_adcig_accumulate: no gathers configured (vti_adcig_config)");
+    int st = run2d_check(src);
+    if (st || (st = run2d_check(rcv))) return st;
     for (hipEvent_t &e : rcv->ev_acc)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
             return fail(VTI_ERR_HIP, "vti_adcig_accumulate: event");
@@ -273,7 +275,7 @@ int vti_adcig_get(vti_ctx *c, int illum_divide, float *adcigs)
     const hipError_t e2 = hipMemcpy(adcigs, tmp ? tmp : c->adcig, c->adcig_n * sizeof(float), hipMemcpyDeviceToHost);
     hipFree(tmp);
     if (e1 != hipSuccess || e2 != hipSuccess) return fail(VTI_ERR_HIP, "vti_adcig_get: copy");
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_adcig_stack(int nx, int nz, int nangle, const float *adcigs, float *migration)

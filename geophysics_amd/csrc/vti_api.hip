@@ -440,7 +440,7 @@ int vti_set_stream(vti_ctx *c, void *s)
         HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         c->own_stream = true;
     }
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_padded_dims(const vti_ctx *c, int *nnx, int *nny, int *nnz)
@@ -648,7 +648,7 @@ static int check_step(vti_ctx *c, int it)
         return fail(VTI_ERR_STATE, "split-form step after unsplit steps: the interior split fields are stale "
                                    "(call vti_reset first)");
     if (it < 0 || it >= c->cfg.nt) return fail(VTI_ERR_ARG, "time index out of range");
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_update_vel(vti_ctx *c, int it)
@@ -741,6 +741,8 @@ long long vti_state_bytes(const vti_ctx *c)
 int vti_save_state(vti_ctx *c, void *dst)
 {
     if (!c || !dst) return fail(VTI_ERR_ARG, "vti_save_state: null argument");
+    const int st = run2d_check(c);
+    if (st) return st;
     char *p = static_cast<char *>(dst);
     for (int k = 0; k < 11; ++k)
         if (c->f[k]) {
@@ -846,6 +848,8 @@ float *vti_record_device(vti_ctx *c) { return c ? c->rec : nullptr; }
 static int mute_common(vti_ctx *c, int form, int a0, int a1, int a2, int a3, int a4, int is, int tt)
 {
     if (!c || !c->rec) return fail(VTI_ERR_STATE, "vti_mute: no receiver buffer");
+    const int st = run2d_check(c);
+    if (st) return st;
     const int nt = c->cfg.nt, nrec = c->nrec, np = c->cfg.npml;
     const vti_shot &s = c->shot;
     HIP_TRY(launch_transpose(c->rec, c->rec_t, nt, nrec, c->stream));
@@ -921,7 +925,7 @@ int vti_set_field(vti_ctx *c, int which, const float *src)
     HIP_TRY(hipMemcpy2DAsync(p, g.ldz * sizeof(float), src, g.nnz * sizeof(float),
                              g.nnz * sizeof(float), (size_t)g.nnx * g.nny, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_get_table(vti_ctx *c, int which, float *dst)
@@ -950,7 +954,7 @@ int vti_prof_enable(vti_ctx *c, int on)
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->prof = on != 0;
     c->ev_used = 0;
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_prof_read(vti_ctx *c, double *vel_ms, double *stress_ms, int *nlaunch)
@@ -969,7 +973,7 @@ int vti_prof_read(vti_ctx *c, double *vel_ms, double *stress_ms, int *nlaunch)
     if (stress_ms) *stress_ms = ss;
     if (nlaunch) *nlaunch = (int)n;
     c->ev_used = 0;
-    return VTI_OK;
+    return run2d_check(c);
 }
 
 int vti_calib_copy(void *dst, const void *src, size_t nbytes, void *stream)

@@ -221,8 +221,9 @@ StressArgs with_snap(vti_ctx *c, StressArgs a, float *snap);
 // state of the context's grid, when the context has gathers configured
 hipError_t launch_adcig(vti_ctx *c, const VtiState &src, const VtiState &rcv);
 // vti_run2d.hip: n steps of the main state in one resident launch (1:
-// launched, 0: not applicable, < 0: error); its workspace; its error check
-// after a wait for the stream
+// launched, 0: not applicable, < 0: error); its workspace; its error check, by
+// every call that waits for the stream, after the wait, and by those that queue
+// work on the state, before it
 int run2d_steps(vti_ctx *c, int it0, int n);
 void run2d_free(vti_ctx *c);
 int run2d_check(vti_ctx *c);

@@ -589,6 +589,8 @@ int vti_image_accumulate(vti_ctx *src, vti_ctx *rcv, float *img, float *illum, i
     const vti_cfg &a = src->cfg, &b = rcv->cfg;
     if (a.ndim != b.ndim || a.nx != b.nx || a.nz != b.nz || (a.ndim == 3 && a.ny != b.ny) || a.npml != b.npml)
         return fail(VTI_ERR_ARG, "vti_image_accumulate: the contexts' grids differ");
+    int st = run2d_check(src);
+    if (st || (st = run2d_check(rcv))) return st;
     for (hipEvent_t &e : rcv->ev_acc)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
             return fail(VTI_ERR_HIP, "vti_image_accumulate: event");

@@ -156,7 +156,11 @@ int vti_update_vel(vti_ctx *ctx, int it);
  * (CPU mode) and the receiver gather of row it (update_stress2d +
  * shot_record2d, :425-429). */
 int vti_update_stress(vti_ctx *ctx, int it);
-/* nsteps full steps starting at it0. */
+/* nsteps full steps starting at it0, queued on the context's stream.  The
+ * resident 2D kernel's one error of its own (vti_resident_wait) is returned
+ * once, by the first call on the context that waits for the stream or, if it
+ * has come by then, that queues work on the state or the record; the fields
+ * and the record are undefined then (vti_reset starts anew). */
 int vti_step(vti_ctx *ctx, int it0, int nsteps);
 /* Launches of the resident 2D kernel (many steps in one launch: vti_step /
  * vti_run of 8 steps or more, vti_rtm_shot, vti_batch_rtm, vti_grad_*) that

@@ -38,6 +38,42 @@ def test_steps(wait, form, unsplit, nx, nz):
             assert n() == 0
 
 
+CALLS = {
+    # these wait for the stream
+    "sync": lambda p, d: p.sync(), "get_record": lambda p, d: p.record(), "get_field": lambda p, d: p.field("P"),
+    "set_field": lambda p, d: p.set_field("u", np.zeros(p.shape, dtype=np.float32)),
+    "set_stream": lambda p, d: vti.check(vti.lib().vti_set_stream(p.h, None)),
+    "prof_enable": lambda p, d: p.prof_enable(False), "prof_read": lambda p, d: p.prof_read(),
+    "adcig_get": lambda p, d: p.adcig(),
+    # these queue work on the state or the record
+    "step": lambda p, d: p.step(0, 2), "update_vel": lambda p, d: p.update_vel(0),
+    "update_stress": lambda p, d: p.update_stress(0), "mute": lambda p, d: p.mute(60, 0, 2, 1),
+    "save_state": lambda p, d: vti.check(vti.lib().vti_save_state(p.h, d.data_ptr())),
+    "image_accumulate": lambda p, d: vti.check(vti.lib().vti_image_accumulate(p.h, p.h, d.data_ptr(), None, 0)),
+    "adcig_accumulate": lambda p, d: vti.check(vti.lib().vti_adcig_accumulate(p.h, p.h)),
+}
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_every_call_reports(wait, call):
+    import torch
+    with build("gpu", 120, 90, 20, 80) as p:
+        d = torch.zeros(p.state_bytes() // 4, device="cuda")
+        torch.cuda.synchronize()
+        p.adcig_config(2)
+        p.step(0, 80)
+        CALLS[call](p, d)
+        wait(0)
+        p.step(0, 80)
+        torch.cuda.synchronize()        # the device, without a call on the context
+        with pytest.raises(vti.VtiError, match=MISSED):
+            CALLS[call](p, d)
+        p.sync()                        # once
+        p.reset()
+        CALLS[call](p, d)
+        p.sync()
+
+
 def test_rtm(wait):
     nx, nz, nt = 333, 71, 40
     with build("gpu", nx, nz, 20, nt, True) as p:
