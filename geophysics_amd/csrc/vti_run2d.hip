@@ -980,19 +980,31 @@ void place_planes(Run2dShot *shots, int n, int nfield, unsigned long long *p)
     }
 }
 
+// Allocations that leave alone a capture of another stream, which the default
+// mode would end.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // a context's exchange planes, zeroed, and its host-visible error word
-bool alloc_plan(std::vector<Run2dShot> &shots, unsigned long long *&xbuf, int *&dead, hipStream_t s)
+bool alloc_plan(const Run2dShot &shot, unsigned long long *&xbuf, int *&dead, hipStream_t s)
 {
-    const size_t n = plane_words(shots.data(), 1, 2);
-    if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess ||
-        launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
+    const size_t n = plane_words(&shot, 1, 2);
+    const RelaxedCapture relaxed;
+    if (hipMalloc(&xbuf, n * sizeof(unsigned long long)) != hipSuccess) xbuf = nullptr;
+    else if (hipHostMalloc(&dead, sizeof(int), hipHostMallocMapped) != hipSuccess) dead = nullptr;
+    else if (launch_zero(reinterpret_cast<float *>(xbuf), 2 * n, s) == hipSuccess) {
+        *dead = 0;
+        return true;
     }
-    *dead = 0;
-    place_planes(shots.data(), 1, 2, xbuf);
-    return true;
+    (void)hipFree(xbuf);
+    (void)hipHostFree(dead);
+    xbuf = nullptr;
+    dead = nullptr;
+    (void)hipGetLastError();
+    return false;
 }
 
 bool capturing(hipStream_t s)
@@ -1035,7 +1047,7 @@ hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, h
 }  // namespace
 
 struct Run2dPlan {
-    int ok = 0;                 // 1: usable, -1: this grid or device takes the per-step kernels
+    int ok = 0;                 // 1: usable, 0: not planned yet, -1: this grid or device takes the per-step kernels
     std::vector<Run2dShot> shot;   // one: the plan's share of it
     int shape = 0, ntile = 0;
     size_t lds = 0;
@@ -1091,21 +1103,18 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     // (5.8 us a step and up).
     if (c->cfg.ndim != 2 || n < 8 || c->cfg.mode == VTI_MODE_OMP_REF || capturing(c->stream)) return 0;
     const bool tti = c->tti != nullptr;
-    if (c->run2d && c->run2d->tti != tti) {
-        if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: sync");
-        run2d_free(c);
-    }
-    if (!c->run2d) {
-        c->run2d = new (std::nothrow) Run2dPlan();
-        if (!c->run2d) return 0;
-        Run2dPlan &p = *c->run2d;
+    if (!c->run2d) c->run2d = new (std::nothrow) Run2dPlan();
+    if (!c->run2d) return 0;
+    Run2dPlan &p = *c->run2d;
+    if (!p.ok || p.tti != tti) {   // both forms use the planes alike
         p.tti = tti;
         p.ok = -1;
         Device2d d;
-        p.shot.push_back(run2d_shot(c, main_state(c)));
+        p.shot.assign(1, run2d_shot(c, main_state(c)));
         if (!device_2d(c->device, d)) return 0;
         const Plan2d one = plan_group(cuts_of_all(p.shot, tti, kNumShapes, d), 0, 1, d);
-        if (one.cut.empty() || !alloc_plan(p.shot, p.xbuf, p.dead, c->stream)) return 0;
+        if (one.cut.empty() || (!p.xbuf && !alloc_plan(p.shot[0], p.xbuf, p.dead, c->stream))) return 0;
+        place_planes(p.shot.data(), 1, 2, p.xbuf);
         p.shape = one.shape;
         p.lds = one.cut[0].lds;
         p.ntile = one.cut[0].tiles;
@@ -1113,7 +1122,6 @@ int run2d_steps(vti_ctx *c, int it0, int n)
         p.shot[0].gz = one.cut[0].gz;
         p.ok = 1;
     }
-    Run2dPlan &p = *c->run2d;
     if (p.ok != 1) return 0;
     Run2dArgs a{};
     const Run2dShot &t = p.shot[0];
