@@ -37,7 +37,10 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <functional>
+#include <map>
 #include <new>
+#include <queue>
 #include <string>
 
 #include "vti_internal.h"
@@ -859,11 +862,17 @@ void cuts_of(int nnx, int nnz, bool tti, int shape, int cus, int lds_max, std::v
     if (uq < 2) return;
     const int nt = kShapes[shape].nt, nu = kShapes[shape].nu;
     std::vector<Cut> best(cus + 1, Cut{0, 0, 0, 0, 1e300});   // by tiles
-    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); ++gx) {
+    // more columns or rows of tiles of the same height or width never pay: go
+    // on to the next smaller one
+    auto next = [](int n, int g) {
+        const int size = (n + g - 1) / g;
+        return size > 1 ? std::max(g + 1, (n + size - 2) / (size - 1)) : n + 1;
+    };
+    for (int gx = 1; gx <= std::min(cus, std::max(1, ux / 7)); gx = next(ux, gx)) {
         const int nx = (ux + gx - 1) / gx, rows = (nx + nu - 1) / nu;
         if (nx + 14 > nt || 8 * rows > nt) continue;
         const int widest = nt / rows / 4;   // units of 4 columns that leave a thread one strip
-        for (int gz = (uq + widest - 1) / widest; gz <= std::min(cus / gx, std::max(1, uq / 2)); ++gz) {
+        for (int gz = (uq + widest - 1) / widest; gz <= std::min(cus / gx, std::max(1, uq / 2)); gz = next(uq, gz)) {
             const int nz = 4 * ((uq + gz - 1) / gz);
             const int strips = rows * nz;
             const size_t b = 4 * (size_t)(tti ? Lds<true>(nx, nz).total : Lds<false>(nx, nz).total);
@@ -900,63 +909,68 @@ bool device_2d(int device, Device2d &d)
     return true;
 }
 
-// One tile per CU for n shots together, the same launch shape: the shape and
-// the cuts with the least cost of the slowest tile.  cuts: [shape][shot].
+// One tile per CU for one shot: the shape and the cut with the least cost.
 struct Plan2d {
     double cost = 1e300;
     int shape = 0;
     std::vector<Cut> cut;
 };
-using Cuts2d = std::vector<std::vector<std::vector<Cut>>>;
-Cuts2d cuts_of_all(const std::vector<Run2dShot> &shots, bool tti, int nshape, const Device2d &d)
-{
-    Cuts2d cuts(nshape);
-    for (int k = 0; k < nshape; ++k) {
-        cuts[k].resize(shots.size());
-        for (size_t s = 0; s < shots.size(); ++s) cuts_of(shots[s].nnx, shots[s].nnz, tti, k, d.cus, d.lds, cuts[k][s]);
-    }
-    return cuts;
-}
-Plan2d plan_group(const Cuts2d &cuts, int first, int n, const Device2d &d)
+Plan2d plan_one(const Run2dShot &s, bool tti, const Device2d &d)
 {
     Plan2d best;
-    std::vector<Cut> pick(n);
-    for (size_t k = 0; k < cuts.size(); ++k) {
-        std::vector<double> costs;
-        bool all = true;
-        for (int s = 0; s < n && all; ++s) {
-            all = !cuts[k][first + s].empty();
-            for (const Cut &c : cuts[k][first + s]) costs.push_back(c.cost);
-        }
-        if (!all) continue;
-        std::sort(costs.begin(), costs.end());
-        auto fits = [&](double c) {   // fewest tiles of every shot within cost c
-            int tiles = 0;
-            for (int s = 0; s < n; ++s) {
-                const Cut *b = nullptr;
-                for (const Cut &x : cuts[k][first + s])
-                    if (x.cost <= c) {
-                        b = &x;
-                        break;
-                    }
-                if (!b || (tiles += b->tiles) > d.cus) return false;
-                pick[s] = *b;
-            }
-            return true;
-        };
-        size_t lo = 0, hi = costs.size();
-        while (lo < hi) {   // the least cost that fits
-            const size_t mid = (lo + hi) / 2;
-            if (fits(costs[mid])) hi = mid;
-            else lo = mid + 1;
-        }
-        if (lo == costs.size() || costs[lo] >= best.cost || !fits(costs[lo])) continue;
-        best.cost = costs[lo];
-        best.shape = (int)k;
-        best.cut = pick;
+    std::vector<Cut> cuts;
+    for (int k = 0; k < kNumShapes; ++k) {
+        cuts_of(s.nnx, s.nnz, tti, k, d.cus, d.lds, cuts);
+        if (!cuts.empty() && cuts.back().cost < best.cost) best = Plan2d{cuts.back().cost, k, {cuts.back()}};
     }
     return best;
 }
+
+// One tile per CU for shots together, with one launch shape: the least cost of
+// the slowest tile, every shot cut into the fewest tiles within it.  Shots are
+// added one by one: the cost only rises then, and a shot's tiles only get fewer
+// (planned anew for every number of shots, 256 shots took 30 ms).
+struct PartPlan {
+    using Cuts = std::vector<Cut>;      // of one grid: ascending tiles, descending cost
+    double cost = 0.0;
+    int tiles = 0;
+    bool fits = true;
+    std::vector<const Cuts *> cuts;     // by shot
+    std::vector<int> pick;
+    std::priority_queue<std::pair<double, int>, std::vector<std::pair<double, int>>, std::greater<>> next;   // cost of
+                                                                                       // the next fewer tiles, shot
+    void take(int s)                    // the fewest tiles within the cost
+    {
+        const Cuts &c = *cuts[s];
+        if (pick[s] >= 0) tiles -= c[pick[s]].tiles;
+        pick[s] = (int)(std::partition_point(c.begin(), c.end(), [&](const Cut &x) { return x.cost > cost; }) - c.begin());
+        tiles += c[pick[s]].tiles;
+        if (pick[s]) next.push({c[pick[s] - 1].cost, s});
+    }
+    void relax()
+    {
+        while (!next.empty() && next.top().first <= cost) {
+            const int s = next.top().second;
+            next.pop();
+            take(s);
+        }
+    }
+    void add(const Cuts &c, int cus)
+    {
+        fits = fits && !c.empty();
+        if (!fits) return;
+        cuts.push_back(&c);
+        pick.push_back(-1);
+        cost = std::max(cost, c.back().cost);
+        relax();
+        take((int)cuts.size() - 1);
+        while (tiles > cus && !next.empty()) {
+            cost = next.top().first;
+            relax();
+        }
+        fits = tiles <= cus;
+    }
+};
 
 size_t plane_of(const Run2dShot &s) { return (size_t)s.ldz * s.nnx; }
 
@@ -1112,7 +1126,7 @@ int run2d_steps(vti_ctx *c, int it0, int n)
         Device2d d;
         p.shot.assign(1, run2d_shot(c, main_state(c)));
         if (!device_2d(c->device, d)) return 0;
-        const Plan2d one = plan_group(cuts_of_all(p.shot, tti, kNumShapes, d), 0, 1, d);
+        const Plan2d one = plan_one(p.shot[0], tti, d);
         if (one.cut.empty() || (!p.xbuf && !alloc_plan(p.shot[0], p.xbuf, p.dead, c->stream))) return 0;
         place_planes(p.shot.data(), 1, 2, p.xbuf);
         p.shape = one.shape;
@@ -1167,7 +1181,18 @@ Run2dParts run2d_parts(const std::vector<Run2dShot> &shots, int device)
     Device2d d;
     if (!device_2d(device, d)) return r;
     const int ns = (int)shots.size();
-    Cuts2d cuts = cuts_of_all(shots, false, kRtmShapes, d);
+    // one list of cuts a shape and grid
+    std::map<std::pair<int, int>, int> grids;
+    std::vector<int> grid(ns);
+    std::vector<PartPlan::Cuts> cuts[kRtmShapes];
+    for (int k = 0; k < ns; ++k) {
+        const auto g = grids.insert({{shots[k].nnx, shots[k].nnz}, (int)grids.size()});
+        grid[k] = g.first->second;
+        for (int j = 0; g.second && j < kRtmShapes; ++j) {
+            cuts[j].emplace_back();
+            cuts_of(shots[k].nnx, shots[k].nnz, false, j, d.cus, d.lds, cuts[j].back());
+        }
+    }
     // strips of 6 spill ~95 registers with the images: for shots that fit no
     // other way (24 shots of 0.1 to 1 M cells: 46 ms in parts of strips of 6
     // taken at their plain cost, 39 with parts of 4)
@@ -1175,14 +1200,21 @@ Run2dParts run2d_parts(const std::vector<Run2dShot> &shots, int device)
         for (Cut &x : c) x.cost *= 2.0;
     for (int first = 0; first < ns;) {
         Plan2d best;
+        PartPlan plan[kRtmShapes];
         double rate = 1e300, cells = 0.0;
         for (int n = 1; first + n <= ns; ++n) {
             cells += (double)shots[first + n - 1].nnx * shots[first + n - 1].nnz;
-            const Plan2d p = plan_group(cuts, first, n, d);
-            if (p.cut.empty()) break;
+            int least = -1;
+            for (int j = 0; j < kRtmShapes; ++j) {
+                plan[j].add(cuts[j][grid[first + n - 1]], d.cus);
+                if (plan[j].fits && (least < 0 || plan[j].cost < plan[least].cost)) least = j;
+            }
+            if (least < 0) break;
+            const PartPlan &p = plan[least];
             if ((p.cost + 4000.0) / cells >= rate) continue;
             rate = (p.cost + 4000.0) / cells;
-            best = p;
+            best = Plan2d{p.cost, least, {}};
+            for (int k = 0; k < n; ++k) best.cut.push_back((*p.cuts[k])[p.pick[k]]);
         }
         if (best.cut.empty()) return Run2dParts{};
         Run2dPart q{first, (int)best.cut.size(), best.shape, 0, 0};

@@ -3,6 +3,7 @@
 // refused as the scenario asks.  No device is touched and no kernel runs.
 // test_host_run2d.py builds it with the device passes left out and runs one
 // scenario (argv[1]) a time; a failed condition names itself and ends it.
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -201,13 +202,146 @@ void missed_exchange()
     CHECK(run2d_group_check(g, nullptr) == VTI_OK);
 }
 
+// The parts of a list of shots by a plain search, every number of shots and
+// every cost anew.
+Run2dParts plain_parts(const std::vector<Run2dShot> &shots, const Device2d &d)
+{
+    Run2dParts r;
+    const int ns = (int)shots.size();
+    std::vector<std::vector<Cut>> cuts[kRtmShapes];
+    for (int j = 0; j < kRtmShapes; ++j)
+        for (const Run2dShot &s : shots) {
+            cuts[j].emplace_back();
+            cuts_of(s.nnx, s.nnz, false, j, d.cus, d.lds, cuts[j].back());
+            if (j == kRtmShapes - 1)
+                for (Cut &c : cuts[j].back()) c.cost *= 2.0;
+        }
+    for (int first = 0; first < ns;) {
+        double rate = 1e300, cells = 0.0;
+        Run2dPart part{};
+        std::vector<Cut> taken;
+        for (int n = 1; first + n <= ns; ++n) {
+            cells += (double)shots[first + n - 1].nnx * shots[first + n - 1].nnz;
+            double least = 1e300;
+            int shape = 0;
+            std::vector<Cut> pick;
+            for (int j = 0; j < kRtmShapes; ++j) {
+                std::vector<double> costs;
+                for (int s = 0; s < n; ++s)
+                    for (const Cut &c : cuts[j][first + s]) costs.push_back(c.cost);
+                std::sort(costs.begin(), costs.end());
+                auto fit = [&](double c) {
+                    std::vector<Cut> p;
+                    int tiles = 0;
+                    for (int s = 0; s < n; ++s) {
+                        const auto &l = cuts[j][first + s];
+                        const auto i = std::find_if(l.begin(), l.end(), [&](const Cut &x) { return x.cost <= c; });
+                        if (i == l.end() || (tiles += i->tiles) > d.cus) return std::vector<Cut>{};
+                        p.push_back(*i);
+                    }
+                    return p;
+                };
+                const auto i = std::partition_point(costs.begin(), costs.end(), [&](double c) { return fit(c).empty(); });
+                if (i == costs.end() || *i >= least) continue;
+                least = *i;
+                shape = j;
+                pick = fit(*i);
+            }
+            if (pick.empty()) break;
+            if ((least + 4000.0) / cells >= rate) continue;
+            rate = (least + 4000.0) / cells;
+            part = Run2dPart{first, n, shape, 0, 0};
+            taken = pick;
+        }
+        if (taken.empty()) return Run2dParts{};
+        for (const Cut &c : taken) {
+            r.gx.push_back(c.gx);
+            r.gz.push_back(c.gz);
+            r.tile0.push_back(part.ntile);
+            part.ntile += c.tiles;
+            part.lds = std::max(part.lds, c.lds);
+        }
+        r.part.push_back(part);
+        first += part.n;
+    }
+    return r;
+}
+
+// The plans are those of the plain search, on a whole and on a smaller device,
+// with shots that no launch holds among them; every cut covers its grid with
+// tiles that the kernel can hold; and a large batch is planned much faster.
+void plans()
+{
+    unsigned seed = 7;
+    auto draw = [&](int lo, int hi) { return lo + (int)((seed = seed * 1664525u + 1013904223u) >> 8) % (hi - lo); };
+    double plain = 0.0, quick = 0.0;
+    for (int t = 0; t < 24; ++t) {
+        g_cus = t % 3 == 2 ? 64 : 256;
+        std::vector<Run2dShot> shots;
+        const int n = draw(1, 40), large = t % 4 == 3 ? 2500 : 900;
+        for (int k = 0; k < n; ++k) {
+            Run2dShot b{};
+            b.nnx = draw(16, k % 5 ? 500 : large);
+            b.nnz = draw(16, k % 5 ? 300 : large);
+            if (k && k % 3 == 0) {      // grids that occur again
+                b.nnx = shots[0].nnx;
+                b.nnz = shots[0].nnz;
+            }
+            shots.push_back(b);
+        }
+        if (t == 23) shots.assign(200, shots[0]);
+        Device2d d;
+        CHECK(device_2d(0, d));
+        auto clock = [] { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); };
+        const double t0 = clock();
+        const Run2dParts a = plain_parts(shots, d);
+        const double t1 = clock();
+        const Run2dParts b = run2d_parts(shots, 0);
+        if (t == 23) {
+            plain = t1 - t0;
+            quick = clock() - t1;
+        }
+        CHECK(a.gx == b.gx && a.gz == b.gz && a.tile0 == b.tile0 && a.part.size() == b.part.size());
+        for (size_t k = 0; k < a.part.size(); ++k) {
+            const Run2dPart &p = a.part[k], &q = b.part[k];
+            CHECK(p.first == q.first && p.n == q.n && p.shape == q.shape && p.ntile == q.ntile && p.lds == q.lds);
+            CHECK(q.ntile <= d.cus && q.lds + kStaticLds <= (size_t)d.lds);
+            for (int s = q.first; s < q.first + q.n; ++s) {
+                const Run2dShot &g = shots[s];
+                const int nt = kShapes[q.shape].nt, nu = kShapes[q.shape].nu;
+                int cells = 0;
+                for (int i = 0; i < b.gx[s] * b.gz[s]; ++i) {
+                    const Tile w = tile_of(g.nnx, g.nnz, b.gx[s], b.gz[s], i / b.gz[s], i % b.gz[s]);
+                    CHECK(w.nx >= std::min(7, g.nnx - 8) && w.nz >= 8 && w.nx + 14 <= nt);
+                    CHECK((w.nx + nu - 1) / nu * w.nz <= nt && 4 * (size_t)Lds<false>(w.nx, w.nz).total <= q.lds);
+                    cells += w.nx * w.nz;
+                }
+                CHECK(cells == (g.nnx - 8) * ((g.nnz - 8 + 3) / 4 * 4));
+            }
+        }
+        for (bool tti : {false, true}) {
+            const Plan2d one = plan_one(shots[0], tti, d);
+            double least = 1e300;
+            std::vector<Cut> c;
+            for (int k = 0; k < kNumShapes; ++k) {
+                cuts_of(shots[0].nnx, shots[0].nnz, tti, k, d.cus, d.lds, c);
+                for (const Cut &x : c) least = std::min(least, x.cost);
+            }
+            CHECK(one.cost == least && one.cut.empty() == (least == 1e300));
+        }
+    }
+    std::printf("200 shots: %.2f ms, plain search %.2f ms\n", 1e3 * quick, 1e3 * plain);
+    CHECK(quick < 0.2 * plain);
+}
+
 }  // namespace vti
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step},
                                                        {"refused_program", vti::refused_program},
-                                                       {"missed_exchange", vti::missed_exchange}};
+                                                       {"missed_exchange", vti::missed_exchange},
+                                                       {"plans", vti::plans}};
     const auto s = all.find(argc > 1 ? argv[1] : "");
     CHECK(s != all.end());
     s->second();
