@@ -189,6 +189,7 @@ struct vti_ctx {
     // volumes; nullptr: VTI
     float *tti = nullptr;
     vti::Run2dPlan *run2d = nullptr;   // resident 2D steps (vti_run2d.hip), made at their first use
+    long long asked2d = 0;             // steps asked of vti_step before that
 };
 
 namespace vti {

@@ -1112,10 +1112,19 @@ Run2dShot run2d_shot(vti_ctx *c, const VtiState &s)
 int run2d_steps(vti_ctx *c, int it0, int n)
 {
     // Two steps let the write-back start after every neighbour has loaded.
-    // Below eight the call's fixed cost (a cooperative launch, the tile's
-    // coefficients, load and store) is more than the per-step kernels take
-    // (5.8 us a step and up).
-    if (c->cfg.ndim != 2 || n < 8 || c->cfg.mode == VTI_MODE_OMP_REF || capturing(c->stream)) return 0;
+    // Below eight the call's fixed cost (launch, the tile's coefficients, load
+    // and store: 25 us at 60 x 50, 55 at 2401 x 803) is what the per-step kernels
+    // take: us a call of 8 / 10 / 16 steps among others, per-step and resident,
+    // 200 x 150 46, 41 / 58, 45 / 91, 56; 400 x 400 58, 53 / 72, 59 / 114, 76;
+    // 2401 x 803 222, 139 / 281, 160 / 460, 224.
+    if (c->cfg.ndim != 2 || c->cfg.mode == VTI_MODE_OMP_REF || capturing(c->stream)) return 0;
+    // The plan and its memory cost a context's first such call 60 to 400 us, a
+    // step saves 4 to 18: us of a fresh context's first call of 16 / 24 / 32
+    // steps, per-step and resident, 200 x 150 106, 108 / 149, 121 / 197, 141;
+    // 601 x 301 139, 167 / 202, 194 / 266, 219; 1401 x 503 254, 457 / 370, 508 /
+    // 488, 535; 2401 x 803 532, 630 / 782, 698 / 1033, 792.
+    if (!c->run2d) c->asked2d += n;
+    if (n < 8 || (!c->run2d && c->asked2d < 24)) return 0;
     const bool tti = c->tti != nullptr;
     if (!c->run2d) c->run2d = new (std::nothrow) Run2dPlan();
     if (!c->run2d) return 0;

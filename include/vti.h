@@ -163,9 +163,10 @@ int vti_update_stress(vti_ctx *ctx, int it);
  * and the record are undefined then (vti_reset starts anew). */
 int vti_step(vti_ctx *ctx, int it0, int nsteps);
 /* Launches of the resident 2D kernel (many steps in one launch: vti_step /
- * vti_run of 8 steps or more, vti_rtm_shot, vti_batch_rtm, vti_grad_*) that
- * calls of this thread have made so far; where it does not apply or cannot be
- * launched, the per-step kernels run and the count stays. */
+ * vti_run of 8 steps or more, from a context's 24th step on; vti_rtm_shot;
+ * vti_batch_rtm; vti_grad_*) that calls of this thread have made so far; where
+ * it does not apply or cannot be launched, the per-step kernels run and the
+ * count stays. */
 long long vti_resident_launches(void);
 /* At most n further ones (n < 0, the default: no limit): a launch above that
  * is refused as the runtime may refuse any, and the call goes on with the

@@ -129,8 +129,8 @@ void lds_attribute()
 {
     Ctx large(1440, 543), small(1340, 543);
     int r = -1;
-    g_after_attribute = [&] { r = run2d_steps(&small, 0, 16); };
-    const int q = run2d_steps(&large, 0, 16);
+    g_after_attribute = [&] { r = run2d_steps(&small, 0, 32); };
+    const int q = run2d_steps(&large, 0, 32);
     CHECK(r == 1 && g_launched.size() >= 1);
     CHECK(q == 1 && g_launched.size() == 2);
     CHECK(g_launched[0].kernel == g_launched[1].kernel && g_launched[0].lds < g_launched[1].lds);
@@ -142,8 +142,8 @@ void refused_step()
 {
     Ctx c(440, 440);
     g_refuse = {hipErrorOutOfMemory};
-    CHECK(run2d_steps(&c, 0, 16) == 0);
-    CHECK(run2d_steps(&c, 16, 16) == 1 && g_launched.size() == 1);
+    CHECK(run2d_steps(&c, 0, 32) == 0);
+    CHECK(run2d_steps(&c, 32, 16) == 1 && g_launched.size() == 1);
     g_refuse = {hipErrorCooperativeLaunchTooLarge};
     CHECK(run2d_steps(&c, 0, 16) == 0);
     CHECK(run2d_steps(&c, 16, 16) == 0 && g_launched.size() == 1);

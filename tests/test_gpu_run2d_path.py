@@ -63,6 +63,17 @@ def test_steps_are_resident(form, unsplit, nx, nz, npml):
         assert n() == 3
 
 
+def test_short_runs_of_a_fresh_context_keep_the_per_step_kernels():
+    """The plan and its memory pay from 24 steps on, in whatever calls."""
+    for calls, launches in (((23,), 0), ((24,), 1), ((8, 15), 0), ((8, 3, 13), 1), ((16, 8, 8), 2), ((23, 7, 8), 1)):
+        with build("gpu", 120, 90, 20, 40) as p, Launches() as n:
+            it = 0
+            for k in calls:
+                p.step(it, k)
+                it += k
+            assert n() == launches, calls
+
+
 # too large for the chip, and the form whose sums are in double
 @pytest.mark.parametrize("form,nx,nz,npml", [("gpu", 2500, 1000, 20), ("tti", 2401, 803, 20), ("omp", 120, 90, 0)])
 def test_steps_keep_the_per_step_kernels(form, nx, nz, npml):

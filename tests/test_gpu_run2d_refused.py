@@ -21,8 +21,8 @@ def test_steps(limit):
     for n in (None, 1, 0):
         with build("gpu", 333, 71, 20, 40) as p:
             limit(n)
-            p.step(0, 20)
-            p.step(20, 20)
+            p.step(0, 26)
+            p.step(26, 14)
             out.append((p.field("P"), p.field("pz"), p.record()))
     for o in out[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(o, out[0]))
