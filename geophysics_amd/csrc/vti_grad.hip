@@ -401,6 +401,7 @@ struct Grad : vti_grad {
     Run2dGroup res2d;            // 2D, FP32: the resident first sweep
     float *damp = nullptr;       // its source gains
     int res2d_state = 0;         // 1: made, -1: not available
+    int sweeps = 0;              // first sweeps so far
 
     ~Grad() override
     {
@@ -620,12 +621,17 @@ struct Grad : vti_grad {
     // The forward sweep with its record as one resident launch (FP32, 2D):
     // q collects the steps and checkpoints.  1040 x 340, 400 steps: 4.4 ms
     // step by step, 1.7 so; recomputation runs of ~10 steps between adjoint
-    // steps stay with the per-step kernels (a resident launch costs ~100 us).
+    // steps stay with the per-step kernels.  The descriptors, gains and program
+    // cost each sweep ~80 us, the object's first one 80 to 250 us more for the
+    // plan and its memory: us of forward(), first / later, step by step and so,
+    // of 12 / 16 / 32 / 64 steps, 60 x 50 106, 174 / 128, 218 / 222, 196 / 416,
+    // 283 and 138, 125 / 168, 135 / 278, 171 / 534, 243; 1000 x 300 194, 268 /
+    // 228, 293 / 417, 380 / 881, 689 and 174, 159 / 229, 178 / 397, 252 / 873, 531.
     // 1: q is set up, 0: not available, < 0: error
     int resident(RtmProgram &q)
     {
         if constexpr (sizeof(T) == 4) {
-            if (g.three || cfg.nt < 8 || res2d_state < 0) return 0;
+            if (g.three || res2d_state < 0 || cfg.nt < (sweeps++ ? 16 : 32)) return 0;
             Run2dShot b{};
             b.nnx = g.nnx; b.nnz = g.nnz; b.ldz = g.ldz; b.M = M;
             T *const fl[8] = {f.u, f.w, f.px, f.pz, f.qx, f.qz, f.P, f.Q};

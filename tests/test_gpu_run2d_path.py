@@ -134,6 +134,21 @@ def test_gradients(nx, nz, npml, fp64, resident):
             assert n() == (2 * k if resident else 0)   # the modelled record; the first sweep
 
 
+@pytest.mark.parametrize("nt,launches", [(12, (0, 0, 0)), (24, (0, 1, 2)), (40, (1, 2, 3))])
+def test_short_gradients(nt, launches):
+    """A few steps pay from the second sweep of an object on, or not at all."""
+    nx, nz = 120, 90
+    cfg = vti.cfg_ref2d(vti.MODE_GPU_REF, nx, nz, 10, 10, 20, 1, 20, nt, 1000)
+    with vti.Gradient(cfg, fp64=False) as G, Launches() as n:
+        G.set_model(*models(nx, nz))
+        G.set_shot(vti.shot_ref2d(cfg, 1, nx // 2, 0, nz // 2, rec_depth=nz // 2))
+        out = []
+        for k in launches:
+            out.append(G.forward())
+            assert n() == k
+        assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
 def test_threads_of_one_launch_shape():
     """Four threads whose grids share a launch shape (threads and rows a strip)
     and need different amounts of LDS: every call is a resident launch, and the
