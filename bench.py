@@ -755,19 +755,17 @@ def main():
     vel_avg = vel_ms / max(nl, 1) / 1e3
     fused = args.fused and args.split
     unsplit = not args.split
-    pad = n + 2 * npml
-    field_mb = 4e-6 * pad * pad * ((pad + 31) // 32 * 32)   # which fields bypass the caches depends on the size
     if fused:
         # one kernel per step: the step's algorithmic bytes over its duration
         kernel = "vti::f3d::fused3d<32, true>"
         achieved = BYTES_STEP * cells / str_avg / 1e9
         tfile = os.path.join(ROOT, "profiles", "fused3d_traffic.json")
     elif unsplit:
-        kernel = f"vti::s3d::stress3d<4, {2 if 2 * field_mb > 160 else int(9.5 * field_mb > 250)}, true, false>"
+        kernel = vti.stress3d_name(cfg, True)
         achieved = BYTES_STRESS * cells / str_avg / 1e9
         tfile = os.path.join(ROOT, "profiles", "stress3d_unsplit_traffic.json")
     else:
-        kernel = f"vti::s3d::stress3d<{16 if field_mb > 500 else 4}, {int(14 * field_mb > 250)}, false, false>"
+        kernel = vti.stress3d_name(cfg, False)
         achieved = BYTES_STRESS * cells / str_avg / 1e9
         tfile = os.path.join(ROOT, "profiles", "stress3d_traffic.json")
     traffic = None

@@ -976,6 +976,20 @@ int vti_prof_read(vti_ctx *c, double *vel_ms, double *stress_ms, int *nlaunch)
     return run2d_check(c);
 }
 
+int vti_stress3d_name(const vti_cfg *c, int unsplit, char *name, int size)
+{
+    if (!c || !name || c->ndim != 3 || c->nx < 1 || c->ny < 1 || c->nz < 1 || c->npml < 0)
+        return fail(VTI_ERR_ARG, "vti_stress3d_name: a 3D configuration and a buffer");
+    Grid g{};
+    g.nnx = c->nx + 2 * c->npml; g.nny = c->ny + 2 * c->npml; g.nnz = c->nz + 2 * c->npml;
+    g.ldz = (g.nnz + 31) / 32 * 32;
+    g.ldxy = (long long)g.ldz * g.nnx;
+    const std::string s = stress3d_name(g, unsplit != 0 && c->mode == VTI_MODE_GPU_REF);
+    if (size < (int)s.size() + 1) return fail(VTI_ERR_ARG, "vti_stress3d_name: buffer too small");
+    std::memcpy(name, s.c_str(), s.size() + 1);
+    return VTI_OK;
+}
+
 int vti_calib_copy(void *dst, const void *src, size_t nbytes, void *stream)
 {
     if (!dst || !src) return fail(VTI_ERR_ARG, "vti_calib_copy: null pointer");

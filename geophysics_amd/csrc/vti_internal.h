@@ -92,6 +92,8 @@ struct FusedArgs {
 hipError_t launch_fused(const FusedArgs &a, hipStream_t s);
 hipError_t launch_vel(int ndim, const VelArgs &a, hipStream_t s);
 hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s);
+// the kernel that launch_stress takes for a 3D grid (without a snapshot copy)
+std::string stress3d_name(const Grid &g, bool us);
 hipError_t launch_pad_model(const Grid &g, int ndim, int nx, int ny, int nz,
                             int npml, const float *src, float *dst, hipStream_t s);
 hipError_t launch_zero(float *p, size_t n, hipStream_t s);

@@ -401,6 +401,16 @@ hipError_t launch_fused(const FusedArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+// the form of a stress update: planes a chunk and what bypasses the caches
+struct Stress3dForm {
+    int chunk, stream;
+};
+inline Stress3dForm stress3d_form_of(const Grid &g, bool us)
+{
+    const int stream = stream_stress(g, us);
+    return Stress3dForm{!us && stream == 1 && field_mb(g) > 500.0 ? kSplitChunk : kStressChunk, stream};
+}
+
 template <int CH, int NT>
 void stress3d_form(const StressArgs &a, bool us, hipStream_t s)
 {
@@ -422,16 +432,20 @@ hipError_t launch_stress(int ndim, const StressArgs &a, hipStream_t s)
         else hipLaunchKernelGGL((stress2d_kernel<false, false>), grd, blk, 0, s, a);
     } else {
         const bool us = a.unsplit && !a.gsrc;
-        switch (stream_stress(a.g, us)) {
-        case 0: stress3d_form<kStressChunk, 0>(a, us, s); break;
-        case 1:
-            if (us || field_mb(a.g) <= 500.0) stress3d_form<kStressChunk, 1>(a, us, s);
-            else stress3d_form<kSplitChunk, 1>(a, us, s);
-            break;
-        default: stress3d_form<kStressChunk, 2>(a, us, s);
-        }
+        const Stress3dForm f = stress3d_form_of(a.g, us);
+        if (f.chunk == kSplitChunk) stress3d_form<kSplitChunk, 1>(a, us, s);
+        else if (f.stream == 0) stress3d_form<kStressChunk, 0>(a, us, s);
+        else if (f.stream == 1) stress3d_form<kStressChunk, 1>(a, us, s);
+        else stress3d_form<kStressChunk, 2>(a, us, s);
     }
     return hipGetLastError();
+}
+
+std::string stress3d_name(const Grid &g, bool us)
+{
+    const Stress3dForm f = stress3d_form_of(g, us);
+    return "vti::s3d::stress3d<" + std::to_string(f.chunk) + ", " + std::to_string(f.stream) + (us ? ", true" : ", false") +
+           ", false>";
 }
 
 hipError_t launch_pad_model(const Grid &g, int ndim, int nx, int ny, int nz, int npml,

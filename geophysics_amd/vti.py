@@ -109,6 +109,7 @@ def _declare(L):
         "vti_get_table": (C.c_int, [VP, C.c_int, FP]),
         "vti_padded_dims": (C.c_int, [VP, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]),
         "vti_prof_enable": (C.c_int, [VP, C.c_int]),
+        "vti_stress3d_name": (C.c_int, [C.POINTER(Cfg), C.c_int, C.c_char_p, C.c_int]),
         "vti_set_fused": (C.c_int, [VP, C.c_int]),
         "vti_set_unsplit": (C.c_int, [VP, C.c_int]),
         "vti_batch_set_unsplit": (C.c_int, [VP, C.c_int]),
@@ -258,6 +259,13 @@ def sweep_check(nt, nslot):
     steps, slots = C.c_longlong(), C.c_int()
     check(lib().vti_sweep_check(nt, nslot, C.byref(steps), C.byref(slots)), "sweep_check")
     return steps.value, slots.value
+
+
+def stress3d_name(cfg, unsplit):
+    """Name of the stress kernel of a 3D configuration, as a profiler shows it."""
+    name = C.create_string_buffer(128)
+    check(lib().vti_stress3d_name(C.byref(cfg), int(unsplit), name, len(name)), "stress3d_name")
+    return name.value.decode()
 
 
 def resident_launches():

@@ -616,6 +616,10 @@ int vti_set_fused(vti_ctx *ctx, int on);
  * events on the context stream; vti_prof_read sums them (ms).  A fused 3D
  * step counts entirely as stress time. */
 int vti_prof_enable(vti_ctx *ctx, int on);
+/* Name of the stress kernel that the steps of a 3D configuration launch, as a
+ * profiler shows it: the rules on the grid's size choose its chunk length and
+ * what bypasses the caches (host only, no device needed). */
+int vti_stress3d_name(const vti_cfg *cfg, int unsplit, char *name, int size);
 int vti_prof_read(vti_ctx *ctx, double *vel_ms, double *stress_ms, int *nlaunch);
 /* Plain device copy of nbytes (bandwidth calibration kernel). */
 int vti_calib_copy(void *dst, const void *src, size_t nbytes, void *hip_stream);
