@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -1030,10 +1031,17 @@ bool capturing(hipStream_t s)
 thread_local long long t_launches = 0;   // vti_resident_launches
 thread_local long long t_left = -1;      // vti_resident_limit
 thread_local unsigned t_wait = kWaitTicks;   // vti_resident_wait
+thread_local std::chrono::steady_clock::time_point t_again{};   // no launch before
 
 hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     if (t_left == 0) return hipErrorOutOfMemory;
+    // While another process has resident kernels on the device, the runtime
+    // may refuse one, and takes 80 to 200 ms to say so; a refusal that took long
+    // is not asked for again until twenty times as long has passed.
+    using clock = std::chrono::steady_clock;
+    const clock::time_point begin = clock::now();
+    if (begin < t_again) return hipErrorOutOfMemory;
     a.wait = t_wait;
     void *args[] = {&a};
     // The function's own limit, which its callers in all threads share: always
@@ -1051,6 +1059,8 @@ hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, h
         e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        const clock::time_point end = clock::now();
+        if (end - begin > std::chrono::milliseconds(1)) t_again = end + 20 * (end - begin);
         return e;
     }
     ++t_launches;

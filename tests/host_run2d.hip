@@ -9,6 +9,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <thread>
 
 #include "../geophysics_amd/csrc/vti_run2d.hip"
 
@@ -30,6 +31,7 @@ static std::vector<Launched> g_launched;
 static std::map<const void *, int> g_lds_max;       // the attribute of each function
 static std::function<void()> g_after_attribute;     // what another thread does after this one's set
 static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
+static int g_asked = 0, g_refuse_ms = 0;              // launches asked for, what a refusal takes
 static bool g_no_memory = false;
 static int g_cus = 256, g_lds = 163840;
 
@@ -81,10 +83,14 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v)
 }
 hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3 b, void **, unsigned lds, hipStream_t)
 {
+    ++g_asked;
     if (!g_refuse.empty()) {
         const hipError_t e = g_refuse.front();
         g_refuse.erase(g_refuse.begin());
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            std::this_thread::sleep_for(std::chrono::milliseconds(g_refuse_ms));
+            return e;
+        }
     }
     if (!g_lds_max.count(f) || (int)lds > g_lds_max[f] || (int)lds > g_lds) return hipErrorInvalidValue;
     if ((int)g.x > g_cus) return hipErrorCooperativeLaunchTooLarge;
@@ -147,6 +153,22 @@ void refused_step()
     g_refuse = {hipErrorCooperativeLaunchTooLarge};
     CHECK(run2d_steps(&c, 0, 16) == 0);
     CHECK(run2d_steps(&c, 16, 16) == 0 && g_launched.size() == 1);
+}
+
+// A refusal that takes long is not asked for again at once.
+void slow_refusal()
+{
+    Ctx c(440, 440);
+    CHECK(run2d_steps(&c, 0, 32) == 1);
+    g_refuse = {hipErrorOutOfMemory};
+    g_refuse_ms = 20;
+    CHECK(run2d_steps(&c, 0, 32) == 0 && g_asked == 2);
+    for (int k = 0; k < 5; ++k) CHECK(run2d_steps(&c, 0, 32) == 0 && g_asked == 2);
+    int other = 0;      // another thread has not been refused
+    std::thread([&] { other = run2d_steps(&c, 0, 32); }).join();
+    CHECK(other == 1 && g_asked == 3);
+    std::this_thread::sleep_for(std::chrono::milliseconds(1000));
+    CHECK(run2d_steps(&c, 0, 32) == 1 && g_asked == 4);
 }
 
 struct Group : Run2dGroup {   // shots of two parts
@@ -339,6 +361,7 @@ void plans()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step},
+                                                       {"slow_refusal", vti::slow_refusal},
                                                        {"refused_program", vti::refused_program},
                                                        {"missed_exchange", vti::missed_exchange},
                                                        {"plans", vti::plans}};
