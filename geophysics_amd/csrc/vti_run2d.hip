@@ -163,7 +163,7 @@ struct Wait {
     __device__ __forceinline__ bool over(unsigned t0) const
     {
         const unsigned d = (unsigned)wall_clock64() - t0;
-        if (d < min(kLookTicks, limit)) return false;
+        if (__builtin_expect(d < min(kLookTicks, limit), 1)) return false;
         if (d <= limit && !__hip_atomic_load(dead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) &&
             !__hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
             return false;
