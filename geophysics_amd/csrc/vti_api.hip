@@ -432,6 +432,7 @@ int vti_set_stream(vti_ctx *c, void *s)
 {
     if (!c) return fail(VTI_ERR_ARG, "vti_set_stream: null ctx");
     HIP_TRY(hipStreamSynchronize(c->stream));
+    run2d_leave(c);
     if (c->own_stream && c->stream) hipStreamDestroy(c->stream);
     if (s) {
         c->stream = static_cast<hipStream_t>(s);

@@ -229,5 +229,6 @@ hipError_t launch_adcig(vti_ctx *c, const VtiState &src, const VtiState &rcv);
 // work on the state, before it
 int run2d_steps(vti_ctx *c, int it0, int n);
 void run2d_free(vti_ctx *c);
+void run2d_leave(vti_ctx *c);   // the context's stream has been waited for and is left
 int run2d_check(vti_ctx *c);
 }  // namespace vti

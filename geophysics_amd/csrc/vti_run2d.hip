@@ -29,17 +29,23 @@
 // (update_vel2d GPU_vti2dfd_kernels.cu:209-238, update_stress2d :240-299,
 // CPU_vti2dfd_kernels.c:78-177, Toa_gpu_2dtti_fd_1orderfunction.cu:81-183).
 //
-// Launch: cooperative (all workgroups resident, or the launch fails and the
-// per-step kernels run).  Every wait ends: a tile that misses a sample for
-// kWaitTicks raises the error word and leaves its loop, and the others, which
-// look at the word while they wait, follow it within milliseconds.
+// Launch: all workgroups get a place on the chip and no other resident launch
+// is under way (Chip, below), or the per-step kernels run.  Every wait ends: a
+// tile that misses a sample for kWaitTicks raises the error word and leaves its
+// loop, and the others, which look at the word while they wait, follow it within
+// milliseconds.
 #include <hip/hip_runtime.h>
 
+#include <sys/socket.h>
+#include <sys/un.h>
+#include <unistd.h>
+
 #include <algorithm>
-#include <chrono>
+#include <cstddef>
 #include <cstdint>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <new>
 #include <queue>
 #include <string>
@@ -900,9 +906,7 @@ struct Device2d {
 };
 bool device_2d(int device, Device2d &d)
 {
-    int coop = 0;
-    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !coop ||
-        hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+    if (hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         hipDeviceGetAttribute(&d.lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) {
         (void)hipGetLastError();
         return false;
@@ -1031,17 +1035,121 @@ bool capturing(hipStream_t s)
 thread_local long long t_launches = 0;   // vti_resident_launches
 thread_local long long t_left = -1;      // vti_resident_limit
 thread_local unsigned t_wait = kWaitTicks;   // vti_resident_wait
-thread_local std::chrono::steady_clock::time_point t_again{};   // no launch before
 
-hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
+// The resident launches on one device.  The workgroups of a launch wait for
+// each other, one a CU at most: they all get a place once the kernels before
+// them and beside them end, unless another resident launch holds some of the
+// places and waits for the rest.  So no two are ever under way at once: those of
+// this process follow each other (one stream's by themselves, those of several
+// streams by events), and a process has the device's resident launches to itself
+// while an object that makes them lives (a name in the abstract socket
+// namespace, which the kernel takes back when the process ends); the others run
+// the per-step kernels.
+// A cooperative launch promises the same, on a hardware queue of its own, the
+// fifth of a process with four.  Two queues then share a pipe, and while both
+// have work every launch on either takes ~25 us instead of 3, also long after
+// the cooperative one: gradients of 60 x 50, 200 steps, in 8 threads took 20 ms
+// before the process's first cooperative launch and 73 after it.
+struct Chip {
+    std::mutex m;
+    std::string id;                      // of the device, the same in every process
+    int name = -1;                       // the socket bound to it
+    std::map<hipStream_t, int> streams;  // of the objects that launch here
+    hipStream_t last = nullptr;          // of the latest launch that may be under way
+    hipEvent_t done = nullptr;           // after it, where there are several streams
+};
+Chip &chip_of(int device)
+{
+    static std::mutex m;
+    static auto *all = new std::map<int, Chip>;   // outlives every thread
+    const std::lock_guard<std::mutex> l(m);
+    return (*all)[device];
+}
+
+bool take_device(Chip &c, int device)
+{
+    if (c.name >= 0) return true;
+    if (c.id.empty()) {
+        char pci[32] = "";
+        hipUUID u{};
+        hipDevice_t d;
+        if (hipDeviceGetPCIBusId(pci, sizeof pci, device) != hipSuccess || hipDeviceGet(&d, device) != hipSuccess ||
+            hipDeviceGetUuid(&u, d) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        c.id = std::string("vti-resident-") + pci + "-";
+        for (const char b : u.bytes) {
+            c.id += "0123456789abcdef"[b >> 4 & 15];
+            c.id += "0123456789abcdef"[b & 15];
+        }
+    }
+    sockaddr_un a{};
+    a.sun_family = AF_UNIX;   // sun_path[0] stays 0: no file
+    c.id.copy(a.sun_path + 1, sizeof a.sun_path - 1);
+    const size_t n = offsetof(sockaddr_un, sun_path) + 1 + std::min(c.id.size(), sizeof a.sun_path - 1);
+    const int fd = socket(AF_UNIX, SOCK_STREAM | SOCK_CLOEXEC, 0);
+    if (fd < 0) return false;
+    if (bind(fd, reinterpret_cast<sockaddr *>(&a), (socklen_t)n)) {
+        close(fd);
+        return false;
+    }
+    c.name = fd;
+    return true;
+}
+
+// the latest launch, waited for by events from here on, or here
+void note(Chip &c)
+{
+    if (!c.last) return;
+    const RelaxedCapture relaxed;
+    if ((!c.done && hipEventCreateWithFlags(&c.done, hipEventDisableTiming) != hipSuccess) ||
+        hipEventRecord(c.done, c.last) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(c.last);
+        c.last = nullptr;
+    }
+}
+
+// An object that launches on s: false: not on this stream (one that may not use
+// all CUs).
+bool chip_enter(int device, hipStream_t s)
+{
+    Device2d d;
+    if (!device_2d(device, d)) return false;
+    uint32_t mask[64] = {};
+    if (hipExtStreamGetCUMask(s, 64, mask) == hipSuccess) {
+        int n = 0;
+        for (const uint32_t w : mask) n += __builtin_popcount(w);
+        if (n < d.cus) return false;
+    } else {
+        (void)hipGetLastError();
+    }
+    Chip &c = chip_of(device);
+    const std::lock_guard<std::mutex> l(c.m);
+    const bool one = c.streams.size() == 1;
+    ++c.streams[s];
+    if (one && c.streams.size() > 1) note(c);
+    return true;
+}
+// its launches have been waited for
+void chip_leave(int device, hipStream_t s)
+{
+    Chip &c = chip_of(device);
+    const std::lock_guard<std::mutex> l(c.m);
+    const auto i = c.streams.find(s);
+    if (i == c.streams.end() || --i->second) return;
+    c.streams.erase(i);
+    if (c.last == s) c.last = nullptr;
+    if (c.streams.empty() && c.name >= 0) {
+        close(c.name);
+        c.name = -1;
+    }
+}
+
+hipError_t launch_resident(int device, KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
 {
     if (t_left == 0) return hipErrorOutOfMemory;
-    // While another process has resident kernels on the device, the runtime
-    // may refuse one, and takes 80 to 200 ms to say so; a refusal that took long
-    // is not asked for again until twenty times as long has passed.
-    using clock = std::chrono::steady_clock;
-    const clock::time_point begin = clock::now();
-    if (begin < t_again) return hipErrorOutOfMemory;
     a.wait = t_wait;
     void *args[] = {&a};
     // The function's own limit, which its callers in all threads share: always
@@ -1053,16 +1161,21 @@ hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, h
             (void)hipGetLastError();
         return n;
     }();
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       std::max((int)lds, lds_max - (int)kStaticLds));
+    Chip &c = chip_of(device);
+    const std::lock_guard<std::mutex> l(c.m);
+    if (!take_device(c, device)) return hipErrorNotReady;
+    hipError_t e = hipSuccess;
+    if (c.last && c.last != s) e = hipStreamWaitEvent(s, c.done, 0);
     if (e == hipSuccess)
-        e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, (unsigned)lds, s);
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                std::max((int)lds, lds_max - (int)kStaticLds));
+    if (e == hipSuccess) e = hipLaunchKernel(reinterpret_cast<const void *>(k), dim3(grid), dim3(nt), args, lds, s);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        const clock::time_point end = clock::now();
-        if (end - begin > std::chrono::milliseconds(1)) t_again = end + 20 * (end - begin);
         return e;
     }
+    c.last = s;
+    if (c.streams.size() > 1) note(c);
     ++t_launches;
     if (t_left > 0) --t_left;
     return e;
@@ -1071,6 +1184,9 @@ hipError_t launch_coop(KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, h
 }  // namespace
 
 struct Run2dPlan {
+    int device = 0;
+    bool entered = false;       // on this stream
+    hipStream_t stream = nullptr;
     int ok = 0;                 // 1: usable, 0: not planned yet, -1: this grid or device takes the per-step kernels
     std::vector<Run2dShot> shot;   // one: the plan's share of it
     int shape = 0, ntile = 0;
@@ -1084,10 +1200,18 @@ struct Run2dPlan {
 void run2d_free(vti_ctx *c)
 {
     if (!c->run2d) return;
-    (void)hipFree(c->run2d->xbuf);
+    (void)hipFree(c->run2d->xbuf);   // waits for the device
     (void)hipHostFree(c->run2d->dead);
+    run2d_leave(c);
     delete c->run2d;
     c->run2d = nullptr;
+}
+
+void run2d_leave(vti_ctx *c)
+{
+    if (!c->run2d || !c->run2d->entered) return;
+    chip_leave(c->run2d->device, c->run2d->stream);
+    c->run2d->entered = false;
 }
 
 // The forward side of a context's shot on state s.
@@ -1168,13 +1292,12 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     const bool us = c->unsplit && c->cfg.mode == VTI_MODE_GPU_REF && !tti;
     const KernelFn k = tti ? kernel_of<true, false, false>(p.shape)
                            : (us ? kernel_of<false, true, false>(p.shape) : kernel_of<false, false, false>(p.shape));
-    const hipError_t e = launch_coop(k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream);
-    if (e != hipSuccess) {
-        // a launch that the device cannot hold never will be; another cause
-        // (scratch or queue memory) may be gone at the next call
-        if (e == hipErrorCooperativeLaunchTooLarge) p.ok = -1;
-        return 0;
-    }
+    if (!p.entered && !chip_enter(c->device, c->stream)) return 0;
+    p.entered = true;
+    p.device = c->device;
+    p.stream = c->stream;
+    // another process has the device, no memory: the next call tries again
+    if (launch_resident(p.device, k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream) != hipSuccess) return 0;
     p.base += (unsigned)n;
     if (us) c->us_dirty = true;
     return 1;
@@ -1256,6 +1379,10 @@ int run2d_group_make(Run2dGroup &g, const Run2dParts &p, std::vector<Run2dShot> 
 {
     g.ok = 0;
     if (p.part.empty() || capturing(s)) return 0;
+    if (hipGetDevice(&g.device) != hipSuccess) return fail(VTI_ERR_HIP, "run2d: device");
+    if (!chip_enter(g.device, s)) return 0;
+    g.entered = true;
+    g.stream = s;
     g.parts = p;
     g.us = us;
     g.words = 0;
@@ -1296,8 +1423,9 @@ int run2d_group_set(Run2dGroup &g, std::vector<Run2dShot> shots, hipStream_t s)
 
 void run2d_group_free(Run2dGroup &g)
 {
-    (void)hipFree(g.mem);
+    (void)hipFree(g.mem);   // waits for the device
     (void)hipFree(g.more);
+    if (g.entered) chip_leave(g.device, g.stream);
     g = Run2dGroup{};
 }
 
@@ -1338,10 +1466,8 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         a.base = g.base;
         a.dead = g.dead;
         const KernelFn k = g.us ? kernel_of<false, true, true>(q.shape) : kernel_of<false, false, true>(q.shape);
-        const hipError_t e = launch_coop(k, q.ntile, kShapes[q.shape].nt, q.lds, a, s);
-        if (e != hipSuccess) {
+        if (launch_resident(g.device, k, q.ntile, kShapes[q.shape].nt, q.lds, a, s) != hipSuccess) {
             g.refused = true;
-            if (e == hipErrorCooperativeLaunchTooLarge) g.ok = -1;
             return &q == &g.parts.part.front() ? 0 : 2;
         }
         g.ran = true;

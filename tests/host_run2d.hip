@@ -31,7 +31,8 @@ static std::vector<Launched> g_launched;
 static std::map<const void *, int> g_lds_max;       // the attribute of each function
 static std::function<void()> g_after_attribute;     // what another thread does after this one's set
 static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
-static int g_asked = 0, g_refuse_ms = 0;              // launches asked for, what a refusal takes
+static std::vector<std::string> g_order;            // launches, events and waits, with their streams
+static int g_mask = 256;                            // CUs that a stream may use
 static bool g_no_memory = false;
 static int g_cus = 256, g_lds = 163840;
 
@@ -41,7 +42,6 @@ void **__hipRegisterFatBinary(const void *) { return nullptr; }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n) { return !g_no_memory && (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipFree(void *p)
@@ -81,20 +81,53 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v)
     if (other) other();
     return hipSuccess;
 }
-hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3 b, void **, unsigned lds, hipStream_t)
+static std::string named(const char *what, hipStream_t s) { return what + std::to_string((size_t)s); }
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t lds, hipStream_t s)
 {
-    ++g_asked;
     if (!g_refuse.empty()) {
         const hipError_t e = g_refuse.front();
         g_refuse.erase(g_refuse.begin());
-        if (e != hipSuccess) {
-            std::this_thread::sleep_for(std::chrono::milliseconds(g_refuse_ms));
-            return e;
-        }
+        if (e != hipSuccess) return e;
     }
     if (!g_lds_max.count(f) || (int)lds > g_lds_max[f] || (int)lds > g_lds) return hipErrorInvalidValue;
-    if ((int)g.x > g_cus) return hipErrorCooperativeLaunchTooLarge;
     g_launched.push_back({f, (int)g.x, (int)b.x, lds});
+    g_order.push_back(named("launch ", s));
+    return hipSuccess;
+}
+hipError_t hipExtStreamGetCUMask(hipStream_t, uint32_t n, uint32_t *m)
+{
+    for (int k = 0; k < (int)n * 32; ++k)
+        if (k < g_mask) m[k / 32] |= 1u << k % 32;
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = reinterpret_cast<hipEvent_t>(1);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t s)
+{
+    g_order.push_back(named("record ", s));
+    return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned)
+{
+    g_order.push_back(named("wait ", s));
+    return hipSuccess;
+}
+hipError_t hipDeviceGetPCIBusId(char *p, int n, int)
+{
+    std::snprintf(p, n, "host-%d", (int)getpid());   // no device's
+    return hipSuccess;
+}
+hipError_t hipDeviceGet(hipDevice_t *d, int)
+{
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetUuid(hipUUID *u, hipDevice_t)
+{
+    *u = hipUUID{};
     return hipSuccess;
 }
 }
@@ -130,45 +163,95 @@ struct Ctx : vti_ctx {   // a 2D context, its padded size
 };
 
 // Two threads whose tiles of one kernel need different amounts of LDS: the
-// smaller one's launch comes between the larger one's attribute and launch.
+// smaller one's launch comes, if it can, between the larger one's attribute and
+// launch.
 void lds_attribute()
 {
     Ctx large(1440, 543), small(1340, 543);
     int r = -1;
-    g_after_attribute = [&] { r = run2d_steps(&small, 0, 32); };
+    std::thread other;
+    g_after_attribute = [&] {
+        other = std::thread([&] { r = run2d_steps(&small, 0, 32); });
+        std::this_thread::sleep_for(std::chrono::milliseconds(200));
+    };
     const int q = run2d_steps(&large, 0, 32);
-    CHECK(r == 1 && g_launched.size() >= 1);
-    CHECK(q == 1 && g_launched.size() == 2);
-    CHECK(g_launched[0].kernel == g_launched[1].kernel && g_launched[0].lds < g_launched[1].lds);
+    other.join();
+    CHECK(q == 1 && r == 1 && g_launched.size() == 2);
+    CHECK(g_launched[0].kernel == g_launched[1].kernel && g_launched[0].lds != g_launched[1].lds);
+    for (const auto &m : g_lds_max) CHECK(m.second == g_lds - (int)kStaticLds);
 }
 
-// A refused launch leaves that call to the per-step kernels and no later one,
-// unless the device can never hold it.
+// A refused launch leaves that call to the per-step kernels and no later one.
 void refused_step()
 {
     Ctx c(440, 440);
     g_refuse = {hipErrorOutOfMemory};
     CHECK(run2d_steps(&c, 0, 32) == 0);
     CHECK(run2d_steps(&c, 32, 16) == 1 && g_launched.size() == 1);
-    g_refuse = {hipErrorCooperativeLaunchTooLarge};
-    CHECK(run2d_steps(&c, 0, 16) == 0);
-    CHECK(run2d_steps(&c, 16, 16) == 0 && g_launched.size() == 1);
 }
 
-// A refusal that takes long is not asked for again at once.
-void slow_refusal()
+hipStream_t stream(int k) { return reinterpret_cast<hipStream_t>((size_t)k); }
+
+// No two resident launches under way at once: those of one stream follow each
+// other by themselves, without events; those of several by events, the launch
+// that was under way when the second stream came included; a stream that its
+// context has left is not touched again.
+void launch_order()
 {
+    using Order = std::vector<std::string>;
+    Ctx a(440, 440), c(240, 240);
+    a.stream = stream(1);
+    c.stream = stream(1);
+    CHECK(run2d_steps(&a, 0, 32) == 1 && run2d_steps(&c, 0, 32) == 1 && run2d_steps(&a, 0, 32) == 1);
+    CHECK((g_order == Order{"launch 1", "launch 1", "launch 1"}));
+    {
+        Ctx b(440, 440);
+        b.stream = stream(2);
+        g_order.clear();
+        CHECK(run2d_steps(&b, 0, 32) == 1 && run2d_steps(&b, 0, 32) == 1);
+        CHECK((g_order == Order{"record 1", "wait 2", "launch 2", "record 2", "launch 2", "record 2"}));
+        g_order.clear();
+        CHECK(run2d_steps(&c, 0, 32) == 1);
+        CHECK((g_order == Order{"wait 1", "launch 1", "record 1"}));
+        run2d_leave(&b);            // vti_set_stream
+        b.stream = stream(3);
+        g_order.clear();
+        CHECK(run2d_steps(&a, 0, 32) == 1 && run2d_steps(&b, 0, 32) == 1);
+        CHECK((g_order == Order{"launch 1", "record 1", "wait 3", "launch 3", "record 3"}));
+    }
+    g_order.clear();                // stream 3 has gone
+    CHECK(run2d_steps(&a, 0, 32) == 1);
+    CHECK((g_order == Order{"launch 1"}));
+}
+
+// Another process that has the device's resident launches (its name, bound
+// here), and a stream that may not use all CUs: the per-step kernels.
+void shared_device()
+{
+    sockaddr_un n{};
+    n.sun_family = AF_UNIX;
+    const int len = std::snprintf(n.sun_path + 1, sizeof n.sun_path - 1, "vti-resident-host-%d-%032d", (int)getpid(), 0);
+    const int fd = socket(AF_UNIX, SOCK_STREAM, 0);
+    const socklen_t size = (socklen_t)(offsetof(sockaddr_un, sun_path) + 1 + len);
+    auto held = [&] { return bind(fd, reinterpret_cast<sockaddr *>(&n), size) != 0; };
+    CHECK(!held());
+    Ctx a(440, 440);
+    CHECK(run2d_steps(&a, 0, 32) == 0 && g_launched.empty());
+    close(fd);
+    CHECK(run2d_steps(&a, 0, 32) == 1);
+    {
+        Ctx b(440, 440);
+        CHECK(run2d_steps(&b, 0, 32) == 1);
+        run2d_free(&a);
+    }
+    const int again = socket(AF_UNIX, SOCK_STREAM, 0);    // given back with the last object
+    CHECK(bind(again, reinterpret_cast<sockaddr *>(&n), size) == 0);
+    close(again);
+    g_mask = 255;
     Ctx c(440, 440);
+    CHECK(run2d_steps(&c, 0, 32) == 0);
+    g_mask = 256;
     CHECK(run2d_steps(&c, 0, 32) == 1);
-    g_refuse = {hipErrorOutOfMemory};
-    g_refuse_ms = 20;
-    CHECK(run2d_steps(&c, 0, 32) == 0 && g_asked == 2);
-    for (int k = 0; k < 5; ++k) CHECK(run2d_steps(&c, 0, 32) == 0 && g_asked == 2);
-    int other = 0;      // another thread has not been refused
-    std::thread([&] { other = run2d_steps(&c, 0, 32); }).join();
-    CHECK(other == 1 && g_asked == 3);
-    std::this_thread::sleep_for(std::chrono::milliseconds(1000));
-    CHECK(run2d_steps(&c, 0, 32) == 1 && g_asked == 4);
 }
 
 struct Group : Run2dGroup {   // shots of two parts
@@ -360,8 +443,10 @@ void plans()
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute}, {"refused_step", vti::refused_step},
-                                                       {"slow_refusal", vti::slow_refusal},
+    const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute},
+                                                       {"refused_step", vti::refused_step},
+                                                       {"launch_order", vti::launch_order},
+                                                       {"shared_device", vti::shared_device},
                                                        {"refused_program", vti::refused_program},
                                                        {"missed_exchange", vti::missed_exchange},
                                                        {"plans", vti::plans}};

@@ -56,3 +56,31 @@ def test_three_processes():
     out = [r.communicate(timeout=100)[0] for r in run]
     print("\n".join(out), flush=True)
     assert all(r.returncode == 0 and "equal" in o for r, o in zip(run, out)), out
+
+
+def test_one_process_at_a_time():
+    """While an object of one process makes resident launches, those of another
+    are refused at once; they are resident when it has gone."""
+    from geophysics_amd import vti
+    from test_gpu_run2d_path import Launches, build
+    code = ("import sys; sys.path[:0] = [%r, %r]\n"
+            "from test_gpu_run2d_path import build, vti\n"
+            "with build('gpu', 120, 90, 20, 200) as p:\n"
+            "    p.step(0, 200); p.sync(); print(vti.resident_launches(), flush=True); sys.stdin.readline()\n"
+            % (ROOT, os.path.join(ROOT, "tests")))
+    r = subprocess.Popen([sys.executable, "-c", code], stdin=subprocess.PIPE, stdout=subprocess.PIPE,
+                         stderr=subprocess.DEVNULL, text=True)
+    try:
+        assert r.stdout.readline().strip() == "1"
+        with build("gpu", 120, 90, 20, 200) as p, Launches() as n:
+            p.step(0, 200)
+            rec = p.record()
+            assert n() == 0
+            r.communicate("\n", timeout=60)
+            assert r.returncode == 0
+            p.reset()
+            p.step(0, 200)
+            assert n() == 1 and np.array_equal(p.record(), rec)
+    finally:
+        r.kill()
+        r.wait()
