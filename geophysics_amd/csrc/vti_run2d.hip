@@ -1111,6 +1111,20 @@ void note(Chip &c)
     }
 }
 
+// A short call does not wait for another stream's launch: the per-step kernels
+// run beside it.  ms for 400 steps of a context, 8 threads, per-step kernels /
+// waiting / this rule, in calls of 8, 16, 24, 32 steps: 60 x 50 0.97, 1.29, 0.86 /
+// 0.96, 1.00, 0.89 / 0.96, 0.91, 0.91 / 0.96, 0.86, 0.87; 400 x 400 1.65, 2.04,
+// 1.60 / 1.65, 1.64, 1.59 / 1.65, 1.52, 1.50 / 1.66, 1.45, 1.43.
+constexpr int kShareSteps = 24;
+bool under_way(const Chip &c)
+{
+    const RelaxedCapture relaxed;
+    const bool yes = hipEventQuery(c.done) == hipErrorNotReady;
+    (void)hipGetLastError();
+    return yes;
+}
+
 // An object that launches on s: false: not on this stream (one that may not use
 // all CUs).
 bool chip_enter(int device, hipStream_t s)
@@ -1147,7 +1161,7 @@ void chip_leave(int device, hipStream_t s)
     }
 }
 
-hipError_t launch_resident(int device, KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, hipStream_t s)
+hipError_t launch_resident(int device, KernelFn k, int grid, int nt, size_t lds, Run2dArgs &a, int steps, hipStream_t s)
 {
     if (t_left == 0) return hipErrorOutOfMemory;
     a.wait = t_wait;
@@ -1165,7 +1179,10 @@ hipError_t launch_resident(int device, KernelFn k, int grid, int nt, size_t lds,
     const std::lock_guard<std::mutex> l(c.m);
     if (!take_device(c, device)) return hipErrorNotReady;
     hipError_t e = hipSuccess;
-    if (c.last && c.last != s) e = hipStreamWaitEvent(s, c.done, 0);
+    if (c.last && c.last != s) {
+        if (steps < kShareSteps && under_way(c)) return hipErrorNotReady;
+        e = hipStreamWaitEvent(s, c.done, 0);
+    }
     if (e == hipSuccess)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 std::max((int)lds, lds_max - (int)kStaticLds));
@@ -1246,17 +1263,16 @@ Run2dShot run2d_shot(vti_ctx *c, const VtiState &s)
 int run2d_steps(vti_ctx *c, int it0, int n)
 {
     // Two steps let the write-back start after every neighbour has loaded.
-    // Below eight the call's fixed cost (launch, the tile's coefficients, load
-    // and store: 25 us at 60 x 50, 55 at 2401 x 803) is what the per-step kernels
-    // take: us a call of 8 / 10 / 16 steps among others, per-step and resident,
-    // 200 x 150 46, 41 / 58, 45 / 91, 56; 400 x 400 58, 53 / 72, 59 / 114, 76;
-    // 2401 x 803 222, 139 / 281, 160 / 460, 224.
+    // Eight are the fewest that were measured, and faster: us a call of 8 / 10 /
+    // 16 steps among others, per-step kernels and resident, 200 x 150 46, 24 /
+    // 58, 27 / 91, 39; 400 x 400 58, 36 / 72, 42 / 114, 60; 2401 x 803 222, 122 /
+    // 281, 143 / 460, 205.
     if (c->cfg.ndim != 2 || c->cfg.mode == VTI_MODE_OMP_REF || capturing(c->stream)) return 0;
     // The plan and its memory cost a context's first such call 60 to 400 us, a
     // step saves 4 to 18: us of a fresh context's first call of 16 / 24 / 32
-    // steps, per-step and resident, 200 x 150 106, 108 / 149, 121 / 197, 141;
-    // 601 x 301 139, 167 / 202, 194 / 266, 219; 1401 x 503 254, 457 / 370, 508 /
-    // 488, 535; 2401 x 803 532, 630 / 782, 698 / 1033, 792.
+    // steps, per-step kernels and resident, 200 x 150 106, 108 / 149, 130 / 197,
+    // 132; 400 x 400 126, 155 / 183, 189 / 240, 207; 1401 x 503 254, 457 / 370,
+    // 226 / 488, 270; 2401 x 803 532, 630 / 782, 475 / 1033, 535.
     if (!c->run2d) c->asked2d += n;
     if (n < 8 || (!c->run2d && c->asked2d < 24)) return 0;
     const bool tti = c->tti != nullptr;
@@ -1297,7 +1313,7 @@ int run2d_steps(vti_ctx *c, int it0, int n)
     p.device = c->device;
     p.stream = c->stream;
     // another process has the device, no memory: the next call tries again
-    if (launch_resident(p.device, k, p.ntile, kShapes[p.shape].nt, p.lds, a, c->stream) != hipSuccess) return 0;
+    if (launch_resident(p.device, k, p.ntile, kShapes[p.shape].nt, p.lds, a, n, c->stream) != hipSuccess) return 0;
     p.base += (unsigned)n;
     if (us) c->us_dirty = true;
     return 1;
@@ -1466,7 +1482,7 @@ int run2d_group_run(Run2dGroup &g, const std::vector<Run2dOp> &ops, const std::v
         a.base = g.base;
         a.dead = g.dead;
         const KernelFn k = g.us ? kernel_of<false, true, true>(q.shape) : kernel_of<false, false, true>(q.shape);
-        if (launch_resident(g.device, k, q.ntile, kShapes[q.shape].nt, q.lds, a, s) != hipSuccess) {
+        if (launch_resident(g.device, k, q.ntile, kShapes[q.shape].nt, q.lds, a, kShareSteps, s) != hipSuccess) {
             g.refused = true;
             return &q == &g.parts.part.front() ? 0 : 2;
         }

@@ -32,6 +32,7 @@ static std::map<const void *, int> g_lds_max;       // the attribute of each fun
 static std::function<void()> g_after_attribute;     // what another thread does after this one's set
 static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
 static std::vector<std::string> g_order;            // launches, events and waits, with their streams
+static bool g_busy = false;                         // the latest noted launch is under way
 static int g_mask = 256;                            // CUs that a stream may use
 static bool g_no_memory = false;
 static int g_cus = 256, g_lds = 163840;
@@ -110,6 +111,7 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t s)
     g_order.push_back(named("record ", s));
     return hipSuccess;
 }
+hipError_t hipEventQuery(hipEvent_t) { return g_busy ? hipErrorNotReady : hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned)
 {
     g_order.push_back(named("wait ", s));
@@ -222,6 +224,22 @@ void launch_order()
     g_order.clear();                // stream 3 has gone
     CHECK(run2d_steps(&a, 0, 32) == 1);
     CHECK((g_order == Order{"launch 1"}));
+}
+
+// A short call does not wait for another stream's launch, a long one and a
+// program do.
+void short_calls()
+{
+    Ctx a(440, 440), b(440, 440);
+    a.stream = stream(1);
+    b.stream = stream(2);
+    CHECK(run2d_steps(&a, 0, 32) == 1 && run2d_steps(&b, 0, 32) == 1);
+    g_busy = true;
+    CHECK(run2d_steps(&a, 0, 23) == 0 && run2d_steps(&b, 0, 23) == 1);   // b's own
+    g_order.clear();
+    CHECK(run2d_steps(&a, 0, 24) == 1 && g_order.front() == "wait 1");
+    g_busy = false;
+    CHECK(run2d_steps(&b, 0, 8) == 1);
 }
 
 // Another process that has the device's resident launches (its name, bound
@@ -446,6 +464,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> all = {{"lds_attribute", vti::lds_attribute},
                                                        {"refused_step", vti::refused_step},
                                                        {"launch_order", vti::launch_order},
+                                                       {"short_calls", vti::short_calls},
                                                        {"shared_device", vti::shared_device},
                                                        {"refused_program", vti::refused_program},
                                                        {"missed_exchange", vti::missed_exchange},

@@ -8,7 +8,8 @@ import pytest
 from conftest import ROOT
 from geophysics_amd import build
 
-SCENARIOS = ["lds_attribute", "refused_step", "launch_order", "shared_device", "refused_program", "missed_exchange", "plans"]
+SCENARIOS = ["lds_attribute", "refused_step", "launch_order", "short_calls", "shared_device", "refused_program", "missed_exchange",
+             "plans"]
 
 
 @pytest.fixture(scope="module")
