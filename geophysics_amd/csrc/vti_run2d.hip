@@ -1126,7 +1126,7 @@ bool under_way(const Chip &c)
 }
 
 // An object that launches on s: false: not on this stream (one that may not use
-// all CUs).
+// all CUs), or not now.
 bool chip_enter(int device, hipStream_t s)
 {
     Device2d d;
@@ -1141,9 +1141,11 @@ bool chip_enter(int device, hipStream_t s)
     }
     Chip &c = chip_of(device);
     const std::lock_guard<std::mutex> l(c.m);
-    const bool one = c.streams.size() == 1;
+    const bool second = c.streams.size() == 1 && !c.streams.count(s);
+    // an event recorded there now would belong to the graph that is captured
+    if (second && c.last && capturing(c.last)) return false;
     ++c.streams[s];
-    if (one && c.streams.size() > 1) note(c);
+    if (second) note(c);
     return true;
 }
 // its launches have been waited for

@@ -33,6 +33,7 @@ static std::function<void()> g_after_attribute;     // what another thread does 
 static std::vector<hipError_t> g_refuse;            // what the next launches return, hipSuccess: as usual
 static std::vector<std::string> g_order;            // launches, events and waits, with their streams
 static bool g_busy = false;                         // the latest noted launch is under way
+static hipStream_t g_capturing = nullptr;
 static int g_mask = 256;                            // CUs that a stream may use
 static bool g_no_memory = false;
 static int g_cus = 256, g_lds = 163840;
@@ -59,9 +60,9 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c)
 {
-    *c = hipStreamCaptureStatusNone;
+    *c = s && s == g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 hipError_t hipGetDevice(int *d)
@@ -210,6 +211,9 @@ void launch_order()
         Ctx b(440, 440);
         b.stream = stream(2);
         g_order.clear();
+        g_capturing = stream(1);        // no event there, so not now
+        CHECK(run2d_steps(&b, 0, 32) == 0 && g_order.empty());
+        g_capturing = nullptr;
         CHECK(run2d_steps(&b, 0, 32) == 1 && run2d_steps(&b, 0, 32) == 1);
         CHECK((g_order == Order{"record 1", "wait 2", "launch 2", "record 2", "launch 2", "record 2"}));
         g_order.clear();
