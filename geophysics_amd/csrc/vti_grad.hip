@@ -620,13 +620,13 @@ struct Grad : vti_grad {
 
     // The forward sweep with its record as one resident launch (FP32, 2D):
     // q collects the steps and checkpoints.  1040 x 340, 400 steps: 4.4 ms
-    // step by step, 1.7 so; recomputation runs of ~10 steps between adjoint
-    // steps stay with the per-step kernels.  The descriptors, gains and program
-    // cost each sweep ~80 us, the object's first one 80 to 250 us more for the
-    // plan and its memory: us of forward(), first / later, step by step and so,
-    // of 12 / 16 / 32 / 64 steps, 60 x 50 106, 174 / 128, 218 / 222, 196 / 416,
-    // 283 and 138, 125 / 168, 135 / 278, 171 / 534, 243; 1000 x 300 194, 268 /
-    // 228, 293 / 417, 380 / 881, 689 and 174, 159 / 229, 178 / 397, 252 / 873, 531.
+    // step by step, 1.7 so; the recomputation runs of ~10 steps between adjoint
+    // steps are per-step kernels.  The descriptors, gains and program cost each
+    // sweep ~80 us, the object's first one ~100 us more for the plan and its
+    // memory: us of forward(), step by step and so, an object's first one of 32 /
+    // 64 steps 60 x 50 222, 205 / 416, 276, 1000 x 300 417, 374 / 881, 608; a later
+    // one of 12 / 16 / 32 steps 60 x 50 116, 123 / 149, 125 / 280, 162, 1000 x 300
+    // 169, 159 / 228, 173 / 402, 244.
     // 1: q is set up, 0: not available, < 0: error
     int resident(RtmProgram &q)
     {

@@ -17,11 +17,12 @@
 // only after it has taken all of step s, so a plane is written again only
 // when its last samples have been read.
 //
-// What bounds a step now: the exchange, ~0.8 us from one XCD's store to
-// another's load, then LDS latency and instruction issue.  Measured (us a
-// step, velocity + stress launches -> this): 60 x 50 with a 20-cell layer
-// 5.8 -> 1.9, 400 x 400 7.2 -> 2.8, TTI 600 x 300 with a 50-cell layer
-// 10.7 -> 5.2, 2401 x 803 unsplit 27.9 -> 11.3.
+// What bounds a step now: on small tiles the chain of exchange, barriers and
+// LDS (60 x 50: wavefronts wait 72 % of their time, VALU 18 % busy), on large
+// ones instructions (2401 x 803: VALU 72 % busy).  Measured (us a step, velocity
+// + stress launches -> this): 60 x 50 with a 20-cell layer 5.8 -> 1.8, 400 x
+// 400 7.2 -> 3.0, TTI 600 x 300 with a 50-cell layer 10.7 -> 5.0, 2401 x 803
+// unsplit 27.9 -> 10.7.
 //
 // The arithmetic is vel2d_kernel's / stress2d_kernel's (and the TTI pair's)
 // term by term; products that do not change from step to step are formed
@@ -1353,7 +1354,7 @@ Run2dParts run2d_parts(const std::vector<Run2dShot> &shots, int device)
             cuts_of(shots[k].nnx, shots[k].nnz, false, j, d.cus, d.lds, cuts[j].back());
         }
     }
-    // strips of 6 spill ~95 registers with the images: for shots that fit no
+    // strips of 6 spill ~80 registers with the images: for shots that fit no
     // other way (24 shots of 0.1 to 1 M cells: 46 ms in parts of strips of 6
     // taken at their plain cost, 39 with parts of 4)
     for (auto &c : cuts[kRtmShapes - 1])
